@@ -53,25 +53,22 @@ enum { PSP_HIP_LDL_1D = 0, PSP_HIP_LDL_SELINV_1D = 1 };
 enum {
     PSP_HIP_OPT_SWEEP_GRAPH = 1,     /* 1 (default): replay the sweep from a captured
                                         hipGraph; 0: launch it kernel by kernel */
-    PSP_HIP_OPT_SOLVE_MIN_TILES = 2, /* front-solve workgroups wanted per launch when
-                                        choosing default tile shapes (default 256) */
-    PSP_HIP_OPT_SOLVE_MAX_SPLIT = 3, /* most inner slices per row block in the
-                                        default tile shapes (default 8) */
-    PSP_HIP_OPT_SOLVE_WIDE_WG = 4,   /* 1: default shapes give levels with few row
-                                        blocks 16-wave workgroups instead of inner
-                                        slices (8 <= k < 32); 0 (default): slices */
-    PSP_HIP_OPT_SOLVE_PERSIST = 5,   /* 1 (default): default shapes run the front
-                                        solves with persistent, pipelined
-                                        workgroups (8 <= k <= 16); 0: one
-                                        workgroup per tile */
-    PSP_HIP_OPT_SOLVE_PERSIST_GRID = 6, /* persistent launches use at most this many
-                                          workgroups (more only when one would
-                                          get over 32 tiles); 0 (default): as many
-                                          as fit on the device at once */
+    PSP_HIP_OPT_SOLVE_MIN_TILES = 2, /* front-solve workgroups wanted per launch:
+                                        tiles are cut until there are about twice
+                                        as many (default 256) */
+    PSP_HIP_OPT_SOLVE_MAX_SPLIT = 3, /* most inner slices a tile is cut into, in
+                                        quarters (default 8: 32 slices) */
+    PSP_HIP_OPT_SOLVE_WIDE_WG = 4,   /* accepted, without effect on the merged solves */
+    PSP_HIP_OPT_SOLVE_PERSIST = 5,   /* accepted, without effect on the merged solves */
+    PSP_HIP_OPT_SOLVE_PERSIST_GRID = 6, /* accepted (>= 0), without effect */
     PSP_HIP_OPT_SOLVE_FUSED = 7,       /* 1: for 8 <= k <= 16, the tree levels from
                                           the cut depth down run as one persistent
                                           launch per direction, a subtree queue per
-                                          XCD; 0 (default): one launch per level */
+                                          XCD, on factors in their own layout (made
+                                          by the next factorization, or from the
+                                          same velocity by the next solve); 0
+                                          (default): merged solves, one launch per
+                                          depth group and direction */
     PSP_HIP_OPT_SOLVE_FUSED_QUEUES = 8, /* queues of the fused launches (default 8,
                                           one per XCD; more leaves queues that the
                                           last workgroup runs alone) */
@@ -83,10 +80,9 @@ enum {
                                           near the cut, row blocks are cut into inner
                                           slices until a level has about that many
                                           tiles per queue; 1: no slices */
-    PSP_HIP_OPT_SOLVE_XCD_REDUCE = 12, /* 1 (default): the inner slices of a row block
+    PSP_HIP_OPT_SOLVE_XCD_REDUCE = 12, /* 1 (default): the inner slices of a tile
                                           run on one XCD and the last to finish sums
-                                          them in the product launch (one-workgroup-
-                                          per-tile levels, 8 <= k < 32), when the
+                                          them in the product launch, when the
                                           device deals workgroups to its XCDs
                                           round-robin (checked at set-up); 0: a
                                           reduce launch follows the product launch */
@@ -230,11 +226,11 @@ int psp_hip_solve_panel(psp_hip_ctx* ctx, void* B, int k, int panel);
 int psp_hip_profile_sweep(psp_hip_ctx* ctx, void* B, int k,
                           psp_hip_kernel_stats* stats);
 
-/* Tile-shape tuner for the front solves (no reference counterpart): for
- * each panel class, tree level and direction, times every candidate shape
- * (rows per tile 64/32/16, inner slices 1/2/4/8) with k right-hand sides on
- * the class's first panel and keeps the fastest; the chosen shapes stay for
- * later solves of this context.  before/after (may be NULL) receive the
+/* Tile tuner for the front solves (no reference counterpart): for each panel
+ * class, depth group and direction, times every candidate tile length (inner
+ * blocks per workgroup) with k right-hand sides on the class's panels and
+ * keeps the fastest; the chosen lengths stay for later solves of this
+ * context.  before/after (may be NULL) receive the
  * estimated front-solve time of one sweep with the old and new shapes.
  * Needs a factored context. */
 int psp_hip_autotune(psp_hip_ctx* ctx, int k, double* before, double* after);
@@ -246,15 +242,12 @@ int psp_hip_autotune(psp_hip_ctx* ctx, int k, double* before, double* after);
  * would alone.  Default: the GMRES steps of all problems in lockstep on the
  * first context's stream, and the sweeps of all unfinished problems merged:
  * the problems form two groups of about equal work, and one launch per
- * sweep step (a panel copy, or one tree level's products or reduce) covers
+ * sweep step (a panel copy, or one depth group's products or reduce) covers
  * that step of every problem of a group; the two groups' launch chains are
  * parallel branches of one hipGraph, replayed for every sweep; one host
- * wait per GMRES step for all problems.  The front products of a
- * problem then run on the one-workgroup-per-tile matrix-core kernel with
- * its tuned tile rows, slices and waves (persistent tiles included), so a
- * problem with k < 8 or k >= 32 sums in another order than alone (results
- * agree to rounding; they are bitwise equal for
- * 8 <= k < 32).  Problems with FP32 and FP64 fronts form two such batches,
+ * wait per GMRES step for all problems.  The front products of a problem run
+ * on its own tiles with the sums of its own sweep, so its solution is bitwise
+ * that of its own solve.  Problems with FP32 and FP64 fronts form two such batches,
  * run in turn.  flags & PSP_HIP_BATCH_THREADS: solve i runs
  * psp_hip_solve on its own host thread and its context's stream instead.
  * Contexts must be distinct.  reports may be NULL (batch-wide phase times

@@ -398,16 +398,6 @@ template <typename T>
 struct Raw2 {
     cx<T> a, b;
 };
-template <typename T>
-struct Raw3 {
-    cx<T> a, b, c;
-};
-template <typename T>
-struct RawRow {  // gathered value of a bottom row (two slot copies) and its parent row
-    cx<T> a, b;
-    int32_t prow;
-};
-
 // The value v, passed through an empty asm: the compiler must hold it in a
 // register at this point, so a load that produced it is not sunk into the
 // arm of a later select (where its wait would sit inside a branch, one
@@ -454,14 +444,6 @@ __device__ __forceinline__ cx<T> StageValue(const NodeDev& nd, const Slots<T>& g
     return *p;
 }
 
-template <typename T, int PH>
-__device__ __forceinline__ cx<T> StageOperand(const NodeDev& nd, const int32_t* structs,
-                                              const Slots<T>& gs, const cx<T>* Xp,
-                                              const cx<T>* W, int col, int rr, int k)
-{
-    return StageValue<T, PH>(nd, gs, Xp, W, col, rr, k, Opaque(StageIndex<PH>(nd, structs, col)));
-}
-
 // N staged elements of a thread; at(q) gives element q's (inner index,
 // right-hand side) as an int2.
 template <typename T, int PH, int N, class AT>
@@ -481,15 +463,6 @@ __device__ __forceinline__ void StageBatch(const NodeDev& nd, const int32_t* str
         const int2 p = at(q);
         sv[q] = StageValue<T, PH>(nd, gs, Xp, W, p.x, p.y, k, sx[q]);
     }
-}
-
-// Factor entry of phase PH at (row, col) of the node's block.
-template <typename T, int PH>
-__device__ __forceinline__ cx<T> FactorEntry(const cx<T>* Lf, const cx<T>* Lt, int s, int fs,
-                                             int row, int col)
-{
-    if (PH == PH_F) return col <= row ? Lf[row + (int64_t)col * fs] : czero<T>();
-    return col >= row ? Lt[row + (int64_t)col * s] : czero<T>();
 }
 
 // Finish of output row `row`, right-hand side r, product a.  F: top rows
@@ -520,111 +493,6 @@ __device__ __forceinline__ void FinishGather(const NodeDev& nd, const Slots<T>& 
                       gs.relinds[nd.ustart + row - nd.s]);
     } else {
         Finish<T, PH>(nd, gs, Xp, W, row, r, k, a, czero<T>(), 0);
-    }
-}
-
-constexpr int kMvThreads = 512;  // 8 waves split each row block's inner indices
-
-// Vector-unit path (k < 8).  One workgroup per tile (a block of RT output
-// rows and an inner range).  Lane l of a wave owns row l % RT and column
-// slot l / RT (64 / RT columns per wave step); the inner range is cut into
-// chunks of NI columns per lane.  For each chunk the lane first issues all
-// NI of its factor loads, then the workgroup stages the matching vector
-// rows in LDS, so the factor and vector reads of a chunk are in flight
-// together.  Column slots are combined by lane shuffles and the 8 waves'
-// partial sums by a fixed-order tree in LDS: every output element is summed
-// in a fixed order.
-template <typename T, int PH, int RT>
-__global__ __launch_bounds__(kMvThreads) void k_mv(const SolveTile* tiles, int start,
-                                                    const int32_t* structs,
-                                                    Slots<T> gs, const cx<T>* L,
-                                                    const cx<T>* LT, cx<T>* Xp, cx<T>* W,
-                                                    cx<T>* P, int k)
-{
-    constexpr int KC = 8, NW = kMvThreads / 64, CPW = 64 / RT, STRIDE = CPW * NW;
-    constexpr int NI = RT == 16 ? 16 : 32, CC = STRIDE * NI;
-    const SolveTile tl = tiles[start + blockIdx.x];
-    if (tl.nrows <= 0) return;  // a hole of the XCD placement
-    const NodeDev nd = tl.nd;
-    const int s = nd.s, fs = nd.s + nd.u;
-    const cx<T>* Lf = L + nd.l;
-    const cx<T>* Lt = LT + nd.l;
-    __shared__ cx<T> vs[CC][KC];            // staged vector chunk
-    __shared__ cx<T> red[NW / 2][RT][KC];   // wave partial sums
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rl = lane % RT, slot = lane / RT;
-    const int row = tl.row0 + rl;
-    const bool rowOk = rl < tl.nrows;
-    const int first = slot + CPW * wave;  // this lane's first column in a chunk
-    for (int r0 = 0; r0 < k; r0 += KC) {
-        const int kc = min(KC, k - r0);
-        cx<T> acc[KC];
-#pragma unroll
-        for (int r = 0; r < KC; ++r) acc[r] = czero<T>();
-        for (int cb = tl.col0; cb < tl.col1; cb += CC) {
-            const int ncol = min(CC, tl.col1 - cb);
-            // staging loads first, then the factor loads, all in flight
-            // together; the LDS stores wait only for the staging loads
-            constexpr int SPT = CC * KC / kMvThreads;
-            cx<T> sv[SPT];
-            StageBatch<T, PH>(nd, structs, gs, Xp, W, k, [&](int q) {
-                const int e = tid + kMvThreads * q, c = e / KC, r = e % KC;
-                return int2{cb + min(c, ncol - 1), min(r0 + r, k - 1)};
-            }, sv);
-            cx<T> m[NI];
-#pragma unroll
-            for (int u = 0; u < NI; ++u) {
-                const int c = first + STRIDE * u;
-                m[u] = (rowOk && c < ncol) ? FactorEntry<T, PH>(Lf, Lt, s, fs, row, cb + c)
-                                           : czero<T>();
-            }
-            LdsBarrier();  // the previous chunk's readers are done with vs
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) {
-                const int e = tid + kMvThreads * q, c = e / KC, r = e % KC;
-                if (c < ncol) vs[c][r] = r < kc ? sv[q] : czero<T>();
-            }
-            LdsBarrier();
-#pragma unroll
-            for (int u = 0; u < NI; ++u) {
-                const int c = first + STRIDE * u;
-                if (c < ncol) {
-#pragma unroll
-                    for (int r = 0; r < KC; ++r) acc[r] = cfma(m[u], vs[c][r], acc[r]);
-                }
-            }
-        }
-        // combine the column slots of a wave (lanes l, l + RT, ...)
-#pragma unroll
-        for (int o = RT; o < 64; o <<= 1) {
-#pragma unroll
-            for (int r = 0; r < KC; ++r) {
-                acc[r].r += __shfl_xor(acc[r].r, o, 64);
-                acc[r].i += __shfl_xor(acc[r].i, o, 64);
-            }
-        }
-        for (int h = NW / 2; h >= 1; h >>= 1) {
-            if (wave >= h && wave < 2 * h && slot == 0) {
-#pragma unroll
-                for (int r = 0; r < KC; ++r) red[wave - h][rl][r] = acc[r];
-            }
-            LdsBarrier();
-            if (wave < h && slot == 0) {
-#pragma unroll
-                for (int r = 0; r < KC; ++r) acc[r] = acc[r] + red[wave][rl][r];
-            }
-            LdsBarrier();
-        }
-        if (wave == 0 && slot == 0 && rowOk) {
-#pragma unroll
-            for (int r = 0; r < KC; ++r)
-                if (r < kc) {
-                    if (tl.slot >= 0)
-                        P[((int64_t)tl.slot * 64 + rl) * k + r0 + r] = acc[r];
-                    else
-                        FinishGather<T, PH>(nd, gs, Xp, W, row, r0 + r, k, acc[r]);
-                }
-        }
     }
 }
 
@@ -665,32 +533,10 @@ struct Mfma<double> {
     static __device__ __forceinline__ int row(int lk, int q) { return lk + 4 * q; }
 };
 
-// Build-time tuning of the matrix-core solve kernel: factor loads in flight
-// per lane (FP32 / FP64 fronts) and the waves per SIMD the register
-// allocation must allow (0: the compiler's choice).
-#ifndef PSP_MVM_U32
-#define PSP_MVM_U32 8
-#endif
-#ifndef PSP_MVM_U64
-#define PSP_MVM_U64 8
-#endif
-// Staged elements (columns x right-hand sides) per chunk, by front precision:
-// smaller chunks keep fewer staging registers, so more workgroups fit on a
-// CU (each launch then runs in fewer rounds of workgroups).
-#ifndef PSP_MVM_CHUNK32
-#define PSP_MVM_CHUNK32 1024
-#endif
-#ifndef PSP_MVM_CHUNK64
-#define PSP_MVM_CHUNK64 512
-#endif
-#ifndef PSP_MVM_WAVES_PER_EU
-#define PSP_MVM_WAVES_PER_EU 0
-#endif
-#if PSP_MVM_WAVES_PER_EU > 0
-#define PSP_MVM_OCCUPANCY __attribute__((amdgpu_waves_per_eu(PSP_MVM_WAVES_PER_EU)))
-#else
-#define PSP_MVM_OCCUPANCY
-#endif
+// Factor loads in flight per lane of the level and fused-subtree kernels, and
+// staged elements (columns x right-hand sides) per chunk by front precision:
+// smaller chunks keep fewer staging registers, so more workgroups fit on a CU.
+constexpr int PSP_MVM_U = 8, PSP_MVM_CHUNK32 = 1024, PSP_MVM_CHUNK64 = 512;
 
 // --------------------------------------------------------------------------
 // Hand-offs between workgroups of one XCD.  Workgroups are dealt to the 8
@@ -779,14 +625,14 @@ __global__ void k_xcc_probe(int32_t* out)
 //
 // MvmTile is the work of one workgroup on tile tl (nrows > 0); k_mvm runs it
 // on one panel solve's tiles, k_mvm_batch on the tiles of many.
-template <typename T, int PH, int RT, int KB, int NWV>
+template <typename T, int PH, int RT, int KB>
 __device__ __forceinline__ void MvmTile(const SolveTile tl, const int32_t* structs,
                                         const Slots<T> gs, const cx<T>* L, const cx<T>* LT,
                                         cx<T>* Xp, cx<T>* W, cx<T>* P, int k, int32_t* redc,
                                         const SolveTile* reds);
 
-template <typename T, int PH, int RT, int KB, int NWV>
-__global__ __launch_bounds__(64 * NWV) PSP_MVM_OCCUPANCY void k_mvm(const SolveTile* tiles, int start,
+template <typename T, int PH, int RT, int KB>
+__global__ __launch_bounds__(256) void k_mvm(const SolveTile* tiles, int start,
                                                      const int32_t* structs,
                                                      Slots<T> gs, const cx<T>* L,
                                                      const cx<T>* LT, cx<T>* Xp, cx<T>* W,
@@ -795,23 +641,20 @@ __global__ __launch_bounds__(64 * NWV) PSP_MVM_OCCUPANCY void k_mvm(const SolveT
 {
     const SolveTile tl = tiles[start + blockIdx.x];
     if (tl.nrows <= 0) return;
-    MvmTile<T, PH, RT, KB, NWV>(tl, structs, gs, L, LT, Xp, W, P, k, redc, reds);
+    MvmTile<T, PH, RT, KB>(tl, structs, gs, L, LT, Xp, W, P, k, redc, reds);
 }
 
-template <typename T, int PH, int RT, int KB, int NWV>
+template <typename T, int PH, int RT, int KB>
 __device__ __forceinline__ void MvmTile(const SolveTile tl, const int32_t* structs,
                                         const Slots<T> gs, const cx<T>* L, const cx<T>* LT,
                                         cx<T>* Xp, cx<T>* W, cx<T>* P, int k, int32_t* redc,
                                         const SolveTile* reds)
 {
     typedef typename Mfma<T>::acc acc_t;
-    constexpr int NT = 64 * NWV, WR = RT / 16, WK = NWV / WR, NB = KB / 8;
-    // factor loads in flight per lane; 16-wave workgroups (128 VGPRs a lane)
-    // keep fewer
-    constexpr int U = (sizeof(T) == 4 ? PSP_MVM_U32 : PSP_MVM_U64) / (NWV == 16 ? 4 : 1);
-    // staged inner columns per chunk; 16-wave tiles reuse the chunk buffer
-    // as reduction scratch and keep the large one
-    constexpr int CC = (NWV == 16 ? 2048 : sizeof(T) == 4 ? PSP_MVM_CHUNK32 : PSP_MVM_CHUNK64) / KB;
+    constexpr int NWV = 4, NT = 64 * NWV, WR = RT / 16, WK = NWV / WR, NB = KB / 8;
+    constexpr int U = PSP_MVM_U;  // factor loads in flight per lane
+    // staged inner columns per chunk
+    constexpr int CC = (sizeof(T) == 4 ? PSP_MVM_CHUNK32 : PSP_MVM_CHUNK64) / KB;
     constexpr bool PRE = KB <= 16 && PH == PH_F;
     static_assert(WR * WK == NWV && CC % 4 == 0 && U >= 1, "tile shape");
     static_assert(WK == 1 || 2 * CC * KB >= WR * (WK / 2) * NB * 256,
@@ -991,345 +834,6 @@ __device__ __forceinline__ void MvmTile(const SolveTile tl, const int32_t* struc
     }
 }
 
-// Persistent, pipelined matrix-core path (8 <= k <= KB, KB = 8 or 16: one
-// pass over the right-hand sides).  gridDim.x workgroups take the launch's
-// tiles round-robin (their descriptors are read into LDS once) and work
-// through them as a sequence of steps of CW inner columns.  Two register
-// sets alternate: while step n is multiplied, the staging and factor loads
-// of step n + 1 are in flight, and in the backward phase also the struct
-// rows that the gather of step n + 2 needs.  The products, the summation
-// order within a tile (4-column steps in increasing order, the waves of a
-// row block summed by the same fixed tree) and the finish are those of
-// k_mvm; only the schedule differs.  No workgroup waits for another.
-//
-// The loop is written for few vector instructions per load: a tile's
-// fields are made wave-uniform (so its base addresses are scalar), every
-// lane's offsets within a step are fixed for the launch, and factor entries
-// are used unmasked.  That relies on the solve storage: the triangles a
-// phase does not use are zero (k_transpose_scale), the factor and vector
-// buffers end in kSolvePad padding columns / rows of zeros, so the entries
-// a partial step reads past its tile are finite and meet a zero in the
-// staged vector (the staged vector is masked), and rows past a partial
-// tile read the tile's last row and give outputs that are not stored.
-constexpr int kMvpTiles = 32;  // tiles per workgroup at most (host sizes the grid)
-#ifndef PSP_MVP_U
-#define PSP_MVP_U 8  // factor loads per lane per step, 64- and 32-row tiles
-#endif
-#ifndef PSP_MVP_U16
-#define PSP_MVP_U16 4  // factor loads per lane per step, 16-row tiles
-#endif
-
-template <typename T, int PH, int RT, int KB>
-struct MvpShape {
-    static constexpr int NT = 256, WR = RT / 16, WK = 4 / WR, NB = KB / 8;
-    static constexpr int U = RT == 16 ? PSP_MVP_U16 : PSP_MVP_U;  // factor loads per lane per step
-    static constexpr int CW = 4 * WK * U;        // inner columns per step
-    static constexpr int SPT = CW * KB / NT;     // staged elements per thread per step
-    static_assert(CW * KB == SPT * NT && SPT >= 1, "step shape");
-    static_assert(CW <= kSolvePad, "a step reads at most kSolvePad columns past its tile");
-};
-
-__device__ __forceinline__ int Uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t Uni(int64_t v)
-{
-    const uint64_t u = (uint64_t)v;
-    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32)) << 32) |
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u));
-}
-
-template <typename T, int PH, int RT, int KB>
-__global__ __launch_bounds__(256) void k_mvp(const SolveTile* tiles, int start, int count,
-                                             const int32_t* structs, Slots<T> gs,
-                                             const cx<T>* L, const cx<T>* LT, cx<T>* Xp,
-                                             cx<T>* W, cx<T>* P, int k)
-{
-    typedef typename Mfma<T>::acc acc_t;
-    typedef MvpShape<T, PH, RT, KB> S;
-    constexpr int NT = S::NT, WK = S::WK, NB = S::NB, U = S::U, CW = S::CW, SPT = S::SPT;
-    constexpr int NRED = WK > 1 ? S::WR * (WK / 2) * NB * 256 : 1;
-    typedef typename std::conditional<PH == PH_F, Raw3<T>, cx<T>>::type Staged;
-    struct Pre {       // forward finish of a tile: gathered rows and parent rows
-        Raw2<T> g[PH == PH_F ? NB : 1][4];
-        int32_t prow[4];
-    };
-    struct Data {      // one step's loads
-        cx<T> m[U];    // factor entries
-        Staged v[SPT]; // staged inner operand (raw)
-        Pre pre;       // forward, last step of a tile: its finish data
-    };
-    struct Idx {       // backward: panel rows of one step's update columns
-        int32_t x[PH == PH_B ? SPT : 1];
-    };
-    struct Tile {      // wave-uniform fields of a tile
-        int64_t l, w;
-        int off, s, u, ustart, pw, cslot, row0, nrows, col0, col1, slot;
-    };
-    __shared__ SolveTile tq[kMvpTiles];
-    // staged vector in the two forms the B operand takes: lanes l % 16 < 8
-    // read (re, -im), the others (im, re)
-    __shared__ T2<T> vs[2][2][CW][KB];
-    __shared__ T red[NRED];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave / WK, wk = wave % WK;
-    const int li = lane & 15, lk = lane >> 4;
-    const int G = gridDim.x;
-    const int nmine = (count - (int)blockIdx.x + G - 1) / G;
-    {
-        const int4* src = reinterpret_cast<const int4*>(tiles + start);
-        int4* dst = reinterpret_cast<int4*>(tq);
-        for (int e = tid; e < nmine * 4; e += NT)
-            dst[e] = src[((int64_t)blockIdx.x + (int64_t)(e >> 2) * G) * 4 + (e & 3)];
-    }
-    LdsBarrier();
-    if (nmine <= 0) return;
-    auto tile = [&](int i) {
-        const SolveTile& t = tq[i];
-        Tile r;
-        r.l = Uni(t.nd.l);
-        r.w = Uni(t.nd.w);
-        r.off = Uni(t.nd.off);
-        r.s = Uni(t.nd.s);
-        r.u = Uni(t.nd.u);
-        r.ustart = Uni(t.nd.ustart);
-        r.pw = Uni(t.nd.pw);
-        r.cslot = Uni(t.nd.cslot);
-        r.row0 = Uni(t.row0);
-        r.nrows = Uni(t.nrows);
-        r.col0 = Uni(t.col0);
-        r.col1 = Uni(t.col1);
-        r.slot = Uni(t.slot);
-        return r;
-    };
-    // lane constants of the launch
-    const int lrow = 16 * wr + li;        // factor row within the tile
-    const int lcol = 4 * wk + lk;         // factor column within a 4 WK-column group
-    int sc[SPT], sr[SPT];                 // staged element: column within the step, rhs
-#pragma unroll
-    for (int q = 0; q < SPT; ++q) sc[q] = (tid + NT * q) / KB, sr[q] = (tid + NT * q) % KB;
-
-    struct Cur {
-        int i, c0;  // tile (of this workgroup) and first inner column of the step
-    };
-    auto ncolsOf = [&](int i) { return max(Uni(tq[i].col1) - Uni(tq[i].col0), 1); };
-    auto advance = [&](Cur c) {
-        if (c.i >= nmine) return c;  // past the end stays there
-        c.c0 += CW;
-        if (c.c0 >= ncolsOf(c.i)) {
-            ++c.i;
-            c.c0 = 0;
-        }
-        return c;
-    };
-    auto issueIdx = [&](Cur c, Idx& ix) {
-        if constexpr (PH == PH_B) {
-            const int ustart = Uni(tq[c.i].nd.ustart), s = Uni(tq[c.i].nd.s);
-            const int cb = Uni(tq[c.i].col0) + c.c0;
-            const int32_t* sb = structs + ustart;  // read up to kSolvePad past the list
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) ix.x[q] = sb[max(cb + sc[q] - s, 0)];
-        }
-    };
-    auto issueData = [&](Cur c, Data& d, Idx& ix) {
-        const Tile t = tile(c.i);
-        const int cb = t.col0 + c.c0;
-        const int fa = PH == PH_F ? t.s + t.u : t.s;  // column stride of the factor block
-        const cx<T>* Ab = (PH == PH_F ? L : LT) + t.l + t.row0 + (int64_t)cb * fa;
-        const uint32_t la = (uint32_t)(min(lrow, t.nrows - 1) + lcol * fa);
-        const int64_t ustep = (int64_t)(4 * WK) * fa;
-        if constexpr (PH == PH_B) {
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) ix.x[q] = Opaque(ix.x[q]);
-        }
-        if constexpr (PH == PH_F) {
-            const cx<T>* g0 = gs.G + (t.w + cb) * k;
-            const cx<T>* g1 = g0 + gs.half;
-            const cx<T>* xb = Xp + (int64_t)(t.off + cb) * k;
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) {
-                const uint32_t o = (uint32_t)(sc[q] * k + sr[q]);
-                d.v[q] = Raw3<T>{g0[o], g1[o], xb[o]};
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) {
-                const int col = cb + sc[q];
-                const int64_t row = col < t.s ? t.w + col : (int64_t)ix.x[q];
-                d.v[q] = (col < t.s ? W : Xp)[row * k + sr[q]];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) d.m[u] = (Ab + u * ustep)[la];
-    };
-    auto issuePre = [&](int i, Pre& pr) {
-        if constexpr (PH == PH_F) {
-            const Tile t = tile(i);
-            const int fs = t.s + t.u;
-            const int32_t* rb = gs.relinds + t.ustart;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = min(t.row0 + 16 * wr + Mfma<T>::row(lk, q), fs - 1);
-                pr.prow[q] = rb[max(row - t.s, 0)];
-            }
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int row = min(t.row0 + 16 * wr + Mfma<T>::row(lk, q), fs - 1);
-                    const int64_t o = (t.w + row) * k + min(8 * b + li, k - 1);
-                    pr.g[b][q] = Raw2<T>{gs.G[o], gs.G[gs.half + o]};
-                }
-        }
-    };
-    acc_t acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
-    auto finishTile = [&](int i, const Pre& pr) {
-        if (WK > 1) {  // waves that share rows sum their partial tiles by a fixed tree
-            for (int h = WK / 2; h >= 1; h >>= 1) {
-                LdsBarrier();
-                if (wk >= h && wk < 2 * h) {
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            red[(((wr * h + wk - h) * NB + b) * 64 + lane) * 4 + q] = acc[b][q];
-                }
-                LdsBarrier();
-                if (wk < h) {
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            acc[b][q] += red[(((wr * h + wk) * NB + b) * 64 + lane) * 4 + q];
-                }
-            }
-        }
-        if (wk == 0) {
-            const Tile t = tile(i);
-            NodeDev nd;
-            nd.l = t.l, nd.w = t.w, nd.off = t.off, nd.s = t.s, nd.u = t.u;
-            nd.ustart = t.ustart, nd.pw = t.pw, nd.cslot = t.cslot;
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const T val = acc[b][q];
-                    const T other = __shfl_xor(val, 8, 64);
-                    const int rl = 16 * wr + Mfma<T>::row(lk, q), rr = 8 * b + li;
-                    if (li < 8 && rl < t.nrows && rr < k) {
-                        const cx<T> a{val, other};
-                        if (t.slot >= 0)
-                            P[((int64_t)t.slot * 64 + rl) * k + rr] = a;
-                        else if constexpr (PH == PH_F)
-                            Finish<T, PH>(nd, gs, Xp, W, t.row0 + rl, rr, k, a,
-                                          pr.g[b][q].a + pr.g[b][q].b, pr.prow[q]);
-                        else
-                            Finish<T, PH>(nd, gs, Xp, W, t.row0 + rl, rr, k, a, czero<T>(), 0);
-                    }
-                }
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
-    };
-    // B operand source of this lane (fixed for the launch)
-    const int form = li < 8 ? 0 : 1, bj = li & 7;
-    auto consume = [&](Cur c, const Data& d, int buf) {
-        const int nc = Uni(tq[c.i].col1) - (Uni(tq[c.i].col0) + c.c0);
-#pragma unroll
-        for (int q = 0; q < SPT; ++q) {
-            cx<T> v;
-            if constexpr (PH == PH_F)
-                v = d.v[q].a + d.v[q].b + d.v[q].c;
-            else
-                v = d.v[q];
-            const bool ok = sc[q] < nc && sr[q] < k;
-            const T re = ok ? v.r : T(0), im = ok ? v.i : T(0);
-            vs[buf][0][sc[q]][sr[q]] = T2<T>{re, -im};
-            vs[buf][1][sc[q]][sr[q]] = T2<T>{im, re};
-        }
-        LdsBarrier();
-        const T2<T>(*vb)[KB] = vs[buf][form];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int cl = lcol + 4 * WK * u;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const T2<T> w = vb[cl][8 * b + bj];
-                acc[b] = Mfma<T>::step(d.m[u].r, w.x, acc[b]);
-                acc[b] = Mfma<T>::step(d.m[u].i, w.y, acc[b]);
-            }
-        }
-        if (c.c0 + CW >= ncolsOf(c.i)) finishTile(c.i, d.pre);
-        if constexpr (PH == PH_F) {  // the finish data was issued one step ago
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    Sink(d.pre.g[b][q].a.r), Sink(d.pre.g[b][q].a.i);
-                    Sink(d.pre.g[b][q].b.r), Sink(d.pre.g[b][q].b.i);
-                }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) Sink(d.pre.prow[q]);
-        }
-    };
-
-    Data d0, d1;
-    Idx i0, i1;
-    // steps n, n + 1, n + 2: data of n sits in d[n % 2], its indices were in
-    // i[n % 2]; a cursor is past the end when its tile index reaches nmine.
-    // The index and data loads are issued unconditionally (a cursor past the
-    // end reloads the current step, unused), so the wait counts before a
-    // step's use never have to allow for a path without the loads issued
-    // after it.  The finish data of a tile travels with its last step in the
-    // same register set; it is issued after the multiply of the previous
-    // step, one step before it is used.
-    Cur cn{0, 0};
-    Cur cn1 = advance(cn);
-    Cur cn2 = advance(cn1);
-    auto lastStep = [&](Cur c) { return c.i < nmine && c.c0 + CW >= ncolsOf(c.i); };
-    issueIdx(cn, i0);
-    issueIdx(cn1.i < nmine ? cn1 : cn, i1);
-    issueData(cn, d0, i0);
-    if (PH == PH_F && lastStep(cn)) issuePre(cn.i, d0.pre);
-    auto half = [&](Idx& iN, Idx& iN1, Data& dN, Data& dN1, int buf) {
-        issueIdx(cn2.i < nmine ? cn2 : cn, iN);
-        issueData(cn1.i < nmine ? cn1 : cn, dN1, iN1);
-        consume(cn, dN, buf);
-        if (PH == PH_F && lastStep(cn1)) issuePre(cn1.i, dN1.pre);
-        cn = cn1;
-        cn1 = cn2;
-        cn2 = advance(cn2);
-    };
-    // On the way out, every load still in flight (the reloads past the end)
-    // is waited for: the compiler merges the two exits with the path back
-    // to the loop head, and a load pending on any of them would otherwise
-    // be drained at the head of every iteration.
-    auto drain = [&](const Data& d, const Idx& ix) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) Sink(d.m[u].r), Sink(d.m[u].i);
-#pragma unroll
-        for (int q = 0; q < SPT; ++q) {
-            if constexpr (PH == PH_F)
-                Sink(d.v[q].a.r), Sink(d.v[q].a.i), Sink(d.v[q].b.r), Sink(d.v[q].b.i),
-                    Sink(d.v[q].c.r), Sink(d.v[q].c.i);
-            else
-                Sink(d.v[q].r), Sink(d.v[q].i), Sink(ix.x[q]);
-        }
-    };
-    for (;;) {
-        half(i0, i1, d0, d1, 0);
-        if (cn.i >= nmine) {
-            drain(d1, i0);
-            break;
-        }
-        half(i1, i0, d1, d0, 1);
-        if (cn.i >= nmine) {
-            drain(d0, i1);
-            break;
-        }
-    }
-}
-
 // --------------------------------------------------------------------------
 // Fused subtree solves (8 <= k <= KB).  One persistent launch runs every
 // level of a phase from the class's cut depth down (forward: deepest level
@@ -1422,7 +926,7 @@ __global__ __launch_bounds__(256) void k_mvq(const QTile* tiles, const int32_t* 
 {
     typedef typename Mfma<T>::acc acc_t;
     constexpr int NWV = 4, NT = 256, WR = RT / 16, WK = NWV / WR, NB = KB / 8;
-    constexpr int U = sizeof(T) == 4 ? PSP_MVM_U32 : PSP_MVM_U64;
+    constexpr int U = PSP_MVM_U;
     constexpr int CC = (sizeof(T) == 4 ? PSP_MVM_CHUNK32 : PSP_MVM_CHUNK64) / KB;
     constexpr int SPT = CC * KB / NT;
     constexpr bool PRE = PH == PH_F;
@@ -1825,117 +1329,6 @@ __device__ __forceinline__ void MmaForEach(const typename Mfma<T>::acc (&acc)[Ti
             }
 }
 
-// Waves per SIMD the wide-block kernel is compiled for (its register budget:
-// 512 / waves), per precision, phase and tile rows; 1 leaves the compiler
-// free.  Each value is the most that compiles without spills.  Unbounded,
-// FP32 64-row forward tiles took 293 registers (one workgroup per CU) and
-// 16-row ones 140 (three).
-template <typename T, int PH, int RT>
-constexpr int MmwWavesPerEu()
-{
-    if (sizeof(T) == 4) return RT == 16 ? 4 : 2;
-    if (RT == 16) return PH == PH_F ? 3 : 1;
-    return RT == 64 && PH == PH_B ? 2 : 1;
-}
-
-// Wide-block front solves (k >= 32): one workgroup per solve tile and pass
-// of 64 right-hand sides, through the tile engine.
-template <typename T, int PH, int RT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MmwWavesPerEu<T, PH, RT>())))
-void k_mmw(const SolveTile* tiles, int start,
-                                              const int32_t* structs, Slots<T> gs,
-                                              const cx<T>* L, const cx<T>* LT, cx<T>* Xp,
-                                              cx<T>* W, cx<T>* P, int k)
-{
-    typedef TileShape<RT> S;
-    constexpr int IX = 2048;  // inner indices whose gather addresses are cached in LDS
-    __shared__ cx<T> As[2][kBK][RT + 1];
-    __shared__ cx<T> Bs[2][kBK][65];
-    __shared__ int32_t ix[PH == PH_F ? 1 : IX];
-    const SolveTile tl = tiles[start + blockIdx.x];
-    if (tl.nrows <= 0) return;  // a hole of the XCD placement
-    const NodeDev nd = tl.nd;
-    const int s = nd.s, fs = nd.s + nd.u;
-    const cx<T>* Lf = L + nd.l;
-    const cx<T>* Lt = LT + nd.l;
-    // B: the panel rows of the update columns are read once into LDS, so each
-    // K stage waits for one memory round trip instead of two (F needs no
-    // indices: its gathered input sits in the slot copies).
-    const int ncols = tl.col1 - tl.col0;
-    const bool cached = PH == PH_B && ncols <= IX;
-    if (cached) {
-        for (int c = threadIdx.x; c < ncols; c += 256) {
-            const int col = tl.col0 + c;
-            ix[c] = col >= s ? structs[nd.ustart + col - s] : col;
-        }
-    }
-    LdsBarrier();  // the cache is read by every thread's stage loads
-    const int ilast = tl.nrows - 1;
-    // A: the factor block, rows clamped into the tile, triangle masked later.
-    auto la = [&](int i, int col) {
-        const int row = tl.row0 + min(i, ilast);
-        return PH == PH_F ? Lf[row + (int64_t)col * fs] : Lt[row + (int64_t)col * s];
-    };
-    auto fa = [&](int i, int col, cx<T> v) {
-        const int row = tl.row0 + i;
-        const bool in = i < tl.nrows && (PH == PH_F ? col <= row : col >= row);
-        return in ? v : czero<T>();
-    };
-    for (int r0 = 0; r0 < k; r0 += 64) {
-        const int kc = min(64, k - r0);
-        typename Mfma<T>::acc acc[S::RB][S::CB];
-        if constexpr (PH == PH_F) {
-            // B: the gathered forward input (slot copies plus the panel rows).
-            auto lb = [&](int col, int j) {
-                const int rr = r0 + min(j, kc - 1);
-                const int64_t g = (nd.w + col) * k + rr;
-                return Raw3<T>{gs.G[g], gs.G[gs.half + g], Xp[(int64_t)(nd.off + col) * k + rr]};
-            };
-            auto fb = [&](int, int j, const Raw3<T>& v) { return j < kc ? v.a + v.b + v.c : czero<T>(); };
-            MmaTile<T, RT, true>(la, fa, lb, fb, tl.col0, tl.col1, As, Bs, acc);
-        } else {
-            auto fb = [&](int, int j, cx<T> v) { return j < kc ? v : czero<T>(); };
-            if (cached) {
-                auto lb = [&](int col, int j) {
-                    const int rr = r0 + min(j, kc - 1);
-                    // ix holds the W row (top columns, plus nd.w) or the
-                    // panel row: the read feeds both arms, so no branch
-                    const int64_t row = (int64_t)ix[col - tl.col0] + (col < s ? nd.w : 0);
-                    return (col < s ? W : Xp)[row * k + rr];
-                };
-                MmaTile<T, RT, true>(la, fa, lb, fb, tl.col0, tl.col1, As, Bs, acc);
-            } else {
-                auto lb = [&](int col, int j) {
-                    return StageOperand<T, PH>(nd, structs, gs, Xp, W, col, r0 + min(j, kc - 1), k);
-                };
-                MmaTile<T, RT, true>(la, fa, lb, fb, tl.col0, tl.col1, As, Bs, acc);
-            }
-        }
-        if (tl.slot >= 0) {
-            MmaForEach<T, RT>(acc, [&](int i, int j, cx<T> a) {
-                if (i < tl.nrows && j < kc) P[((int64_t)tl.slot * 64 + i) * k + r0 + j] = a;
-            });
-        } else if constexpr (PH == PH_F) {
-            // Bottom rows add their gathered value; its loads (and the parent
-            // row of each) are issued for a whole row block before any store.
-            auto ld = [&](int i, int j) {
-                const int row = tl.row0 + min(i, ilast);
-                const int64_t g = (nd.w + row) * k + r0 + min(j, kc - 1);
-                return RawRow<T>{gs.G[g], gs.G[gs.half + g],
-                                 gs.relinds[nd.ustart + max(row - s, 0)]};
-            };
-            MmaEpilogue<T, RT>(acc, ld, [&](int i, int j, cx<T> a, const RawRow<T>& g) {
-                if (i < tl.nrows && j < kc)
-                    Finish<T, PH>(nd, gs, Xp, W, tl.row0 + i, r0 + j, k, a, g.a + g.b, g.prow);
-            });
-        } else {
-            MmaForEach<T, RT>(acc, [&](int i, int j, cx<T> a) {
-                if (i < tl.nrows && j < kc) Finish<T, PH>(nd, gs, Xp, W, tl.row0 + i, r0 + j, k, a, czero<T>(), 0);
-            });
-        }
-    }
-}
-
 // Batched tile GEMM on the matrix cores: C (+)= +/- opA(A) diag(D) opB(B)
 // over a list of 64x64 tiles (see GemmFlags), through the tile engine.
 // 8-column LDS stages keep the registers low enough for 5 waves per SIMD in
@@ -2044,6 +1437,658 @@ __global__ __launch_bounds__(kThreads) void k_mv_reduce(const SolveTile* items, 
 }
 
 // --------------------------------------------------------------------------
+// Merged solves: F in blocks of 16 x 16 (see BlockTile), one launch per depth
+// group and direction, for any number of right-hand sides.
+//
+// A workgroup has 4 waves; wave q owns output block ob0 + q of its tile and
+// runs over the tile's inner blocks.  Factor blocks go straight from HBM into
+// the A operands: forward, lane l of a step t loads row l % 16 of column
+// 4 t + l / 16; backward the block is used transposed, and lane l loads rows
+// 4 (l / 16) .. + 4 of column l % 16 (the four steps then take the inner
+// index in the order t, 4 + t, 8 + t, 12 + t, which the staged vector
+// follows).  Either way a wave reads whole blocks, 2 or 4 KB, contiguous.
+// The inner vector is shared by the waves through LDS, CB blocks at a time in
+// two buffers: one barrier per chunk, the next chunk's vector and factor
+// loads in flight while a chunk is multiplied.  The first two chunks' factor
+// loads go out before anything is waited for; a tile is cut (DefaultSlices)
+// so that most waves have little more than that.
+//
+// What bounds it: for k <= 16 the factor stream (HBM) and, on small launches,
+// the dependent round trips record -> (indices ->) operands -> stores; for
+// k >= 32 the matrix cores.
+// --------------------------------------------------------------------------
+template <typename T>
+struct BlockBufs {
+    const cx<T>* F;      // one panel's blocks
+    cx<T>* V;            // the class's solve vector (VecRows)
+    const int32_t* bsrc;
+    const int32_t* blist;
+    const int32_t* udst;
+    const cx<T>* dinv;   // one panel's D^-1, by panel-vector row
+    cx<T>* P;            // partial sums, 64 rows per slot
+    int64_t w, g0, g1;   // VecRows
+    int32_t xrows, zero; // zero: a block of zeros in F
+};
+
+typedef const __attribute__((address_space(4))) int32_t* ConstInts;
+__device__ __forceinline__ ConstInts Const(const void* p) { return (ConstInts)(uintptr_t)p; }
+
+__device__ __forceinline__ int Uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Vector rows of an update row: where it is written, and what is added (the
+// children's contributions to it, and what a pivot row of the parent holds).
+template <typename T>
+__device__ __forceinline__ cx<T> UpdateBase(const BlockBufs<T>& a, int u, int work, int leaf,
+                                            int dst, int r, int k)
+{
+    cx<T> g = czero<T>();
+    if (!leaf) g = a.V[(a.g0 + u) * k + r] + a.V[(a.g1 + work) * k + r];
+    if (dst < a.xrows) g = g + a.V[(int64_t)dst * k + r];
+    return g;
+}
+
+// Output row `row` of a merged front (product v), right-hand side r.
+template <typename T, int PH>
+__device__ __forceinline__ void BlockFinish(const BlockBufs<T>& a, int x0, int w0, int u0, int s,
+                                            int u, int sb, int leaf, int row, int r, int k, cx<T> v)
+{
+    if (PH == PH_B) {
+        if (row < s) a.V[(int64_t)(x0 + row) * k + r] = v;
+    } else if (row < s) {
+        a.V[(a.w + x0 + row) * k + r] = v * a.dinv[x0 + row];
+    } else if (row >= kBlk * sb && row - kBlk * sb < u) {
+        const int ur = u0 + row - kBlk * sb, dst = a.udst[ur];
+        a.V[(int64_t)dst * k + r] = UpdateBase(a, ur, w0 + row, leaf, dst, r, k) + v;
+    }
+}
+
+template <typename T, int KB>
+struct BlockShape {
+    static constexpr int NB = KB / 8;
+    // blocks in flight per wave: 32 registers, so that 4 to 7 workgroups fit on
+    // a CU (twice as many in flight and half the workgroups: 5% slower)
+    static constexpr int U = sizeof(T) == 4 ? 4 : 2;
+    // inner blocks per chunk of the staged vector
+    static constexpr int CB = 16 / (KB / 8) / (sizeof(T) == 8 ? 2 : 1);
+    static constexpr int SPT = CB * kBlk * KB / 256;  // staged elements per thread
+    static_assert(CB % U == 0 || U % CB == 0, "chunk shape");
+};
+
+// Fields of a tile (scalar loads).
+struct TileRec {
+    int x0, w0, u0, s, u, sb, leaf, ob0, nob, ib0, nib, lst, slot, red;
+    __device__ explicit TileRec(ConstInts t)
+        : x0(t[0]), w0(t[1]), u0(t[2]), s(t[3]), u(t[4]), sb(t[5]), leaf(t[6]), ob0(t[7]),
+          nob(t[8]), ib0(t[9]), nib(t[10]), lst(t[11]), slot(t[12]), red(t[13])
+    {
+    }
+};
+
+// Inner slices of a tile: each wave's partial sums are in P; the slice that
+// arrives last sums the slots in slot order and finishes the rows.
+template <typename T, int PH>
+__device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& a, int k,
+                                          int32_t* redc, const BlockRed* reds)
+{
+    __shared__ int arrived;
+    const int tid = threadIdx.x;
+    WaitVmem();
+    LdsBarrier();  // every wave's partial sums have reached the L2
+    if (tid == 0) arrived = AddAgent(redc + t.red, 1);
+    LdsBarrier();
+    const ConstInts rd = Const(reds + t.red);
+    const int slot0 = rd[9], nslots = rd[10];
+    if (Uni(arrived) != nslots - 1) return;
+    const L2Buf<T> lP(a.P);
+    constexpr int kS = 8;  // slots loaded together
+    for (int e = tid; e < t.nob * kBlk * k; e += 256) {
+        const int rl = e / k, r = e % k;
+        cx<T> v = czero<T>();
+        for (int j0 = 0; j0 < nslots; j0 += kS) {
+            cx<T> pv[kS];
+#pragma unroll
+            for (int j = 0; j < kS; ++j)
+                pv[j] = lP[((int64_t)(slot0 + min(j0 + j, nslots - 1)) * 64 + rl) * k + r];
+#pragma unroll
+            for (int j = 0; j < kS; ++j)
+                if (j0 + j < nslots) v = v + pv[j];
+        }
+        BlockFinish<T, PH>(a, t.x0, t.w0, t.u0, t.s, t.u, t.sb, t.leaf, kBlk * t.ob0 + rl, r, k, v);
+    }
+    if (tid == 0) redc[t.red] = 0;  // no slice of this launch counts any more
+}
+
+// One workgroup on tile tp, up to KB = 8 or 16 right-hand sides (shared by
+// k_block and k_block_batch).  Reads of the vector and of the index lists may
+// run past the tile's inner range (up to a chunk; the buffers are padded);
+// those rows are not multiplied.
+template <typename T, int PH, int KB>
+__device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBufs<T>& a, int k,
+                                              int32_t* redc, const BlockRed* reds)
+{
+    typedef typename Mfma<T>::acc acc_t;
+    typedef BlockShape<T, KB> S;
+    constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT, U = S::U;
+    constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
+    __shared__ cx<T> vs[CB * kBlk][KB];
+    const ConstInts tw = Const(tp);
+    const TileRec t(tw);
+    const int tid = threadIdx.x, lane = tid & 63, q = Uni(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ob = t.ob0 + q;
+    const bool own = q < t.nob, top = ob < t.sb;
+    const int base = PH == PH_F ? tw[16 + q] : 0, blo = PH == PH_F ? tw[20 + q] : 0;
+    const int bhi = PH == PH_F ? tw[24 + q] : 0;
+    const int nch = (t.nib + CB - 1) / CB;
+    const int32_t* src = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0);
+    const uint32_t loff = PH == PH_F ? lk * kBlk + li : li * kBlk + 4 * lk;
+    const uint32_t rk = min(tid % KB, k - 1);           // staged right-hand side
+    const uint32_t voff = (tid / KB) * k + rk;
+
+    // backward: lane l holds the block at inner index c CB + l
+    int list = 0;
+    auto loadList = [&](int c) {
+        if constexpr (PH == PH_B)
+            list = a.blist[4 * (int64_t)(t.lst + t.ib0 + min(c * CB + lane, t.nib - 1)) + q];
+    };
+    // loads of the wave's block at inner index c CB + i (the zero block where
+    // it has none)
+    cx<T> m[U][4];
+    auto issue = [&](int u, int c, int i) {
+        int blk;
+        if constexpr (PH == PH_F) {
+            const int j = t.ib0 + c * CB + i;
+            blk = j >= blo && j < bhi ? base + j : a.zero;
+        } else {
+            blk = __builtin_amdgcn_readlane(list, i);
+        }
+        if (c * CB + i >= t.nib) blk = a.zero;
+        const cx<T>* p = a.F + (int64_t)blk * (kBlk * kBlk);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) m[u][st] = (p + (PH == PH_F ? 4 * kBlk * st : st))[loff];
+    };
+    cx<T> sa[SPT], sg[PH == PH_F ? SPT : 1];
+    auto stage = [&](int c) {
+        const int row0 = kBlk * (t.ib0 + c * CB);
+        if constexpr (PH == PH_F) {
+            const cx<T>* x = a.V + (int64_t)(t.x0 + row0) * k;
+            const cx<T>* g = a.V + (a.g1 + t.w0 + row0) * k;
+#pragma unroll
+            for (int p = 0; p < SPT; ++p) sa[p] = (x + p * RP * k)[voff];
+            if (!t.leaf) {
+#pragma unroll
+                for (int p = 0; p < SPT; ++p) sg[p] = (g + p * RP * k)[voff];
+            } else {
+#pragma unroll
+                for (int p = 0; p < SPT; ++p) sg[p] = czero<T>();
+            }
+        } else {
+            const int32_t* ix = src + c * CB * kBlk;
+            uint32_t sx[SPT];
+#pragma unroll
+            for (int p = 0; p < SPT; ++p) sx[p] = (uint32_t)(ix + p * RP)[tid / KB];
+#pragma unroll
+            for (int p = 0; p < SPT; ++p) sa[p] = a.V[sx[p] * (uint32_t)k + rk];
+        }
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int p = 0; p < SPT; ++p) {
+            const int c = tid / KB + RP * p;
+            // backward: inner index 4 a + b of a block sits at 4 b + a
+            const int row = PH == PH_F ? c : (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3);
+            cx<T> v = sa[p];
+            if constexpr (PH == PH_F) v = v + sg[p];
+            vs[row][tid % KB] = mk(v.r, v.i);
+        }
+    };
+    acc_t acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
+    // vector operands of the block at inner index i of the chunk
+    struct Operand {
+        cx<T> v[4][NB];
+    };
+    auto operand = [&](int i) {
+        Operand o;
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) o.v[st][n] = vs[kBlk * i + 4 * st + lk][8 * n + (li & 7)];
+        return o;
+    };
+    auto multiply = [&](int u, const Operand& o) {
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const cx<T> v = o.v[st][n];
+                const T b1 = li < 8 ? v.r : v.i;
+                const T b2 = li < 8 ? -v.i : v.r;
+                acc[n] = Mfma<T>::step(m[u][st].r, b1, acc[n]);
+                acc[n] = Mfma<T>::step(m[u][st].i, b2, acc[n]);
+            }
+    };
+    // finish operands of this lane's rows: D^-1, or where update rows go
+    const bool fin = own && t.slot < 0 && PH == PH_F;
+    uint32_t dst[4] = {0, 0, 0, 0};
+    cx<T> fd[PH == PH_F ? 4 : 1];
+    if (fin) {
+        if (top) {
+            const cx<T>* d = a.dinv + t.x0 + kBlk * ob;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) fd[PH == PH_F ? p : 0] = d[Mfma<T>::row(lk, p)];
+        } else {
+            const int32_t* d = a.udst + t.u0 + kBlk * (ob - t.sb);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) dst[p] = d[Mfma<T>::row(lk, p)];
+        }
+    }
+    // the chunk's products, half a ring at a time (blocks past the range are
+    // the zero block), each register group refilled as soon as it is used
+    auto run = [&](int c) {
+        const int left = t.nib - c * CB;
+        constexpr int H = U / 2;
+        Operand o = operand(0);
+        for (int i0 = 0;; i0 += U) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int u = H * h; u < H * h + H; ++u) {
+                    const Operand o1 = operand(min(i0 + u + 1, CB - 1));
+                    multiply(u, o);
+                    o = o1;
+                }
+                if (i0 + H * h + H >= left) return;
+#pragma unroll
+                for (int u = H * h; u < H * h + H; ++u) issue(u, c, i0 + u + U);
+            }
+            if (i0 + U >= CB) return;
+        }
+    };
+    loadList(0);
+    stage(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) issue(u, 0, u);
+    __builtin_amdgcn_sched_barrier(0);  // all loads go out before the first wait
+    put();
+    LdsBarrier();
+    run(0);
+    for (int c = 1; c < nch; ++c) {
+        loadList(c);
+        stage(c);
+        LdsBarrier();  // the previous chunk's readers are done
+        put();
+        LdsBarrier();
+        run(c);
+    }
+    if (own) {
+        cx<T> o[NB][4];
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                o[n][p] = cx<T>{T(acc[n][p]), T(__shfl_xor(acc[n][p], 8, 64))};
+        // element (n, p): row kBlk ob + row(lk, p), right-hand side 8 n + li
+        const int ru = kBlk * (ob - t.sb);  // first update row
+        auto each = [&](auto&& f) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) f(n, p, Mfma<T>::row(lk, p), 8 * n + li);
+        };
+        if (t.slot >= 0) {
+            cx<T>* out = a.P + ((int64_t)t.slot * 64 + kBlk * q) * k;
+            each([&](int n, int p, int row, int r) {
+                if (li < 8 && r < k) out[row * k + r] = o[n][p];
+            });
+        } else if (PH == PH_B) {
+            cx<T>* out = a.V + (int64_t)(t.x0 + kBlk * ob) * k;
+            each([&](int n, int p, int row, int r) {
+                if (li < 8 && r < k && kBlk * ob + row < t.s) out[row * k + r] = o[n][p];
+            });
+        } else if (top) {
+            cx<T>* out = a.V + (a.w + t.x0 + kBlk * ob) * k;
+            each([&](int n, int p, int row, int r) {
+                if (li < 8 && r < k && kBlk * ob + row < t.s)
+                    out[row * k + r] = o[n][p] * fd[PH == PH_F ? p : 0];
+            });
+        } else {
+            // an update row: the children's contributions to it and, for a
+            // pivot row of the parent, what that holds
+            const cx<T>* g0 = a.V + (a.g0 + t.u0 + ru) * k;
+            const cx<T>* g1 = a.V + (a.g1 + t.w0 + kBlk * ob) * k;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const int r = 8 * n + li, rc = min(r, k - 1);
+                cx<T> x[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) x[p] = a.V[dst[p] * (uint32_t)k + rc];
+                if (!t.leaf) {
+                    cx<T> ga[4], gb[4];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        ga[p] = g0[Mfma<T>::row(lk, p) * k + rc];
+                        gb[p] = g1[Mfma<T>::row(lk, p) * k + rc];
+                    }
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) o[n][p] = ga[p] + gb[p] + o[n][p];
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const cx<T> v = (int)dst[p] < a.xrows ? x[p] + o[n][p] : o[n][p];
+                    if (li < 8 && r < k && ru + Mfma<T>::row(lk, p) < t.u)
+                        a.V[dst[p] * (uint32_t)k + r] = v;
+                }
+            }
+        }
+    }
+    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, redc, reds);
+}
+
+// The same for wide blocks of right-hand sides: passes of up to KB = 32 or 64
+// over the tile, CB inner blocks at a time in two LDS buffers; the vector and
+// factor loads of the next chunks are in flight while a chunk is multiplied.
+template <typename T, int KB>
+struct WideShape {
+    static constexpr int NB = KB / 8;
+    static constexpr int CB = sizeof(T) == 4 && KB == 32 ? 4 : 2;
+    static constexpr int SPT = CB * kBlk * KB / 256;  // staged elements per thread
+};
+
+template <typename T, int PH, int KB>
+__device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBufs<T>& a, int k,
+                                              int32_t* redc, const BlockRed* reds)
+{
+    typedef typename Mfma<T>::acc acc_t;
+    typedef WideShape<T, KB> S;
+    constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT;
+    __shared__ cx<T> vs[2][CB * kBlk][KB];
+    const ConstInts tw = Const(tp);
+    const TileRec t(tw);
+    const int tid = threadIdx.x, lane = tid & 63, q = Uni(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ob = t.ob0 + q;
+    const int base = PH == PH_F ? tw[16 + q] : 0, blo = PH == PH_F ? tw[20 + q] : 0;
+    const int bhi = PH == PH_F ? tw[24 + q] : 0;
+    const ConstInts bl = Const(a.blist) + 4 * (int64_t)(t.lst + t.ib0) + q;
+    const int32_t* src = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0);
+    const uint32_t loff = PH == PH_F ? lk * kBlk + li : li * kBlk + 4 * lk;
+    const int nch = (t.nib + CB - 1) / CB;
+    struct Chunk {
+        cx<T> m[CB][4];
+    };
+    auto factor = [&](int c, Chunk& d) {
+#pragma unroll
+        for (int b = 0; b < CB; ++b) {
+            const int i = c * CB + b;
+            int blk = a.zero;
+            if (i < t.nib) {
+                if constexpr (PH == PH_F) {
+                    const int j = t.ib0 + i;
+                    if (j >= blo && j < bhi) blk = base + j;
+                } else {
+                    blk = bl[4 * i];
+                }
+            }
+            const cx<T>* p = a.F + (int64_t)blk * (kBlk * kBlk);
+#pragma unroll
+            for (int st = 0; st < 4; ++st) d.m[b][st] = (p + (PH == PH_F ? 4 * kBlk * st : st))[loff];
+        }
+    };
+    for (int r0 = 0; r0 < k; r0 += KB) {
+        const int kc = min(KB, k - r0);
+        acc_t acc[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
+        constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
+        const int rr = r0 + min(tid % KB, kc - 1);
+        const uint32_t voff = (tid / KB) * k + rr;
+        // (stages past the end read the last chunk again, unused)
+        int32_t sx[PH == PH_B ? SPT : 1];
+        auto indices = [&](int c) {
+            if constexpr (PH == PH_B) {
+                const int32_t* ix = src + min(c, nch - 1) * CB * kBlk;
+#pragma unroll
+                for (int p = 0; p < SPT; ++p) sx[p] = (ix + p * RP)[tid / KB];
+            }
+        };
+        cx<T> sa[SPT], sg[PH == PH_F ? SPT : 1];
+        auto stage = [&](int c) {
+            if constexpr (PH == PH_F) {
+                const int row0 = kBlk * (t.ib0 + min(c, nch - 1) * CB);
+                const cx<T>* x = a.V + (int64_t)(t.x0 + row0) * k;
+                const cx<T>* g = a.V + (a.g1 + t.w0 + row0) * k;
+#pragma unroll
+                for (int p = 0; p < SPT; ++p) sa[p] = (x + p * RP * k)[voff];
+                if (!t.leaf) {
+#pragma unroll
+                    for (int p = 0; p < SPT; ++p) sg[p] = (g + p * RP * k)[voff];
+                } else {
+#pragma unroll
+                    for (int p = 0; p < SPT; ++p) sg[p] = czero<T>();
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < SPT; ++p) sa[p] = a.V[(int64_t)sx[p] * k + rr];
+            }
+        };
+        auto put = [&](int buf) {
+#pragma unroll
+            for (int p = 0; p < SPT; ++p) {
+                const int c = tid / KB + RP * p;
+                const int row = PH == PH_F ? c : (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3);
+                cx<T> v = sa[p];
+                if constexpr (PH == PH_F) v = v + sg[p];
+                vs[buf][row][tid % KB] = mk(v.r, v.i);
+            }
+        };
+        Chunk d0, d1;
+        indices(0);
+        stage(0);
+        indices(1);
+        factor(0, d0);
+        factor(1, d1);
+        auto step = [&](int c, Chunk& d) {
+            put(c & 1);
+            stage(c + 1);
+            indices(c + 2);
+            LdsBarrier();
+#pragma unroll
+            for (int b = 0; b < CB; ++b)
+#pragma unroll
+                for (int st = 0; st < 4; ++st)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) {
+                        const cx<T> v = vs[c & 1][kBlk * b + 4 * st + lk][8 * n + (li & 7)];
+                        const T b1 = li < 8 ? v.r : v.i;
+                        const T b2 = li < 8 ? -v.i : v.r;
+                        acc[n] = Mfma<T>::step(d.m[b][st].r, b1, acc[n]);
+                        acc[n] = Mfma<T>::step(d.m[b][st].i, b2, acc[n]);
+                    }
+            factor(c + 2, d);
+        };
+        for (int c = 0; c < nch; c += 2) {
+            step(c, d0);
+            if (c + 1 >= nch) break;
+            step(c + 1, d1);
+        }
+        if (q < t.nob) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const T val = acc[n][p];
+                    const T other = __shfl_xor(val, 8, 64);
+                    const int rl = Mfma<T>::row(lk, p), rr = 8 * n + li;
+                    if (li >= 8 || rr >= kc) continue;
+                    const cx<T> v{val, other};
+                    if (t.slot >= 0)
+                        a.P[((int64_t)t.slot * 64 + kBlk * q + rl) * k + r0 + rr] = v;
+                    else
+                        BlockFinish<T, PH>(a, t.x0, t.w0, t.u0, t.s, t.u, t.sb, t.leaf,
+                                           kBlk * ob + rl, r0 + rr, k, v);
+                }
+            }
+        }
+        LdsBarrier();  // the next pass overwrites the staged chunks
+    }
+    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, redc, reds);
+}
+
+// KB right-hand sides per pass: 8 and 16 one pass, 32 and 64 as many as k needs.
+template <typename T, int PH, int KB>
+__device__ __forceinline__ void BlockWork(const BlockTile* tp, const BlockBufs<T>& a, int k,
+                                          int32_t* redc, const BlockRed* reds)
+{
+    if constexpr (KB <= 16)
+        BlockTileWork<T, PH, KB>(tp, a, k, redc, reds);
+    else
+        BlockTileWide<T, PH, KB>(tp, a, k, redc, reds);
+}
+
+// Workgroups per CU the register budget allows for (the most without spills).
+template <typename T, int PH, int KB>
+constexpr int BlockOccupancy()
+{
+    if (KB > 16) return 2;
+    return PH == PH_B ? 6 : 4;
+}
+
+template <typename T, int PH, int KB>
+__global__ __launch_bounds__(256, (BlockOccupancy<T, PH, KB>())) void k_block(
+    const BlockTile* tiles, BlockBufs<T> a, int k, int32_t* redc, const BlockRed* reds)
+{
+    const BlockTile* tp = tiles + blockIdx.x;
+    if (Const(tp)[8] <= 0) return;  // a hole of the XCD placement
+    BlockWork<T, PH, KB>(tp, a, k, redc, reds);
+}
+
+// Sum of the slices of one tile in slot order, then the finish (where the
+// product launch does not do it).
+template <typename T, int PH>
+__device__ __forceinline__ void BlockReduceItem(const BlockRed& it, const BlockBufs<T>& a, int k)
+{
+    for (int e = threadIdx.x; e < it.nob * kBlk * k; e += kThreads) {
+        const int rl = e / k, r = e % k;
+        cx<T> v = czero<T>();
+        for (int j = 0; j < it.nslots; ++j)
+            v = v + a.P[((int64_t)(it.slot0 + j) * 64 + rl) * k + r];
+        BlockFinish<T, PH>(a, it.x0, it.w0, it.u0, it.s, it.u, it.sb, it.leaf, kBlk * it.ob0 + rl,
+                           r, k, v);
+    }
+}
+
+template <typename T, int PH>
+__global__ __launch_bounds__(kThreads) void k_block_reduce(const BlockRed* reds, BlockBufs<T> a,
+                                                           int k)
+{
+    BlockReduceItem<T, PH>(reds[blockIdx.x], a, k);
+}
+
+// --------------------------------------------------------------------------
+// Fold: the merged fronts' F from the factored fine fronts (L after the
+// selective inversion: Linv below the diagonal, D on it, L_BL below; E =
+// -L_BL Linv from a batched product).
+// --------------------------------------------------------------------------
+// Address of (row, column) of a merged front in F.
+__device__ __forceinline__ int64_t BlockAt(int browBase, int row, int col)
+{
+    return (int64_t)(browBase + (col >> 4)) * (kBlk * kBlk) + (col & 15) * kBlk + (row & 15);
+}
+
+// Copies a 32 x 32 piece of a node's front: its own lower triangle (with the
+// unit diagonal; D^-1 goes to dinv), or rows of E of a group's top node.
+// Entries of F outside every piece stay zero from its allocation.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_pack(const TransItem* items, const FoldNode* nodes,
+                                                   const int32_t* browBase, const cx<T>* L,
+                                                   int64_t fstore, const cx<T>* E, int64_t estride,
+                                                   cx<T>* F, int64_t fentries, cx<T>* dinv,
+                                                   int xrows)
+{
+    const TransItem it = items[blockIdx.x];
+    const FoldNode f = nodes[it.node];
+    const cx<T>* Lf = L + (int64_t)blockIdx.y * fstore + f.l;
+    const cx<T>* Ef = E + (int64_t)blockIdx.y * estride + f.e;
+    cx<T>* Fp = F + (int64_t)blockIdx.y * fentries;
+    const int fs = f.s + f.u, i = it.i0 + (threadIdx.x & 31);
+    const bool own = it.i0 < f.s;
+    if (i >= (own ? f.s : fs)) return;
+    const int row = own ? f.mcol + i : f.urow + i - f.s;
+    const int bb = browBase[f.br0 + (row >> 4)];
+    for (int j = it.j0 + (threadIdx.x >> 5); j < min(it.j0 + 32, f.s); j += 8) {
+        if (own && i < j) break;
+        cx<T> v;
+        if (!own) {
+            v = Ef[i - f.s + (int64_t)j * f.u];
+        } else {
+            v = Lf[i + (int64_t)j * fs];
+            if (i == j) {
+                dinv[(int64_t)blockIdx.y * xrows + f.x0 + i] = cinv(v);
+                v = cx<T>{T(1), T(0)};
+            }
+        }
+        Fp[BlockAt(bb, row, f.mcol + j)] = v;
+    }
+}
+
+// Columns of a node below its group's top: F_c = F_A P + ext(E_c) (see
+// ComposeDesc), one 64 x 64 tile per workgroup through the tile engine.
+template <typename T>
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_compose(
+    const GemmTile* tiles, const ComposeDesc* descs, const int32_t* flist, const int32_t* fsrc,
+    const ComposeKey* fkeys, const int32_t* browBase, const cx<T>* E, int64_t estride, cx<T>* F, int64_t fentries)
+{
+    constexpr int BK = 8, TS = 64;
+    __shared__ cx<T> As[2][BK][TS + 1];
+    __shared__ cx<T> Bs[2][BK][TS + 1];
+    __shared__ int rowOf[TS], baseOf[TS], srcOf[TS];
+    const GemmTile tl = tiles[blockIdx.x];
+    const ComposeDesc g = descs[tl.desc];
+    const cx<T>* Ec = E + (int64_t)blockIdx.y * estride + g.e;
+    cx<T>* Fp = F + (int64_t)blockIdx.y * fentries;
+    const int tm = tl.tm, tn = tl.tn;
+    if (threadIdx.x < TS) {
+        const int i = min(tm + (int)threadIdx.x, g.rows - 1);
+        const int row = flist[g.list + i];
+        rowOf[threadIdx.x] = row;
+        baseOf[threadIdx.x] = browBase[g.br0 + (row >> 4)];
+        srcOf[threadIdx.x] = fsrc[g.src + i];
+    }
+    __syncthreads();
+    const ComposeKey* keys = fkeys + g.kl;
+    // F_A is lower triangular: entries past a pivot row are not stored, and
+    // the row's diagonal is read instead, unused
+    struct RawA {
+        cx<T> v;
+        int pos;
+    };
+    auto la = [&](int i, int k) {
+        const ComposeKey key = keys[k];
+        const int col = tm + i >= key.pos ? key.col : rowOf[i];
+        return RawA{Fp[BlockAt(baseOf[i], rowOf[i], col)], key.pos};
+    };
+    auto fa = [&](int i, int, const RawA& a) {
+        return tm + i < g.rows && tm + i >= a.pos ? a.v : czero<T>();
+    };
+    auto lb = [&](int k, int j) {
+        return Ec[keys[k].row + (int64_t)min(tn + j, g.n - 1) * g.lde];
+    };
+    auto fb = [&](int, int j, cx<T> v) { return tn + j < g.n ? v : czero<T>(); };
+    typename Mfma<T>::acc acc[TileShape<TS, TS>::RB][TileShape<TS, TS>::CB];
+    MmaTile<T, TS, false, BK, TS>(la, fa, lb, fb, 0, tl.pad_, As, Bs, acc);
+    auto ld = [&](int i, int j) {
+        return Ec[max(srcOf[i], 0) + (int64_t)min(tn + j, g.n - 1) * g.lde];
+    };
+    MmaEpilogue<T, TS, TS>(acc, ld, [&](int i, int j, cx<T> v, cx<T> e) {
+        if (tm + i >= g.rows || tn + j >= g.n) return;
+        if (tm + i >= g.piv && srcOf[i] >= 0) v = v + e;
+        Fp[BlockAt(baseOf[i], rowOf[i], g.ccol + tn + j)] = v;
+    });
+}
+
+// --------------------------------------------------------------------------
 // Batched panel solves: one launch runs the same step (a tree level's
 // products or reduce, a panel copy) of the sweeps of many independent
 // problems.  Every workgroup reads its BatchBlock: the tile or reduce item it
@@ -2053,31 +2098,35 @@ __global__ __launch_bounds__(kThreads) void k_mv_reduce(const SolveTile* items, 
 // workgroups then exit at once).  The work of a workgroup is that of the
 // single-problem kernels, with the same summation order.
 // --------------------------------------------------------------------------
-template <typename T, int PH, int RT, int KB, int NWV>
-__global__ __launch_bounds__(64 * NWV) PSP_MVM_OCCUPANCY void k_mvm_batch(
-    const BatchBlock* blocks, const BatchSolveSeg* segs, const int32_t* active)
+template <typename T>
+__device__ __forceinline__ BlockBufs<T> SegBufs(const BatchSolveSeg& sg)
+{
+    return BlockBufs<T>{(const cx<T>*)sg.F, (cx<T>*)sg.V, sg.bsrc, sg.blist, sg.udst,
+                        (const cx<T>*)sg.dinv, (cx<T>*)sg.P, sg.w, sg.g0, sg.g1, sg.xrows,
+                        sg.zero};
+}
+
+template <typename T, int PH, int KB>
+__global__ __launch_bounds__(256, (BlockOccupancy<T, PH, KB>())) void k_block_batch(const BatchBlock* blocks,
+                                                     const BatchSolveSeg* segs,
+                                                     const int32_t* active)
 {
     const BatchBlock bb = blocks[blockIdx.x];
-    const SolveTile tl = *bb.item;
+    const BlockTile* tp = (const BlockTile*)bb.item;
     const BatchSolveSeg sg = segs[bb.seg];
-    if (!active[bb.problem] || tl.nrows <= 0) return;
-    const Slots<T> gs{(cx<T>*)sg.G, sg.half, sg.relinds};
-    MvmTile<T, PH, RT, KB, NWV>(tl, sg.structs, gs, (const cx<T>*)sg.L, (const cx<T>*)sg.LT,
-                                (cx<T>*)sg.Xp, (cx<T>*)sg.W, (cx<T>*)sg.P, sg.k, nullptr,
-                                nullptr);
+    if (!active[bb.problem] || Const(tp)[8] <= 0) return;
+    BlockWork<T, PH, KB>(tp, SegBufs<T>(sg), sg.k, nullptr, nullptr);
 }
 
 template <typename T, int PH>
-__global__ __launch_bounds__(kThreads) void k_mv_reduce_batch(const BatchBlock* blocks,
-                                                              const BatchSolveSeg* segs,
-                                                              const int32_t* active)
+__global__ __launch_bounds__(kThreads) void k_block_reduce_batch(const BatchBlock* blocks,
+                                                                 const BatchSolveSeg* segs,
+                                                                 const int32_t* active)
 {
     const BatchBlock bb = blocks[blockIdx.x];
-    const SolveTile it = *bb.item;
     const BatchSolveSeg sg = segs[bb.seg];
     if (!active[bb.problem]) return;
-    const Slots<T> gs{(cx<T>*)sg.G, sg.half, sg.relinds};
-    MvReduceItem<T, PH>(it, gs, (cx<T>*)sg.Xp, (cx<T>*)sg.W, (const cx<T>*)sg.P, sg.k);
+    BlockReduceItem<T, PH>(*(const BlockRed*)bb.item, SegBufs<T>(sg), sg.k);
 }
 
 // LT[:, :s] = Linv^T D^-1 per front (upper triangle; D^-1 on the diagonal),
@@ -2634,24 +2683,6 @@ void LaunchInvDiag(const ClassDev& c, int nb, hipStream_t s)
                        (cx<T>*)c.L, c.fstore);
 }
 
-// Workgroups of a persistent solve launch: as many as fit on the device at
-// once, more only when a workgroup would otherwise get over kMvpTiles tiles.
-template <typename T, int PH, int RT, int KB>
-int MvpGrid(int cus, int count, int cap0 = 0)
-{
-    static const int perCU = [] {
-        int b = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_mvp<T, PH, RT, KB>, 256, 0) !=
-                hipSuccess ||
-            b < 1)
-            b = 1;
-        return b;
-    }();
-    const int fit = cap0 > 0 ? cap0 : perCU * std::max(cus, 1);
-    const int cap = std::max(fit, (count + kMvpTiles - 1) / kMvpTiles);
-    return std::max(1, std::min(count, cap));
-}
-
 // Workgroups of a fused launch: as many as fit on the device at once.
 template <typename T, int PH, int RT, int KB>
 int MvqGrid(int cus)
@@ -2671,12 +2702,6 @@ void PrimeSolveOccupancy()
 {
     auto prime = [](auto t) {
         typedef decltype(t) T;
-        (void)MvpGrid<T, PH_F, 64, 8>(1, 1), (void)MvpGrid<T, PH_F, 32, 8>(1, 1);
-        (void)MvpGrid<T, PH_F, 16, 8>(1, 1), (void)MvpGrid<T, PH_F, 64, 16>(1, 1);
-        (void)MvpGrid<T, PH_F, 32, 16>(1, 1), (void)MvpGrid<T, PH_F, 16, 16>(1, 1);
-        (void)MvpGrid<T, PH_B, 64, 8>(1, 1), (void)MvpGrid<T, PH_B, 32, 8>(1, 1);
-        (void)MvpGrid<T, PH_B, 16, 8>(1, 1), (void)MvpGrid<T, PH_B, 64, 16>(1, 1);
-        (void)MvpGrid<T, PH_B, 32, 16>(1, 1), (void)MvpGrid<T, PH_B, 16, 16>(1, 1);
         (void)MvqGrid<T, PH_F, 64, 8>(1), (void)MvqGrid<T, PH_F, 32, 8>(1);
         (void)MvqGrid<T, PH_F, 16, 8>(1), (void)MvqGrid<T, PH_F, 64, 16>(1);
         (void)MvqGrid<T, PH_F, 32, 16>(1), (void)MvqGrid<T, PH_F, 16, 16>(1);
@@ -2688,10 +2713,96 @@ void PrimeSolveOccupancy()
     prime(double());
 }
 
+// Start and end of a timed product launch, and its algorithmic work.
+static void ProfBegin(MvProfile* prof, hipStream_t s)
+{
+    if (prof) (void)hipEventRecord(prof->a, s);
+}
+
+static void ProfEnd(MvProfile* prof, hipStream_t s, double bytes, double flops)
+{
+    if (!prof) return;
+    (void)hipEventRecord(prof->b, s);
+    (void)hipEventSynchronize(prof->b);
+    float ms = 0;
+    (void)hipEventElapsedTime(&ms, prof->a, prof->b);
+    prof->launches += 1;
+    prof->seconds += ms * 1e-3;
+    prof->bytes += bytes;
+    prof->flops += flops;
+}
+
 template <typename T>
-void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* Xpv, void* Wv, void* Pv,
-                      void* Gv, int k, hipStream_t s, MvProfile* prof, int onlyLevel,
-                      int onlyPhase, int32_t* sync)
+void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, void* P, int k,
+                      hipStream_t s, MvProfile* prof, int onlyGroup, int onlyPhase)
+{
+    const VecRows vr(plan);
+    const BlockBufs<T> bufs{(const cx<T>*)c.F + (int64_t)b * c.fentries,
+                            (cx<T>*)V,
+                            c.bsrc,
+                            c.blist,
+                            c.udst,
+                            (const cx<T>*)c.dinv + (int64_t)b * c.xrows,
+                            (cx<T>*)P,
+                            vr.w,
+                            vr.g0,
+                            vr.g1,
+                            c.xrows,
+                            plan.nblocks};
+    // the partial sums are read through a buffer of at most 4 GiB
+    const bool pfits = (int64_t)sizeof(cx<T>) * k * 64 * plan.bslots < ((int64_t)1 << 32);
+    int32_t* rc = pfits ? c.bredc : nullptr;
+    auto go = [&](auto ph, int g) {
+        constexpr int PH = decltype(ph)::value;
+        const ClassPlan::BlockLevel& L = plan.blevels[g];
+        if (L.count[PH] <= 0) return;
+        auto run = [&](auto kb) {
+            hipLaunchKernelGGL((k_block<T, PH, decltype(kb)::value>), dim3(L.count[PH]), dim3(256),
+                               0, s, c.btiles + L.start[PH], bufs, k, rc, c.breds);
+        };
+        ProfBegin(prof, s);
+        if (k <= 8)
+            run(std::integral_constant<int, 8>());
+        else if (k <= 16)
+            run(std::integral_constant<int, 16>());
+        else if (k <= 32)
+            run(std::integral_constant<int, 32>());
+        else
+            run(std::integral_constant<int, 64>());
+        ProfEnd(prof, s, sizeof(cx<T>) * (L.entries[PH] + L.vecRows[PH] * k),
+                8.0 * L.entries[PH] * k);
+        if (L.rcount[PH] > 0 && !rc)
+            hipLaunchKernelGGL((k_block_reduce<T, PH>), dim3(L.rcount[PH]), dim3(kThreads), 0, s,
+                               c.breds + L.rstart[PH], bufs, k);
+    };
+    const int ng = (int)plan.blevels.size();
+    const std::integral_constant<int, PH_F> F;
+    const std::integral_constant<int, PH_B> B;
+    if (onlyGroup >= 0) {  // one launch, for tuning
+        if (onlyPhase == PH_F)
+            go(F, onlyGroup);
+        else
+            go(B, onlyGroup);
+        return;
+    }
+    for (int g = ng - 1; g >= 0; --g) go(F, g);
+    for (int g = 0; g < ng; ++g) go(B, g);
+}
+
+bool FusedApplies(const ClassDev& c, const ClassPlan& plan, int k, int64_t eb)
+{
+    // the fused kernel reads its vectors through buffer descriptors: each
+    // buffer must span less than 4 GiB
+    const int64_t span = (int64_t)1 << 32;
+    return c.nqueues > 0 && plan.qcut >= 0 && k >= 8 && k <= 16 &&
+           eb * k * (2 * c.wstore + kSolvePad + 2) < span &&
+           eb * k * (int64_t)(c.n + kSolvePad + 2) < span &&
+           eb * k * 64 * (int64_t)plan.maxSlots < span;
+}
+
+template <typename T>
+void LaunchPanelSolveFused(const ClassDev& c, const ClassPlan& plan, int b, void* Xpv, void* Wv,
+                           void* Pv, void* Gv, int k, hipStream_t s, MvProfile* prof, int32_t* sync)
 {
     const cx<T>* L = (const cx<T>*)c.L + (int64_t)b * c.fstore;
     const cx<T>* LT = (const cx<T>*)c.LT + (int64_t)b * c.fstore;
@@ -2699,159 +2810,80 @@ void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* Xpv
     cx<T>* W = (cx<T>*)Wv;
     cx<T>* P = (cx<T>*)Pv;
     const Slots<T> gs{(cx<T>*)Gv, c.wstore * k, c.relinds};
-    auto mv = [&](auto ph, const ClassPlan::SolveLevel& lv, const ClassPlan::Range& r) {
-        if (r.count <= 0) return;
-        constexpr int PH = decltype(ph)::value;
-        bool reduced = false;  // split row blocks already summed by the product launch
-        if (prof) (void)hipEventRecord(prof->a, s);
-        if (k >= 32) {
-            if (r.rows == 64)
-                hipLaunchKernelGGL((k_mmw<T, PH, 64>), dim3(r.count), dim3(256), 0, s, c.mv,
-                                   r.start, c.structs, gs, L, LT, Xp, W, P, k);
-            else if (r.rows == 32)
-                hipLaunchKernelGGL((k_mmw<T, PH, 32>), dim3(r.count), dim3(256), 0, s, c.mv,
-                                   r.start, c.structs, gs, L, LT, Xp, W, P, k);
-            else
-                hipLaunchKernelGGL((k_mmw<T, PH, 16>), dim3(r.count), dim3(256), 0, s, c.mv,
-                                   r.start, c.structs, gs, L, LT, Xp, W, P, k);
-        } else if (k >= 8 && k <= 16 && r.persist && r.waves == 4) {
-            auto launchP = [&](auto rt, auto kb) {
-                constexpr int RT = decltype(rt)::value, KB = decltype(kb)::value;
-                const int G = MvpGrid<T, PH, RT, KB>(c.cus, r.count, c.mvpGrid);
-                hipLaunchKernelGGL((k_mvp<T, PH, RT, KB>), dim3(G), dim3(256), 0, s, c.mv,
-                                   r.start, r.count, c.structs, gs, L, LT, Xp, W, P, k);
-            };
-            auto byRowsP = [&](auto kb) {
-                if (r.rows == 64)
-                    launchP(std::integral_constant<int, 64>(), kb);
-                else if (r.rows == 32)
-                    launchP(std::integral_constant<int, 32>(), kb);
-                else
-                    launchP(std::integral_constant<int, 16>(), kb);
-            };
-            if (k <= 8)
-                byRowsP(std::integral_constant<int, 8>());
-            else
-                byRowsP(std::integral_constant<int, 16>());
-        } else if (k >= 8) {
-            // split row blocks summed in the launch (slices placed per XCD;
-            // the partial sums are read through a buffer of at most 4 GiB)
-            const bool pfits = (int64_t)sizeof(cx<T>) * k * 64 * plan.maxSlots < ((int64_t)1 << 32);
-            int32_t* rc = r.xcd && c.redc && pfits ? c.redc : nullptr;
-            reduced = rc != nullptr;
-            auto launch = [&](auto rt, auto kb) {
-                constexpr int RT = decltype(rt)::value, KB = decltype(kb)::value;
-                if (r.waves == 16)
-                    hipLaunchKernelGGL((k_mvm<T, PH, RT, KB, 16>), dim3(r.count), dim3(1024), 0,
-                                       s, c.mv, r.start, c.structs, gs, L, LT, Xp, W, P, k, rc,
-                                       c.mvred);
-                else
-                    hipLaunchKernelGGL((k_mvm<T, PH, RT, KB, 4>), dim3(r.count), dim3(256), 0, s,
-                                       c.mv, r.start, c.structs, gs, L, LT, Xp, W, P, k, rc,
-                                       c.mvred);
-            };
-            auto byRows = [&](auto kb) {
-                if (r.rows == 64)
-                    launch(std::integral_constant<int, 64>(), kb);
-                else if (r.rows == 32)
-                    launch(std::integral_constant<int, 32>(), kb);
-                else
-                    launch(std::integral_constant<int, 16>(), kb);
-            };
-            if (k <= 8)
-                byRows(std::integral_constant<int, 8>());
-            else
-                byRows(std::integral_constant<int, 16>());
-        } else if (r.rows == 64)
-            hipLaunchKernelGGL((k_mv<T, PH, 64>), dim3(r.count), dim3(kMvThreads), 0, s, c.mv,
-                               r.start, c.structs, gs, L, LT, Xp, W, P, k);
-        else if (r.rows == 32)
-            hipLaunchKernelGGL((k_mv<T, PH, 32>), dim3(r.count), dim3(kMvThreads), 0, s, c.mv,
-                               r.start, c.structs, gs, L, LT, Xp, W, P, k);
-        else
-            hipLaunchKernelGGL((k_mv<T, PH, 16>), dim3(r.count), dim3(kMvThreads), 0, s, c.mv,
-                               r.start, c.structs, gs, L, LT, Xp, W, P, k);
-        if (prof) {
-            (void)hipEventRecord(prof->b, s);
-            (void)hipEventSynchronize(prof->b);
-            float ms = 0;
-            (void)hipEventElapsedTime(&ms, prof->a, prof->b);
-            prof->launches += 1;
-            prof->seconds += ms * 1e-3;
-            const double eb = sizeof(cx<T>);
-            prof->bytes += eb * (lv.entries[PH] + lv.vecRows[PH] * k);
-            prof->flops += 8.0 * lv.entries[PH] * k;
-        }
-        if (r.rcount > 0 && !reduced)
-            hipLaunchKernelGGL((k_mv_reduce<T, PH>), dim3(r.rcount), dim3(kThreads), 0, s,
-                               c.mvred, r.rstart, gs, Xp, W, P, k);
-    };
-    if (onlyLevel >= 0) {  // one (level, phase) launch, for tile-shape tuning
-        const ClassPlan::SolveLevel& lv = plan.solveLevels[onlyLevel];
-        if (onlyPhase == PH_F)
-            mv(std::integral_constant<int, PH_F>(), lv, lv.f);
-        else
-            mv(std::integral_constant<int, PH_B>(), lv, lv.b);
-        return;
-    }
-    // Fused subtree launches: the levels from the cut down as one launch
-    // per phase (8 <= k <= 16, with the class's launch state to count on).
-    // (the fused kernel reads its vectors through buffer descriptors: each
-    // buffer must span less than 4 GiB)
-    const int64_t eb_ = sizeof(cx<T>), span = (int64_t)1 << 32;
-    const bool fits = eb_ * k * (2 * c.wstore + kSolvePad + 2) < span &&
-                      eb_ * k * (int64_t)(c.n + kSolvePad + 2) < span &&
-                      eb_ * k * 64 * (int64_t)plan.maxSlots < span;
-    const bool fused = sync && c.nqueues > 0 && plan.qcut >= 0 && k >= 8 && k <= 16 && fits;
-    auto fusedLaunch = [&](auto ph) {
-        constexpr int PH = decltype(ph)::value;
-        const int nt = c.nqtiles[PH];
-        if (nt <= 0) return;
-        int32_t* st = sync + (PH == PH_F ? 0 : QueueSyncInts(c.nnodes, c.nqueues, c.nqreds[0]));
-        if (prof) (void)hipEventRecord(prof->a, s);
-        auto go = [&](auto rt, auto kb) {
-            constexpr int RT = decltype(rt)::value, KB = decltype(kb)::value;
-            const int G = std::max(1, std::min(nt, MvqGrid<T, PH, RT, KB>(c.cus)));
-            hipLaunchKernelGGL((k_mvq<T, PH, RT, KB>), dim3(G), dim3(256), 0, s, c.qtiles[PH],
-                               c.qstart[PH], c.qreds[PH], c.qdep[PH], c.nodes, st, c.nnodes,
-                               c.nqueues, c.structs, gs, L, LT, Xp, W, P, k);
-        };
+    const double eb = sizeof(cx<T>);
+    auto byKb = [&](int rows, const auto& go) {
         auto byRows = [&](auto kb) {
-            if (c.queueRows == 64)
+            if (rows == 64)
                 go(std::integral_constant<int, 64>(), kb);
-            else if (c.queueRows == 16)
-                go(std::integral_constant<int, 16>(), kb);
-            else
+            else if (rows == 32)
                 go(std::integral_constant<int, 32>(), kb);
+            else
+                go(std::integral_constant<int, 16>(), kb);
         };
         if (k <= 8)
             byRows(std::integral_constant<int, 8>());
         else
             byRows(std::integral_constant<int, 16>());
-        if (prof) {
-            (void)hipEventRecord(prof->b, s);
-            (void)hipEventSynchronize(prof->b);
-            float ms = 0;
-            (void)hipEventElapsedTime(&ms, prof->a, prof->b);
-            prof->launches += 1;
-            prof->seconds += ms * 1e-3;
-            const double eb = sizeof(cx<T>);
-            const ClassPlan::QueuePhase& Q = plan.queue[PH];
-            prof->bytes += eb * (Q.entries + Q.vecRows * k);
-            prof->flops += 8.0 * Q.entries * k;
-        }
     };
-    const int lowest = fused ? plan.qcut : plan.maxDepth + 1;  // first level of the fused launch
-    if (fused) fusedLaunch(std::integral_constant<int, PH_F>());
-    for (int d = std::min(plan.maxDepth, lowest - 1); d >= 0; --d) {
+    // one level above the cut; split row blocks are summed in the launch
+    // where their slices were placed per XCD
+    auto level = [&](auto ph, int d) {
+        constexpr int PH = decltype(ph)::value;
         const ClassPlan::SolveLevel& lv = plan.solveLevels[d];
-        mv(std::integral_constant<int, PH_F>(), lv, lv.f);
-    }
-    for (int d = 0; d < std::min(plan.maxDepth + 1, lowest); ++d) {
-        const ClassPlan::SolveLevel& lv = plan.solveLevels[d];
-        mv(std::integral_constant<int, PH_B>(), lv, lv.b);
-    }
-    if (fused) fusedLaunch(std::integral_constant<int, PH_B>());
+        const ClassPlan::Range& r = PH == PH_F ? lv.f : lv.b;
+        if (r.count <= 0) return;
+        int32_t* rc = r.xcd ? c.redc : nullptr;
+        ProfBegin(prof, s);
+        byKb(r.rows, [&](auto rt, auto kb) {
+            hipLaunchKernelGGL((k_mvm<T, PH, decltype(rt)::value, decltype(kb)::value>),
+                               dim3(r.count), dim3(256), 0, s, c.mv, r.start, c.structs, gs, L, LT,
+                               Xp, W, P, k, rc, c.mvred);
+        });
+        ProfEnd(prof, s, eb * (lv.entries[PH] + lv.vecRows[PH] * k), 8.0 * lv.entries[PH] * k);
+        if (r.rcount > 0 && !rc)
+            hipLaunchKernelGGL((k_mv_reduce<T, PH>), dim3(r.rcount), dim3(kThreads), 0, s,
+                               c.mvred, r.rstart, gs, Xp, W, P, k);
+    };
+    auto subtrees = [&](auto ph) {
+        constexpr int PH = decltype(ph)::value;
+        const int nt = c.nqtiles[PH];
+        if (nt <= 0) return;
+        int32_t* st = sync + (PH == PH_F ? 0 : QueueSyncInts(c.nnodes, c.nqueues, c.nqreds[0]));
+        ProfBegin(prof, s);
+        byKb(c.queueRows, [&](auto rt, auto kb) {
+            constexpr int RT = decltype(rt)::value, KB = decltype(kb)::value;
+            const int G = std::max(1, std::min(nt, MvqGrid<T, PH, RT, KB>(c.cus)));
+            hipLaunchKernelGGL((k_mvq<T, PH, RT, KB>), dim3(G), dim3(256), 0, s, c.qtiles[PH],
+                               c.qstart[PH], c.qreds[PH], c.qdep[PH], c.nodes, st, c.nnodes,
+                               c.nqueues, c.structs, gs, L, LT, Xp, W, P, k);
+        });
+        const ClassPlan::QueuePhase& Q = plan.queue[PH];
+        ProfEnd(prof, s, eb * (Q.entries + Q.vecRows * k), 8.0 * Q.entries * k);
+    };
+    const std::integral_constant<int, PH_F> F;
+    const std::integral_constant<int, PH_B> B;
+    subtrees(F);
+    for (int d = std::min(plan.maxDepth, plan.qcut - 1); d >= 0; --d) level(F, d);
+    for (int d = 0; d < std::min(plan.maxDepth + 1, plan.qcut); ++d) level(B, d);
+    subtrees(B);
+}
+
+template <typename T>
+void LaunchPack(const ClassDev& c, hipStream_t s)
+{
+    if (c.npacks <= 0) return;
+    hipLaunchKernelGGL((k_pack<T>), dim3(c.npacks, c.npanels), dim3(kThreads), 0, s, c.packs,
+                       c.foldNodes, c.browBase, (const cx<T>*)c.L, c.fstore, (const cx<T>*)c.U,
+                       c.ustore, (cx<T>*)c.F, c.fentries, (cx<T>*)c.dinv, c.xrows);
+}
+
+template <typename T>
+void LaunchCompose(const ClassDev& c, int tileStart, int tileCount, hipStream_t s)
+{
+    if (tileCount <= 0) return;
+    hipLaunchKernelGGL((k_compose<T>), dim3(tileCount, c.npanels), dim3(256), 0, s,
+                       c.composeTiles + tileStart, c.compose, c.flist, c.fsrc, c.fkeys, c.browBase,
+                       (const cx<T>*)c.U, c.ustore, (cx<T>*)c.F, c.fentries);
 }
 
 template <typename T>
@@ -2871,68 +2903,59 @@ void LaunchFoldBack(const ClassDev& c, hipStream_t s)
 }
 
 template <typename T>
-void LaunchCopyIn(const ClassDev& c, const c128* B, void* Xp, int k, int nx, int ny, int nz,
-                  int vOffset, int padding, hipStream_t s, int32_t* sync)
+void LaunchCopyIn(const PanelMap& m, const c128* B, void* Xp, int k, int nx, int ny, int nz,
+                  int vOffset, int padding, hipStream_t s, int32_t* sync, int nsync)
 {
-    hipLaunchKernelGGL((k_copy_in<T>), dim3(Blocks((int64_t)c.n * k)), dim3(kThreads), 0, s, c.n,
-                       k, c.qxy, c.qv, B, (cx<T>*)Xp, nx, ny, nz, vOffset, padding, sync,
-                       sync ? c.nsync : 0);
+    hipLaunchKernelGGL((k_copy_in<T>), dim3(Blocks((int64_t)m.n * k)), dim3(kThreads), 0, s, m.n,
+                       k, m.xy, m.v, B, (cx<T>*)Xp, nx, ny, nz, vOffset, padding, sync,
+                       sync ? nsync : 0);
 }
 
 template <typename T>
-void LaunchCopyOut(const ClassDev& c, c128* B, const void* Xp, int k, int nx, int ny, int nz,
+void LaunchCopyOut(const PanelMap& m, c128* B, const void* Xp, int k, int nx, int ny, int nz,
                    int vOffset, int padding, int mode, hipStream_t s, const StencilArgs* st,
                    const double* vel, int v1)
 {
     const StencilArgs none{};
-    hipLaunchKernelGGL((k_copy_out<T>), dim3(Blocks((int64_t)c.n * k)), dim3(kThreads), 0, s, c.n,
-                       k, c.qxy, c.qv, B, (const cx<T>*)Xp, nx, ny, nz, vOffset, padding, mode,
+    hipLaunchKernelGGL((k_copy_out<T>), dim3(Blocks((int64_t)m.n * k)), dim3(kThreads), 0, s, m.n,
+                       k, m.xy, m.v, B, (const cx<T>*)Xp, nx, ny, nz, vOffset, padding, mode,
                        st ? *st : none, vel, st ? v1 : -1);
 }
 
 template <typename T>
-void LaunchZeroSetPlane(const ClassDev& c, const StencilArgs& st, const double* vel,
+void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* vel,
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,
-                        int32_t* sync)
+                        int32_t* sync, int nsync)
 {
-    hipLaunchKernelGGL((k_zero_set_plane<T>), dim3(Blocks((int64_t)c.n * k)), dim3(kThreads), 0, s,
-                       c.n, k, c.qxy, c.qv, st, vel, B, (cx<T>*)Xp, v2, vlLast, sync,
-                       sync ? c.nsync : 0);
+    hipLaunchKernelGGL((k_zero_set_plane<T>), dim3(Blocks((int64_t)m.n * k)), dim3(kThreads), 0, s,
+                       m.n, k, m.xy, m.v, st, vel, B, (cx<T>*)Xp, v2, vlLast, sync,
+                       sync ? nsync : 0);
 }
 
 template <typename T>
-void LaunchSolveBatch(int ph, int rows, int waves, int kb, const BatchBlock* blocks, int nblocks,
+void LaunchSolveBatch(int ph, int kb, const BatchBlock* blocks, int nblocks,
                       const BatchSolveSeg* segs, const int32_t* active, hipStream_t s)
 {
     if (nblocks <= 0) return;
-    auto go = [&](auto phc, auto rt) {
-        constexpr int PH = decltype(phc)::value, RT = decltype(rt)::value;
-        auto byKb = [&](auto kbc) {
-            constexpr int KB = decltype(kbc)::value;
-            if (waves == 16)
-                hipLaunchKernelGGL((k_mvm_batch<T, PH, RT, KB, 16>), dim3(nblocks), dim3(1024), 0,
-                                   s, blocks, segs, active);
-            else
-                hipLaunchKernelGGL((k_mvm_batch<T, PH, RT, KB, 4>), dim3(nblocks), dim3(256), 0, s,
-                                   blocks, segs, active);
+    auto go = [&](auto phc) {
+        constexpr int PH = decltype(phc)::value;
+        auto run = [&](auto kbc) {
+            hipLaunchKernelGGL((k_block_batch<T, PH, decltype(kbc)::value>), dim3(nblocks),
+                               dim3(256), 0, s, blocks, segs, active);
         };
-        if (kb == 8)
-            byKb(std::integral_constant<int, 8>());
+        if (kb <= 8)
+            run(std::integral_constant<int, 8>());
+        else if (kb <= 16)
+            run(std::integral_constant<int, 16>());
+        else if (kb <= 32)
+            run(std::integral_constant<int, 32>());
         else
-            byKb(std::integral_constant<int, 16>());
-    };
-    auto byRows = [&](auto phc) {
-        if (rows == 64)
-            go(phc, std::integral_constant<int, 64>());
-        else if (rows == 32)
-            go(phc, std::integral_constant<int, 32>());
-        else
-            go(phc, std::integral_constant<int, 16>());
+            run(std::integral_constant<int, 64>());
     };
     if (ph == PH_F)
-        byRows(std::integral_constant<int, PH_F>());
+        go(std::integral_constant<int, PH_F>());
     else
-        byRows(std::integral_constant<int, PH_B>());
+        go(std::integral_constant<int, PH_B>());
 }
 
 template <typename T>
@@ -2941,10 +2964,10 @@ void LaunchReduceBatch(int ph, const BatchBlock* blocks, int nblocks, const Batc
 {
     if (nblocks <= 0) return;
     if (ph == PH_F)
-        hipLaunchKernelGGL((k_mv_reduce_batch<T, PH_F>), dim3(nblocks), dim3(kThreads), 0, s,
+        hipLaunchKernelGGL((k_block_reduce_batch<T, PH_F>), dim3(nblocks), dim3(kThreads), 0, s,
                            blocks, segs, active);
     else
-        hipLaunchKernelGGL((k_mv_reduce_batch<T, PH_B>), dim3(nblocks), dim3(kThreads), 0, s,
+        hipLaunchKernelGGL((k_block_reduce_batch<T, PH_B>), dim3(nblocks), dim3(kThreads), 0, s,
                            blocks, segs, active);
 }
 
@@ -3042,19 +3065,24 @@ void LaunchAdjointGrad(const StencilArgs& st, const c128* u, const c128* lam, in
     template void LaunchLdlTrsm<T>(const ClassDev&, int, int, int, hipStream_t);                  \
     template void LaunchGemm<T>(const ClassDev&, int, int, hipStream_t);                          \
     template void LaunchInvDiag<T>(const ClassDev&, int, hipStream_t);                            \
-    template void LaunchPanelSolve<T>(const ClassDev&, const ClassPlan&, int, void*, void*, void*,   \
-                                      void*, int, hipStream_t, MvProfile*, int, int, int32_t*);   \
+    template void LaunchPanelSolve<T>(const ClassDev&, const ClassPlan&, int, void*, void*, int,   \
+                                      hipStream_t, MvProfile*, int, int);                         \
+    template void LaunchPanelSolveFused<T>(const ClassDev&, const ClassPlan&, int, void*, void*,  \
+                                           void*, void*, int, hipStream_t, MvProfile*, int32_t*); \
+    template void LaunchPack<T>(const ClassDev&, hipStream_t);                                    \
+    template void LaunchCompose<T>(const ClassDev&, int, int, hipStream_t);                       \
     template void LaunchTransposeScale<T>(const ClassDev&, hipStream_t);                          \
     template void LaunchFoldBack<T>(const ClassDev&, hipStream_t);                                \
-    template void LaunchCopyIn<T>(const ClassDev&, const c128*, void*, int, int, int, int, int,   \
-                                  int, hipStream_t, int32_t*);                                    \
-    template void LaunchCopyOut<T>(const ClassDev&, c128*, const void*, int, int, int, int, int,  \
+    template void LaunchCopyIn<T>(const PanelMap&, const c128*, void*, int, int, int, int, int,   \
+                                  int, hipStream_t, int32_t*, int);                               \
+    template void LaunchCopyOut<T>(const PanelMap&, c128*, const void*, int, int, int, int, int,  \
                                    int, int, hipStream_t, const StencilArgs*, const double*,      \
                                    int);                                                          \
-    template void LaunchZeroSetPlane<T>(const ClassDev&, const StencilArgs&, const double*,       \
-                                        const c128*, void*, int, int, int, hipStream_t, int32_t*); \
-    template void LaunchSolveBatch<T>(int, int, int, int, const BatchBlock*, int,                 \
-                                      const BatchSolveSeg*, const int32_t*, hipStream_t);         \
+    template void LaunchZeroSetPlane<T>(const PanelMap&, const StencilArgs&, const double*,       \
+                                        const c128*, void*, int, int, int, hipStream_t, int32_t*, \
+                                        int);                                                     \
+    template void LaunchSolveBatch<T>(int, int, const BatchBlock*, int, const BatchSolveSeg*,     \
+                                      const int32_t*, hipStream_t);                               \
     template void LaunchReduceBatch<T>(int, const BatchBlock*, int, const BatchSolveSeg*,         \
                                        const int32_t*, hipStream_t);                              \
     template void LaunchCopyBatch<T>(int, const BatchBlock*, int, const BatchCopySeg*,            \

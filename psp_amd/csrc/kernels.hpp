@@ -86,7 +86,6 @@ struct ClassDev {
     void* T = nullptr;              // npanels * tstore
     void* LT = nullptr;             // npanels * fstore: per front L^T (s x (s+u), ld s)
     int cus = 0;                    // compute units of the device (persistent grids)
-    int mvpGrid = 0;                // persistent solve launches: workgroup cap (0: none)
     // fused subtree solves, per phase (F, B): queue tiles, queue starts
     // (nqueues + 1), split row blocks, per-node dependencies {dep0, dep1,
     // row blocks of dep0, of dep1} (-1: none)
@@ -98,6 +97,30 @@ struct ClassDev {
     int nqtiles[2] = {0, 0}, nqreds[2] = {0, 0};
     int queueRows = 32;             // output rows per fused tile
     int nsync = 0;                  // ints of fused-launch state per class (both phases)
+    // merged solves
+    BlockTile* btiles = nullptr;
+    BlockRed* breds = nullptr;
+    int32_t* bredcBuf = nullptr;    // one arrival counter per reduce item (zero between launches)
+    int32_t* bredc = nullptr;       // bredcBuf when slices are summed in the launch
+    int32_t *blist = nullptr, *bsrc = nullptr, *udst = nullptr;
+    int32_t *sxy = nullptr, *sv = nullptr;
+    int32_t xrows = 0;
+    int64_t fentries = 0;           // entries of one panel's F
+    void* F = nullptr;              // npanels * fentries
+    void* dinv = nullptr;           // npanels * xrows
+    int32_t *browBase = nullptr, *flist = nullptr, *fsrc = nullptr;
+    FoldNode* foldNodes = nullptr;
+    TransItem* packs = nullptr;
+    int npacks = 0;
+    ComposeDesc* compose = nullptr;
+    ComposeKey* fkeys = nullptr;
+    GemmTile* composeTiles = nullptr;
+};
+
+// Rows of a panel vector and the unknowns they hold (v < 0: padding).
+struct PanelMap {
+    int n;
+    const int32_t *xy, *v;
 };
 
 // Ints of fused-launch state of one phase: per-node done counters, queue
@@ -105,23 +128,21 @@ struct ClassDev {
 inline int QueueSyncInts(int nnodes, int nqueues, int nreds) { return nnodes + nqueues + 1 + nreds; }
 
 // ---- batched sweeps of many problems (one launch per step of all sweeps) ----
-// One workgroup of a batched launch: its tile or reduce item (products,
+// One workgroup of a batched launch: its BlockTile or BlockRed (products,
 // reduces), its segment and problem, and its workgroup index inside the
 // segment (copies).
 struct BatchBlock {
-    const SolveTile* item;
+    const void* item;
     int32_t seg, problem, blk, pad_;
 };
 // One problem's panel solve in a batched product or reduce launch (front
 // precision erased: the kernels cast to their cx<T>).
 struct BatchSolveSeg {
-    const int32_t* structs;
-    void* G;                 // slot copies of the panel's class, slot 1 at G + half elements
-    int64_t half;
-    const int32_t* relinds;
-    const void *L, *LT;      // this panel's factors
-    void *Xp, *W, *P;
-    int32_t k, pad_;
+    const void *F, *dinv;    // this panel's factor
+    void *V, *P;
+    const int32_t *bsrc, *blist, *udst;
+    int64_t w, g0, g1;       // VecRows
+    int32_t xrows, zero, k;
 };
 enum BatchCopyOp : int { BATCH_COPY_IN = 0, BATCH_COPY_OUT = 1, BATCH_ZERO_SET_PLANE = 2 };
 constexpr int kBatchCopyThreads = 256;  // elements per workgroup of a batched copy
@@ -170,16 +191,27 @@ struct MvProfile {
     double seconds = 0, bytes = 0, flops = 0;
 };
 
-// Solve of one panel (batch entry b of class c) on the padded ND vector Xp
-// (n x k, k interleaved) with node work vectors W (wstore x k).
-// sync: the class's fused-launch state (cleared by the copy-in or
-// zero-set launch before the panel solve); null runs every level as its own
-// launch.
+// Solve of one panel (batch entry b of class c) on the class's solve vector V
+// (VecRows, k right-hand sides interleaved); P: partial sums (bslots x 64
+// rows).  onlyGroup >= 0: that group's launch of phase onlyPhase alone.
 template <typename T>
-void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* Xp, void* W,
-                      void* P, void* G,
-                      int k, hipStream_t s, MvProfile* prof = nullptr, int onlyLevel = -1,
-                      int onlyPhase = -1, int32_t* sync = nullptr);
+void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, void* P, int k,
+                      hipStream_t s, MvProfile* prof = nullptr, int onlyGroup = -1,
+                      int onlyPhase = -1);
+// The same through the fused subtree launches (PSP_HIP_OPT_SOLVE_FUSED) on
+// the padded ND vector Xp (n x k) with node work vectors W (wstore x k);
+// sync: the class's fused-launch state, cleared by the copy-in or zero-set
+// launch before.  FusedApplies: whether the class has them for k.
+template <typename T>
+void LaunchPanelSolveFused(const ClassDev& c, const ClassPlan& plan, int b, void* Xp, void* W,
+                           void* P, void* G, int k, hipStream_t s, MvProfile* prof, int32_t* sync);
+bool FusedApplies(const ClassDev& c, const ClassPlan& plan, int k, int64_t eb);
+// Fold of the factored fronts into F: the copied pieces, then the composed
+// columns of one depth below the groups' tops.
+template <typename T>
+void LaunchPack(const ClassDev& c, hipStream_t s);
+template <typename T>
+void LaunchCompose(const ClassDev& c, int tileStart, int tileCount, hipStream_t s);
 template <typename T>
 void LaunchTransposeScale(const ClassDev& c, hipStream_t s);
 template <typename T>
@@ -189,23 +221,23 @@ void LaunchFoldBack(const ClassDev& c, hipStream_t s);
 // sync (nsync ints, may be null): the class's fused-launch state, cleared
 // by the same launch (the panel solve that follows starts from zero).
 template <typename T>
-void LaunchCopyIn(const ClassDev& c, const c128* B, void* Xp, int k, int nx, int ny, int nz,
-                  int vOffset, int padding, hipStream_t s, int32_t* sync = nullptr);
+void LaunchCopyIn(const PanelMap& m, const c128* B, void* Xp, int k, int nx, int ny, int nz,
+                  int vOffset, int padding, hipStream_t s, int32_t* sync = nullptr, int nsync = 0);
 template <typename T>
-void LaunchCopyOut(const ClassDev& c, c128* B, const void* Xp, int k, int nx, int ny, int nz,
+void LaunchCopyOut(const PanelMap& m, c128* B, const void* Xp, int k, int nx, int ny, int nz,
                    int vOffset, int padding, int mode, hipStream_t s,
                    const StencilArgs* st = nullptr, const double* vel = nullptr, int v1 = -1);
 // Backward sweep, one pass: Xp = 0 except the superdiagonal coupling on the
 // panel's last local plane (MultiplySuperdiagonal, solve.hpp:725-733).
 template <typename T>
-void LaunchZeroSetPlane(const ClassDev& c, const StencilArgs& st, const double* vel,
+void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* vel,
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,
-                        int32_t* sync = nullptr);
-// Batched launches over nblocks BatchBlocks: products of phase ph with
-// rows-per-tile rows, waves waves per workgroup and kb (8 or 16) right-hand
-// sides per pass (k_mvm's tile work), reduce items, or panel copies (op).
+                        int32_t* sync = nullptr, int nsync = 0);
+// Batched launches over nblocks BatchBlocks: products of phase ph with up to
+// kb (8, 16, 32 or 64) right-hand sides per pass, reduce items, or panel
+// copies (op).
 template <typename T>
-void LaunchSolveBatch(int ph, int rows, int waves, int kb, const BatchBlock* blocks, int nblocks,
+void LaunchSolveBatch(int ph, int kb, const BatchBlock* blocks, int nblocks,
                       const BatchSolveSeg* segs, const int32_t* active, hipStream_t s);
 template <typename T>
 void LaunchReduceBatch(int ph, const BatchBlock* blocks, int nblocks, const BatchSolveSeg* segs,

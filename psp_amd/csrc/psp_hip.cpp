@@ -56,9 +56,12 @@ struct psp_hip_ctx {
     std::vector<void*> wsAllocs;
     int64_t wsSlots = 0;  // partial-sum slots the workspace holds
     std::vector<void*> facAllocs;  // Schur-complement and inversion scratch, only while factoring
-    std::vector<void*> facStore;   // L and LT of every panel, from Initialize to Finalize
+    std::vector<void*> facStore;   // factors of every panel, from Initialize to Finalize
+    bool facFused = false;         // the factors include those of the fused launches
+    void* vec[3] = {nullptr, nullptr, nullptr};  // per class: the solve vector (VecRows)
+    void* P = nullptr;  // partial sums of split output blocks (64 rows x k per slot)
+    // fused subtree launches only
     void *Xp = nullptr, *W = nullptr;
-    void* P = nullptr;  // partial sums of split solve row blocks (64 rows x k per slot)
     void* G[3] = {nullptr, nullptr, nullptr};  // per class: the children's update rows, two slot copies
     int32_t* S[3] = {nullptr, nullptr, nullptr};  // per class: fused-launch state (counters)
     c128 *V = nullptr, *x = nullptr, *x0 = nullptr, *w = nullptr, *b = nullptr;
@@ -66,7 +69,6 @@ struct psp_hip_ctx {
     c128 *partC = nullptr, *Hcol = nullptr, *ydev = nullptr;
     // captured sweeps, keyed on (block pointer, k)
     bool useGraph = true;
-    int mvpGrid = 0;  // persistent solve launches: workgroup cap (0: none)
     bool xcdReduce = true;  // split row blocks summed in the product launch (option)
     bool xcdOk = false;     // the device deals workgroups to its XCDs round-robin
     bool factorOverlap = true;  // panel classes 1 and 2 factored on side streams (option)
@@ -223,10 +225,10 @@ std::vector<SolveTile> SolveTiles(const ClassPlan& P, const std::vector<MvTile>&
     return out;
 }
 
-// Zeroed arrival counters, one per reduce item of the class.
-std::vector<int32_t> ReduceCounters(const ClassPlan& P)
+// Zeroed arrival counters, one per reduce item.
+std::vector<int32_t> ReduceCounters(size_t items)
 {
-    return std::vector<int32_t>(std::max<size_t>(1, P.mvred.size()), 0);
+    return std::vector<int32_t>(std::max<size_t>(1, items), 0);
 }
 
 // Whether the product launches of a class sum split row blocks themselves
@@ -247,9 +249,10 @@ bool XcdDealing(psp_hip_ctx* c)
 void SetSliceReduce(psp_hip_ctx* c, ClassDev& D)
 {
     D.redc = c->xcdReduce && c->xcdOk ? D.redcBuf : nullptr;
+    D.bredc = c->xcdReduce && c->xcdOk ? D.bredcBuf : nullptr;
 }
 
-int UploadQueues(psp_hip_ctx* c, int cl);
+int UploadTiles(psp_hip_ctx* c, int cl);
 
 // Scratch of psp_hip_precondition_noalloc, the sweep entry point that
 // allocates nothing: the sweep buffers (SweepBufferSizes) live in this
@@ -338,13 +341,16 @@ int EnsureDevice(psp_hip_ctx* c)
         const ClassPlan& P = c->plan.cls[cl];
         ClassDev& D = c->dev[cl];
         D.cus = cus;
-        D.mvpGrid = c->mvpGrid;
         D.n = P.n;
         D.vsize = P.vsize;
         D.nnodes = (int)P.nodes.size();
         D.npanels = (int)c->classPanels[cl].size();
         D.fstore = P.fstore;
-        D.ustore = P.ustore;
+        // the update scratch also holds the fold's E (read one entry past it)
+        D.ustore = std::max(P.ustore, P.estore + 1);
+        D.xrows = P.xrows;
+        D.fentries = (int64_t)(P.nblocks + 1) * kBlk * kBlk;  // and a block of zeros
+        D.npacks = (int)P.packs.size();
         D.tstore = P.tstore;
         D.wstore = P.wstore;
         D.ninv = (int)P.inv.size();
@@ -380,9 +386,12 @@ int EnsureDevice(psp_hip_ctx* c)
             (st = Upload(c, &D.relinds, WithSentinel(P.relinds))) || (st = Upload(c, &D.extadd, P.extadd)) ||
             (st = Upload(c, &D.ldl, P.ldl)) || (st = Upload(c, &D.gemms, P.gemms)) ||
             (st = Upload(c, &D.tiles, P.tiles)) || (st = Upload(c, &D.inv, P.inv)) ||
-            (st = Upload(c, &D.mv, SolveTiles(P, P.mv))) ||
-            (st = Upload(c, &D.mvred, SolveTiles(P, P.mvred))) ||
-            (st = Upload(c, &D.redcBuf, ReduceCounters(P))) ||
+            (st = Upload(c, &D.sxy, P.sxy)) || (st = Upload(c, &D.sv, P.sv)) ||
+            (st = Upload(c, &D.browBase, P.browBase)) || (st = Upload(c, &D.udst, P.udst)) ||
+            (st = Upload(c, &D.flist, P.flist)) || (st = Upload(c, &D.fsrc, P.fsrc)) ||
+            (st = Upload(c, &D.foldNodes, P.foldNodes)) || (st = Upload(c, &D.packs, P.packs)) ||
+            (st = Upload(c, &D.compose, P.compose)) || (st = Upload(c, &D.fkeys, P.fkeys)) ||
+            (st = Upload(c, &D.composeTiles, P.composeTiles)) ||
             (st = Upload(c, &D.trans, P.trans)) || (st = Upload(c, &D.ginv, P.ginv)) ||
             (st = Upload(c, &D.foldBack, P.foldBack)) ||
             (st = Upload(c, &D.panelVOff, vOff)))
@@ -390,39 +399,53 @@ int EnsureDevice(psp_hip_ctx* c)
         std::vector<NodeDev> nd(D.nnodes);
         for (int t = 0; t < D.nnodes; ++t) nd[t] = MakeNodeDev(P, t);
         if ((st = Upload(c, &D.nodes, nd))) return st;
-        SetSliceReduce(c, D);
         D.ntrans = (int)P.trans.size();
         D.nfold = (int)P.foldBack.size();
         std::vector<c128> s3c = ToC128(s3a);
         if ((st = Upload(c, &D.s3art, s3c))) return st;
-        if ((st = UploadQueues(c, cl))) return st;
+        if ((st = UploadTiles(c, cl))) return st;
     }
     c->devReady = true;
     return PSP_HIP_OK;
 }
 
-// Factor storage (L and LT of every panel), allocated by the first
-// Initialize after construction or Finalize and kept until Finalize.
+// Factor storage, allocated by the first Initialize after construction or
+// Finalize and kept until Finalize: L (the factorization), F and D^-1 (the
+// merged solves) and, for the fused subtree launches, LT.
 int EnsureFactorStorage(psp_hip_ctx* c)
 {
     const size_t eb = FrontBytes(c);
     for (int cl = 0; cl < 3; ++cl) {
         if (!c->plan.present[cl]) continue;
         ClassDev& D = c->dev[cl];
-        if (D.L) continue;
         const ClassPlan& P = c->plan.cls[cl];
-        // factor arrays end in kSolvePad columns of the tallest front (zeros)
+        // L and LT end in kSolvePad columns of the tallest front (zeros)
         int64_t maxFs = 1;
         for (const Node& nd : P.nodes) maxFs = std::max<int64_t>(maxFs, nd.size + nd.usize);
-        const size_t fb = eb * ((size_t)D.npanels * D.fstore + (size_t)kSolvePad * maxFs);
-        int st;
-        if ((st = Alloc(c, &D.L, fb, c->facStore))) return st;
-        if ((st = Alloc(c, &D.LT, fb, c->facStore))) return st;
-        // only the padding needs zeroing here: every factorization zeroes L
-        // before assembly, and the fold writes every entry of LT
         const size_t body = eb * (size_t)D.npanels * D.fstore;
-        HIPCHK(c, hipMemsetAsync((char*)D.L + body, 0, fb - body, c->stream));
-        HIPCHK(c, hipMemsetAsync((char*)D.LT + body, 0, fb - body, c->stream));
+        const size_t fb = body + eb * (size_t)kSolvePad * maxFs;
+        int st;
+        if (!D.L) {
+            // only the padding needs zeroing here: every factorization
+            // zeroes L before assembly
+            if ((st = Alloc(c, &D.L, fb, c->facStore))) return st;
+            HIPCHK(c, hipMemsetAsync((char*)D.L + body, 0, fb - body, c->stream));
+        }
+        if (!D.F) {
+            // entries of F and D^-1 that no fold writes (padding of the
+            // blocks) stay zero
+            const size_t f = eb * (size_t)D.npanels * D.fentries;
+            const size_t v = eb * (size_t)D.npanels * D.xrows;
+            if ((st = Alloc(c, &D.F, f, c->facStore))) return st;
+            HIPCHK(c, hipMemsetAsync(D.F, 0, std::max<size_t>(f, 16), c->stream));
+            if ((st = Alloc(c, &D.dinv, v, c->facStore))) return st;
+            HIPCHK(c, hipMemsetAsync(D.dinv, 0, std::max<size_t>(v, 16), c->stream));
+        }
+        if (c->plan.fused && !D.LT) {
+            // the fold writes every entry of LT
+            if ((st = Alloc(c, &D.LT, fb, c->facStore))) return st;
+            HIPCHK(c, hipMemsetAsync((char*)D.LT + body, 0, fb - body, c->stream));
+        }
     }
     return PSP_HIP_OK;
 }
@@ -434,8 +457,11 @@ void FreeFactorStorage(psp_hip_ctx* c)
     for (int cl = 0; cl < 3; ++cl) {
         c->dev[cl].L = nullptr;
         c->dev[cl].LT = nullptr;
+        c->dev[cl].F = nullptr;
+        c->dev[cl].dinv = nullptr;
     }
     c->factored = false;
+    c->facFused = false;
 }
 
 void FreeGraphs(psp_hip_ctx* c)
@@ -469,39 +495,39 @@ int64_t NeededSlots(const psp_hip_ctx* c)
 {
     int64_t maxs = 1;
     for (int cl = 0; cl < 3; ++cl)
-        if (c->plan.present[cl]) maxs = std::max<int64_t>(maxs, c->plan.cls[cl].maxSlots);
+        if (c->plan.present[cl]) {
+            maxs = std::max<int64_t>(maxs, c->plan.cls[cl].bslots);
+            if (c->plan.fused) maxs = std::max<int64_t>(maxs, c->plan.cls[cl].maxSlots);
+        }
     return maxs;
 }
 
-// Byte sizes of the sweep's buffers for k right-hand sides: the padded
-// panel vector Xp, the node work vectors W, the partial sums P of split
-// solve row blocks and, per panel class, the two slot copies G of the
-// children's update rows.  Vectors and slot copies end in kSolvePad + 2
-// rows that must read as zero (the solve kernels read past a tile's rows).
+// Byte sizes of the sweep's buffers for k right-hand sides: per panel class
+// the solve vector (VecRows; the rows nothing writes must read as zero) and
+// the partial sums P.  The fused launches add the padded panel vector Xp, the
+// node work vectors W and per class the two slot copies G of the children's
+// update rows, each ending in kSolvePad + 2 rows that must read as zero (the
+// kernels read past a tile's rows), and their launch state.
 struct SweepSizes {
-    size_t xp = 0, w = 0, p = 0, g[3] = {0, 0, 0}, s[3] = {0, 0, 0};
+    size_t v[3] = {0, 0, 0}, p = 0, xp = 0, w = 0, g[3] = {0, 0, 0}, s[3] = {0, 0, 0};
 };
 
 SweepSizes SweepBufferSizes(const psp_hip_ctx* c, int k)
 {
     const size_t eb = FrontBytes(c);
-    int64_t maxn = 0, maxw = 0, maxs = 1;
-    for (int cl = 0; cl < 3; ++cl)
-        if (c->plan.present[cl]) {
-            maxn = std::max<int64_t>(maxn, c->plan.cls[cl].n);
-            maxw = std::max<int64_t>(maxw, c->plan.cls[cl].wstore);
-            maxs = std::max<int64_t>(maxs, c->plan.cls[cl].maxSlots);
-        }
     const size_t padRows = (size_t)kSolvePad + 2;
     SweepSizes z;
-    z.xp = eb * (maxn + padRows) * k;
-    z.w = eb * (maxw + padRows) * k;
-    z.p = eb * maxs * 64 * k;
-    for (int cl = 0; cl < 3; ++cl)
-        if (c->plan.present[cl]) {
-            z.g[cl] = eb * (2 * (size_t)c->plan.cls[cl].wstore + padRows) * k;
-            z.s[cl] = sizeof(int32_t) * (size_t)std::max(c->dev[cl].nsync, 1);
-        }
+    z.p = eb * NeededSlots(c) * 64 * k;
+    for (int cl = 0; cl < 3; ++cl) {
+        if (!c->plan.present[cl]) continue;
+        const ClassPlan& C = c->plan.cls[cl];
+        z.v[cl] = eb * (size_t)VecRows(C).total * k;
+        if (!c->plan.fused) continue;
+        z.xp = std::max(z.xp, eb * ((size_t)C.n + padRows) * k);
+        z.w = std::max(z.w, eb * ((size_t)C.wstore + padRows) * k);
+        z.g[cl] = eb * (2 * (size_t)C.wstore + padRows) * k;
+        z.s[cl] = sizeof(int32_t) * (size_t)std::max(c->dev[cl].nsync, 1);
+    }
     return z;
 }
 
@@ -513,18 +539,22 @@ int EnsureWorkspace(psp_hip_ctx* c, int k, int m)
     const SweepSizes z = SweepBufferSizes(c, k);
     int st;
     void* p;
-    if ((st = Alloc(c, &c->Xp, z.xp, c->wsAllocs))) return st;
-    if ((st = Alloc(c, &c->W, z.w, c->wsAllocs))) return st;
-    HIPCHK(c, hipMemsetAsync(c->Xp, 0, z.xp, c->stream));
-    HIPCHK(c, hipMemsetAsync(c->W, 0, z.w, c->stream));
     if ((st = Alloc(c, &c->P, z.p, c->wsAllocs))) return st;
+    // Zeroed once: a class writes the same rows of its solve vector and slot
+    // copies in every solve, and the rows it never writes must read as zero.
+    auto zeroed = [&](void** q, size_t bytes) -> int {
+        int e = Alloc(c, q, bytes, c->wsAllocs);
+        if (e) return e;
+        HIPCHK(c, hipMemsetAsync(*q, 0, bytes, c->stream));
+        return PSP_HIP_OK;
+    };
+    if (c->plan.fused && ((st = zeroed(&c->Xp, z.xp)) || (st = zeroed(&c->W, z.w)))) return st;
     for (int cl = 0; cl < 3; ++cl) {
-        c->G[cl] = nullptr;
+        c->vec[cl] = c->G[cl] = nullptr;
         if (!c->plan.present[cl]) continue;
-        // Zero once: each class writes the same rows of its slot copies in
-        // every solve, and the rows it never writes must read as zero.
-        if ((st = Alloc(c, &c->G[cl], z.g[cl], c->wsAllocs))) return st;
-        HIPCHK(c, hipMemsetAsync(c->G[cl], 0, z.g[cl], c->stream));
+        if ((st = zeroed(&c->vec[cl], z.v[cl]))) return st;
+        if (!c->plan.fused) continue;
+        if ((st = zeroed(&c->G[cl], z.g[cl]))) return st;
         void* sp = nullptr;
         if ((st = Alloc(c, &sp, z.s[cl], c->wsAllocs))) return st;
         c->S[cl] = (int32_t*)sp;
@@ -607,6 +637,26 @@ void BuildClassQueues(psp_hip_ctx* c, ClassPlan& P)
     BuildQueues(P, pl.fused ? pl.fusedQueues : 0, pl.fusedRows, pl.fusedCut, pl.fusedWgPerQueue);
 }
 
+// Device copies of a class's solve tiles: the merged solves' and, with the
+// fused launches on, the levels' and the queues'.
+int UploadTiles(psp_hip_ctx* c, int cl)
+{
+    const ClassPlan& P = c->plan.cls[cl];
+    ClassDev& D = c->dev[cl];
+    const bool fused = c->plan.fused;
+    int st;
+    if ((st = ReUpload(c, &D.btiles, P.btiles)) || (st = ReUpload(c, &D.breds, P.breds)) ||
+        (st = ReUpload(c, &D.blist, P.blist)) || (st = ReUpload(c, &D.bsrc, P.bsrc)) ||
+        (st = ReUpload(c, &D.bredcBuf, ReduceCounters(P.breds.size()))) ||
+        (st = ReUpload(c, &D.mv, fused ? SolveTiles(P, P.mv) : std::vector<SolveTile>{})) ||
+        (st = ReUpload(c, &D.mvred, fused ? SolveTiles(P, P.mvred) : std::vector<SolveTile>{})) ||
+        (st = ReUpload(c, &D.redcBuf, ReduceCounters(fused ? P.mvred.size() : 0))) ||
+        (st = UploadQueues(c, cl)))
+        return st;
+    SetSliceReduce(c, D);
+    return PSP_HIP_OK;
+}
+
 // Rebuilds the front-solve tiles of every class from its shapes and, once
 // the device is set up, replaces the device copies; the workspace (partial
 // buffer sized by the slots) and the captured sweep graphs are dropped.
@@ -616,16 +666,11 @@ int RebuildSolveTiles(psp_hip_ctx* c)
     for (int cl = 0; cl < 3; ++cl) {
         if (!c->plan.present[cl]) continue;
         ClassPlan& P = c->plan.cls[cl];
+        BuildBlockTiles(P);
         BuildSolveTiles(P);
         BuildClassQueues(c, P);
-        if (!c->devReady) continue;
-        ClassDev& D = c->dev[cl];
         int st;
-        if ((st = ReUpload(c, &D.mv, SolveTiles(P, P.mv))) ||
-            (st = ReUpload(c, &D.mvred, SolveTiles(P, P.mvred))) ||
-            (st = ReUpload(c, &D.redcBuf, ReduceCounters(P))) || (st = UploadQueues(c, cl)))
-            return st;
-        SetSliceReduce(c, D);
+        if (c->devReady && (st = UploadTiles(c, cl))) return st;
     }
     FreeWorkspace(c);
     return PSP_HIP_OK;
@@ -708,11 +753,19 @@ int FactorClasses(psp_hip_ctx* c, double* tFill, double* tLdl, double* tInv, dou
         HIPCHK(c, mark(2));
         LaunchInvDiag<T>(D, nb, s);
         for (const GemmLaunch& gl : P.invGemm) LaunchGemm<T>(D, gl.tileStart, gl.tileCount, s);
-        // solve layout: LT[:, :s] = Linv^T D^-1, LT[:, s:] = (-L_BL Linv)^T, then
-        // L_BL = -L_BL Linv and a unit diagonal in L
-        LaunchTransposeScale<T>(D, s);
-        LaunchGemm<T>(D, P.fold.tileStart, P.fold.tileCount, s);
-        LaunchFoldBack<T>(D, s);
+        // merged fronts: E = -L_BL Linv per node, copied pieces, then the
+        // columns of the nodes below the groups' tops, depth by depth
+        LaunchGemm<T>(D, P.foldE.tileStart, P.foldE.tileCount, s);
+        LaunchPack<T>(D, s);
+        for (const GemmLaunch& gl : P.composeSteps)
+            LaunchCompose<T>(D, gl.tileStart, gl.tileCount, s);
+        if (c->plan.fused) {
+            // layout of the fused launches: LT[:, :s] = Linv^T D^-1, LT[:, s:] =
+            // (-L_BL Linv)^T, then L_BL = -L_BL Linv and a unit diagonal in L
+            LaunchTransposeScale<T>(D, s);
+            LaunchGemm<T>(D, P.fold.tileStart, P.fold.tileCount, s);
+            LaunchFoldBack<T>(D, s);
+        }
         HIPCHK(c, mark(3));
         HIPCHK(c, hipGetLastError());
         if (cl > 0) HIPCHK(c, hipStreamWaitEvent(c->stream, evs.v[ce[cl][3]], 0));  // join
@@ -740,25 +793,98 @@ int FactorClasses(psp_hip_ctx* c, double* tFill, double* tLdl, double* tInv, dou
     return PSP_HIP_OK;
 }
 
+// Factors every panel of the velocity in c->vel; t: seconds of the phases
+// (fill, LDL, inversion and fold, Schur GEMMs).
+int Factor(psp_hip_ctx* c, double t[4])
+{
+    int st = EnsureFactorStorage(c);
+    if (st) return st;
+    // a new factorization invalidates the captured sweeps' results only, not
+    // their launches: the graphs keep reading the same factor arrays
+    c->factored = false;
+    // The Schur-complement (U) and inversion (T) scratch lives only while
+    // factoring, so that many factored problems fit in HBM at once.
+    const size_t eb = FrontBytes(c);
+    for (int cl = 0; cl < 3; ++cl) {
+        if (!c->plan.present[cl]) continue;
+        ClassDev& D = c->dev[cl];
+        if ((st = Alloc(c, &D.U, eb * (size_t)D.npanels * D.ustore, c->facAllocs)) ||
+            (st = Alloc(c, &D.T, eb * (size_t)D.npanels * D.tstore, c->facAllocs))) {
+            FreeFactorScratch(c);
+            return st;
+        }
+    }
+    st = c->desc.precision == PSP_HIP_FRONTS_FP32
+             ? FactorClasses<float>(c, &t[0], &t[1], &t[2], &t[3])
+             : FactorClasses<double>(c, &t[0], &t[1], &t[2], &t[3]);
+    if (st) {
+        (void)hipStreamSynchronize(c->stream);
+        for (hipStream_t x : c->side)
+            if (x) (void)hipStreamSynchronize(x);
+        FreeFactorScratch(c);
+        return st;
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    FreeFactorScratch(c);
+    c->factored = true;
+    c->facFused = c->plan.fused;
+    return PSP_HIP_OK;
+}
+
+// The fused launches were switched on after Initialize: factor once more, with
+// their layout.
+int EnsureFusedFactors(psp_hip_ctx* c)
+{
+    if (!c->plan.fused || c->facFused) return PSP_HIP_OK;
+    double t[4];
+    return Factor(c, t);
+}
+
 // ---------------------------------------------------------------------------
 // Sweep: Precondition (solve.hpp:681-734) on a natural-order device block.
 // ---------------------------------------------------------------------------
 // couple >= 0: the copy-out also applies the subdiagonal coupling into the
 // next panel's first plane `couple` (SolvePanel + MultiplySubdiagonal).
+// The panel vector of a class's panel solves and its map to grid points, and
+// the solve between a copy in and a copy out.
+template <typename T>
+struct PanelSolver {
+    psp_hip_ctx* c;
+    int cl, k;
+    const ClassDev& D;
+    bool fused;
+    PanelMap map;
+    void* x;
+    int32_t* sync;
+    PanelSolver(psp_hip_ctx* c_, int cl_, int k_)
+        : c(c_), cl(cl_), k(k_), D(c_->dev[cl_]),
+          fused(c_->plan.fused && FusedApplies(D, c_->plan.cls[cl_], k_, sizeof(cx<T>))),
+          map(fused ? PanelMap{D.n, D.qxy, D.qv} : PanelMap{D.xrows, D.sxy, D.sv}),
+          x(fused ? c_->Xp : c_->vec[cl_]), sync(fused ? c_->S[cl_] : nullptr)
+    {
+    }
+    void Solve(int b, MvProfile* prof) const
+    {
+        const ClassPlan& P = c->plan.cls[cl];
+        if (fused)
+            LaunchPanelSolveFused<T>(D, P, b, c->Xp, c->W, c->P, c->G[cl], k, c->stream, prof, sync);
+        else
+            LaunchPanelSolve<T>(D, P, b, c->vec[cl], c->P, k, c->stream, prof);
+    }
+};
+
 template <typename T>
 void PanelForward(psp_hip_ctx* c, c128* B, int k, int p, MvProfile* prof = nullptr,
                   int couple = -1)
 {
     const Geometry& g = c->plan.geo;
-    const int cl = g.cls(p);
-    const ClassDev& D = c->dev[cl];
+    const PanelSolver<T> ps(c, g.cls(p), k);
     hipStream_t s = c->stream;
     const StencilArgs st = Stencil(c);
-    int32_t* sync = D.nqueues > 0 ? c->S[cl] : nullptr;
-    LaunchCopyIn<T>(D, B, c->Xp, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), s, sync);
-    LaunchPanelSolve<T>(D, c->plan.cls[cl], c->panelBatch[p], c->Xp, c->W, c->P, c->G[cl], k, s,
-                        prof, -1, -1, sync);
-    LaunchCopyOut<T>(D, B, c->Xp, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), 0, s,
+    LaunchCopyIn<T>(ps.map, B, ps.x, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), s, ps.sync,
+                    ps.D.nsync);
+    ps.Solve(c->panelBatch[p], prof);
+    LaunchCopyOut<T>(ps.map, B, ps.x, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), 0, s,
                      couple >= 0 ? &st : nullptr, c->vel, couple);
 }
 
@@ -769,17 +895,16 @@ void PanelBackward(psp_hip_ctx* c, c128* B, int k, int p, MvProfile* prof = null
     // (solve.hpp:725-733): B_i still holds Z, so the solve of the coupling
     // term is added onto it.
     const Geometry& g = c->plan.geo;
-    const int cl = g.cls(p);
-    const ClassDev& D = c->dev[cl];
+    const PanelSolver<T> ps(c, g.cls(p), k);
     hipStream_t s = c->stream;
-    // Xp = 0 except the superdiagonal coupling on the panel's last plane
+    // the panel vector is 0 except the superdiagonal coupling on the panel's
+    // last plane
     const int v2 = g.panelV(p) + g.depth(p) - 1;
     const int vlLast = g.padding(p) + g.depth(p) - 1;
-    int32_t* sync = D.nqueues > 0 ? c->S[cl] : nullptr;
-    LaunchZeroSetPlane<T>(D, Stencil(c), c->vel, B, c->Xp, k, v2, vlLast, s, sync);
-    LaunchPanelSolve<T>(D, c->plan.cls[cl], c->panelBatch[p], c->Xp, c->W, c->P, c->G[cl], k, s,
-                        prof, -1, -1, sync);
-    LaunchCopyOut<T>(D, B, c->Xp, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), 1, s);
+    LaunchZeroSetPlane<T>(ps.map, Stencil(c), c->vel, B, ps.x, k, v2, vlLast, s, ps.sync,
+                          ps.D.nsync);
+    ps.Solve(c->panelBatch[p], prof);
+    LaunchCopyOut<T>(ps.map, B, ps.x, k, g.nx, g.ny, g.nz, g.vOffset(p), g.padding(p), 1, s);
 }
 
 template <typename T>
@@ -1048,7 +1173,7 @@ int CheckSolveArgs(psp_hip_ctx* c, const void* B, int k, int m)
     if (!B) return Fail(c, PSP_HIP_ERR_INVALID, "null right-hand side");
     if (k < 1 || k > 256) return Fail(c, PSP_HIP_ERR_INVALID, "number of RHS must be in [1, 256]");
     if (m < 1) return Fail(c, PSP_HIP_ERR_INVALID, "GMRES restart length must be >= 1");
-    return PSP_HIP_OK;
+    return EnsureFusedFactors(c);
 }
 
 int RunSolve(psp_hip_ctx* c, void* B, int k, int m, double relTol, int maxIts, int flags,
@@ -1098,14 +1223,14 @@ int RunSolve(psp_hip_ctx* c, void* B, int k, int m, double relTol, int maxIts, i
 // where a panel solve is the forward phase over the tree levels from the
 // leaves (level d at step D - d, D the deepest level over all problems, so
 // the roots line up) and the backward phase from the roots.
-// A step's products go in one launch per tile shape (rows per tile, waves)
-// present at that step.  Each problem's kernels see the tiles, factors and
+// A step's products go in one launch per number of right-hand sides a pass
+// covers (8, 16, 32 or 64).  Each problem's kernels see the tiles, factors and
 // buffers of its own single-problem sweep, in the same order.
 struct BatchSweep {
     enum Kind { PRODUCTS = 0, REDUCE = 1, COPY = 2 };
     struct Launch {
         int group = 0;  // problem group: its launches form one branch of the graph
-        int kind = PRODUCTS, ph = 0, rows = 64, waves = 4, kb = 16, op = 0;
+        int kind = PRODUCTS, ph = 0, kb = 16, op = 0;
         int64_t blk0 = 0;
         int nblocks = 0;
     };
@@ -1138,19 +1263,21 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
     // stage key: sweep direction (0 forward, 1 backward), panel step,
     // sub-step (0: first copy; 1 .. 1 + D: forward phase, level D + 1 - sub;
     // 2 + D .. 2 + 2D: backward phase, level sub - 2 - D; 3 + 2D: copy-out),
-    // part (0 products, 1 reduce), kernel shape (rows * 10000 + waves * 100 +
-    // right-hand sides per pass: 8 for k <= 8, else 16; 0 for copies)
+    // part (0 products, 1 reduce), right-hand sides per pass (8, 16, 32, 64;
+    // 0 for copies and reduces); a level is a depth group of the merged solves
     using Key = std::array<int, 5>;
     struct Entry {
         int problem, seg;
-        const SolveTile* items;
-        int count;  // tiles / reduce items; copies: workgroups
+        const char* items;
+        int stride;  // bytes per item
+        int count;   // tiles / reduce items; copies: workgroups
     };
     std::map<Key, std::vector<Entry>> stages;
     int dmax = 0;
     for (int i : members)
         for (int cl = 0; cl < 3; ++cl)
-            if (cs[i]->plan.present[cl]) dmax = std::max(dmax, cs[i]->plan.cls[cl].maxDepth);
+            if (cs[i]->plan.present[cl])
+                dmax = std::max(dmax, (int)cs[i]->plan.cls[cl].blevels.size() - 1);
     const int subOut = 2 * dmax + 3;
     for (int i : members) {
         psp_hip_ctx* c = cs[i];
@@ -1164,11 +1291,11 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             BatchCopySeg s{};
             s.st = st;
             s.vel = c->vel;
-            s.qxy = D.qxy;
-            s.qv = D.qv;
+            s.qxy = D.sxy;
+            s.qv = D.sv;
             s.B = c->w;
-            s.Xp = c->Xp;
-            s.n = D.n;
+            s.Xp = c->vec[g.cls(p)];
+            s.n = D.xrows;
             s.k = k;
             s.vOffset = g.vOffset(p);
             s.padding = g.padding(p);
@@ -1177,24 +1304,29 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             s.v2 = g.panelV(p) + g.depth(p) - 1;
             s.vlLast = g.padding(p) + g.depth(p) - 1;
             bs.copySegs.push_back(s);
-            const int nb = (int)(((int64_t)D.n * k + kBatchCopyThreads - 1) / kBatchCopyThreads);
-            return Entry{i, (int)bs.copySegs.size() - 1, nullptr, nb};
+            const int nb =
+                (int)(((int64_t)D.xrows * k + kBatchCopyThreads - 1) / kBatchCopyThreads);
+            return Entry{i, (int)bs.copySegs.size() - 1, nullptr, 0, nb};
         };
         auto solveSeg = [&](int p) {
             const int cl = g.cls(p);
             const ClassDev& D = c->dev[cl];
             const size_t eb = f32 ? sizeof(c64) : sizeof(c128);
             const int64_t b = c->panelBatch[p];
+            const VecRows vr(c->plan.cls[cl]);
             BatchSolveSeg s{};
-            s.structs = D.structs;
-            s.G = c->G[cl];
-            s.half = D.wstore * k;
-            s.relinds = D.relinds;
-            s.L = (const char*)D.L + eb * b * D.fstore;
-            s.LT = (const char*)D.LT + eb * b * D.fstore;
-            s.Xp = c->Xp;
-            s.W = c->W;
+            s.F = (const char*)D.F + eb * b * D.fentries;
+            s.dinv = (const char*)D.dinv + eb * b * D.xrows;
+            s.V = c->vec[cl];
             s.P = c->P;
+            s.bsrc = D.bsrc;
+            s.blist = D.blist;
+            s.udst = D.udst;
+            s.w = vr.w;
+            s.g0 = vr.g0;
+            s.g1 = vr.g1;
+            s.xrows = D.xrows;
+            s.zero = c->plan.cls[cl].nblocks;
             s.k = k;
             bs.solveSegs.push_back(s);
             return (int)bs.solveSegs.size() - 1;
@@ -1204,18 +1336,19 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             const ClassPlan& plan = c->plan.cls[cl];
             const ClassDev& D = c->dev[cl];
             const int seg = solveSeg(p);
-            const int kb = k <= 8 ? 8 : 16;
+            const int kb = k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : 64;
             for (int ph = 0; ph < 2; ++ph)
-                for (int d = 0; d <= plan.maxDepth; ++d) {
-                    const ClassPlan::SolveLevel& lv = plan.solveLevels[d];
-                    const ClassPlan::Range& r = ph == 0 ? lv.f : lv.b;
+                for (int d = 0; d < (int)plan.blevels.size(); ++d) {
+                    const ClassPlan::BlockLevel& lv = plan.blevels[d];
                     const int sub = ph == 0 ? 1 + dmax - d : 2 + dmax + d;
-                    if (r.count > 0)
-                        stages[Key{dir, t, sub, 0, r.rows * 10000 + r.waves * 100 + kb}]
-                            .push_back(Entry{i, seg, D.mv + r.start, r.count});
-                    if (r.rcount > 0)
+                    if (lv.count[ph] > 0)
+                        stages[Key{dir, t, sub, 0, kb}].push_back(
+                            Entry{i, seg, (const char*)(D.btiles + lv.start[ph]),
+                                  (int)sizeof(BlockTile), lv.count[ph]});
+                    if (lv.rcount[ph] > 0)
                         stages[Key{dir, t, sub, 1, 0}].push_back(
-                            Entry{i, seg, D.mvred + r.rstart, r.rcount});
+                            Entry{i, seg, (const char*)(D.breds + lv.rstart[ph]),
+                                  (int)sizeof(BlockRed), lv.rcount[ph]});
                 }
         };
         for (int p = 0; p < g.numPanels; ++p) {
@@ -1241,14 +1374,12 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
         if (copy)
             L.op = key[2] == 0 ? (key[0] == 0 ? BATCH_COPY_IN : BATCH_ZERO_SET_PLANE)
                                : BATCH_COPY_OUT;
-        L.rows = key[4] / 10000;
-        L.waves = key[4] / 100 % 100;
-        L.kb = key[4] % 100;
+        L.kb = key[4];
         L.blk0 = (int64_t)bs.blocks.size();
         for (const Entry& e : kv.second)
             for (int j = 0; j < e.count; ++j) {
                 BatchBlock b{};
-                b.item = copy ? nullptr : e.items + j;
+                b.item = copy ? nullptr : e.items + (size_t)j * e.stride;
                 b.seg = e.seg;
                 b.problem = e.problem;
                 b.blk = j;
@@ -1266,8 +1397,7 @@ void LaunchBatchSweep(const BatchSweep& bs, const hipStream_t* gs)
         const hipStream_t s = gs[L.group];
         const BatchBlock* b = bs.dBlocks + L.blk0;
         if (L.kind == BatchSweep::PRODUCTS)
-            LaunchSolveBatch<T>(L.ph, L.rows, L.waves, L.kb, b, L.nblocks, bs.dSolve, bs.dActive,
-                                s);
+            LaunchSolveBatch<T>(L.ph, L.kb, b, L.nblocks, bs.dSolve, bs.dActive, s);
         else if (L.kind == BatchSweep::REDUCE)
             LaunchReduceBatch<T>(L.ph, b, L.nblocks, bs.dSolve, bs.dActive, s);
         else
@@ -1662,111 +1792,98 @@ int SolveBatchMerged(psp_hip_ctx* const* ctxs, void* const* Bs, const int* ks, i
 
 namespace {
 
-// Tile-shape tuner for the front solves: for every panel class, level and
-// phase, times the launch (products + reduce) of each candidate shape on the
-// class's panels (one launch per panel, cold factors) and keeps the fastest.  The estimate of one sweep's
-// product time weighs each class by its panel solves per sweep (2P - 1 in
-// all: every panel forward, every panel but the last backward).
+// Tuner of the merged solves' tiles: for every panel class, depth group and
+// direction, times the launch with each candidate number of inner blocks per
+// tile on the class's panels (one launch per panel, cold factors) and keeps
+// the fastest.  The estimate of one sweep's product time weighs each class
+// by its panel solves per sweep (2P - 1 in all: every panel forward, every
+// panel but the last backward).
 template <typename T>
 int Autotune(psp_hip_ctx* c, int k, double* before, double* after)
 {
-    // Candidate shapes replace the device tile lists that captured sweeps
-    // read: drop the graphs first, and on any failure put the old shapes and
-    // their tiles back.
+    // Candidates replace the device tile lists that captured sweeps read:
+    // drop the graphs first, and on any failure put the old tiles back.
     HIPCHK(c, hipStreamSynchronize(c->stream));
     FreeGraphs(c);
-    std::array<std::vector<std::array<SolveShape, 2>>, 3> saved;
+    std::array<std::vector<std::array<int, 2>>, 3> saved;
     for (int cl = 0; cl < 3; ++cl)
-        if (c->plan.present[cl]) saved[cl] = c->plan.cls[cl].shapes;
+        if (c->plan.present[cl]) saved[cl] = c->plan.cls[cl].slices;
     auto restore = [&](int code) {
         (void)hipStreamSynchronize(c->stream);
         for (int cl = 0; cl < 3; ++cl)
-            if (c->plan.present[cl]) c->plan.cls[cl].shapes = saved[cl];
+            if (c->plan.present[cl]) c->plan.cls[cl].slices = saved[cl];
         const std::string msg = c->err;
         (void)RebuildSolveTiles(c);
         c->err = msg;
         return code;
     };
+    struct Events {
+        hipEvent_t e[2] = {nullptr, nullptr};
+        ~Events()
+        {
+            for (hipEvent_t x : e)
+                if (x) (void)hipEventDestroy(x);
+        }
+    } ev;
     int rc = EnsureWorkspace(c, k, 1);
     if (rc) return restore(rc);
     hipStream_t s = c->stream;
-    hipEvent_t ea, eb;
-    HIPCHK(c, hipEventCreate(&ea));
-    HIPCHK(c, hipEventCreate(&eb));
+    for (hipEvent_t& x : ev.e) HIPCHK(c, hipEventCreate(&x));
     const Geometry& g = c->plan.geo;
     double tb = 0, ta = 0;
     for (int cl = 0; cl < 3 && !rc; ++cl) {
         if (!c->plan.present[cl]) continue;
         ClassPlan& P = c->plan.cls[cl];
-        ClassDev& D = c->dev[cl];
+        const ClassDev& D = c->dev[cl];
         double weight = 0;
         for (int p = 0; p < g.numPanels; ++p)
             if (g.cls(p) == cl) weight += p + 1 < g.numPanels ? 2 : 1;
-        auto timeShape = [&](int d, int ph, SolveShape sh, double* t) -> int {
-            P.shapes[d][ph] = sh;
-            BuildSolveTiles(P);
-            BuildClassQueues(c, P);  // keeps the partial slots of the fused launches
+        // seconds of every (group, direction) launch with the current slices
+        auto timeAll = [&](std::vector<std::array<double, 2>>& t) -> int {
+            BuildBlockTiles(P);
             int st;
-            if ((st = ReUpload(c, &D.mv, SolveTiles(P, P.mv))) ||
-                (st = ReUpload(c, &D.mvred, SolveTiles(P, P.mvred))) ||
-                (st = ReUpload(c, &D.redcBuf, ReduceCounters(P))) ||
-                (st = EnsureWorkspace(c, k, 1)))
-                return st;
-            SetSliceReduce(c, D);
-            const size_t eb_ = FrontBytes(c);
-            LaunchFillZero(c->Xp, (int64_t)(eb_ * P.n * k), s);
-            LaunchFillZero(c->W, (int64_t)(eb_ * P.wstore * k), s);
-            LaunchPanelSolve<T>(D, P, 0, c->Xp, c->W, c->P, c->G[cl], k, s, nullptr, d, ph);  // warm
-            // each repetition applies another panel's factors (where the
-            // class has several), so they come from HBM as in a sweep rather
-            // than from the caches the previous repetition filled
-            constexpr int kReps = 3;
-            HIPCHK(c, hipEventRecord(ea, s));
-            for (int r = 0; r < kReps; ++r)
-                LaunchPanelSolve<T>(D, P, (r + 1) % D.npanels, c->Xp, c->W, c->P, c->G[cl], k, s,
-                                    nullptr, d, ph);
-            HIPCHK(c, hipEventRecord(eb, s));
-            HIPCHK(c, hipEventSynchronize(eb));
-            HIPCHK(c, hipGetLastError());
-            float ms = 0;
-            HIPCHK(c, hipEventElapsedTime(&ms, ea, eb));
-            *t = ms * 1e-3 / kReps;
+            if ((st = UploadTiles(c, cl)) || (st = EnsureWorkspace(c, k, 1))) return st;
+            LaunchFillZero(c->vec[cl], (int64_t)(FrontBytes(c) * VecRows(P).total * k), s);
+            t.assign(P.groups.size(), {0, 0});
+            for (size_t d = 0; d < P.groups.size(); ++d)
+                for (int ph = 0; ph < 2; ++ph) {
+                    auto launch = [&](int b) {
+                        LaunchPanelSolve<T>(D, P, b, c->vec[cl], c->P, k, s, nullptr, (int)d, ph);
+                    };
+                    launch(0);  // warm
+                    // each repetition applies another panel's factors (where
+                    // the class has several), so they come from HBM as in a
+                    // sweep rather than from the caches
+                    constexpr int kReps = 3;
+                    HIPCHK(c, hipEventRecord(ev.e[0], s));
+                    for (int r = 0; r < kReps; ++r) launch((r + 1) % D.npanels);
+                    HIPCHK(c, hipEventRecord(ev.e[1], s));
+                    HIPCHK(c, hipEventSynchronize(ev.e[1]));
+                    HIPCHK(c, hipGetLastError());
+                    float ms = 0;
+                    HIPCHK(c, hipEventElapsedTime(&ms, ev.e[0], ev.e[1]));
+                    t[d][ph] = ms * 1e-3 / kReps;
+                }
             return PSP_HIP_OK;
         };
-        for (int d = 0; d <= P.maxDepth && !rc; ++d)
-            for (int ph = 0; ph < 2 && !rc; ++ph) {
-                const SolveShape cur = P.shapes[d][ph];
-                SolveShape best = cur;
-                double tcur = 0;
-                if ((rc = timeShape(d, ph, cur, &tcur))) break;
-                double tbest = tcur;
-                std::vector<SolveShape> cands;
-                for (int rows : {64, 32, 16})
-                    for (int split : {1, 2, 4, 8, 16}) cands.push_back(SolveShape{rows, split, 4});
-                if (k >= 8 && k < 32)  // 16-wave workgroups exist on the matrix-core path
-                    for (int rows : {32, 16})
-                        for (int split : {1, 2, 4}) cands.push_back(SolveShape{rows, split, 16});
-                if (k >= 8 && k <= 16)  // persistent pipelined workgroups
-                    for (int rows : {64, 32, 16})
-                        for (int split : {1, 2, 4}) cands.push_back(SolveShape{rows, split, 4, 1});
-                for (const SolveShape& cand : cands) {
-                    if (rc || (cand.rows == cur.rows && cand.split == cur.split &&
-                               cand.waves == cur.waves && cand.persist == cur.persist))
-                        continue;
-                    double t = 0;
-                    if ((rc = timeShape(d, ph, cand, &t))) break;
-                    if (t < 0.97 * tbest) {
-                        tbest = t;
-                        best = cand;
+        std::vector<std::array<double, 2>> best, t;
+        std::vector<std::array<int, 2>> keep = P.slices;
+        if ((rc = timeAll(best))) break;
+        for (const auto& x : best) tb += weight * (x[0] + x[1]);
+        for (int inner : {4, 8, 12, 16, 24, 32, 48, 64, 96}) {
+            for (auto& x : P.slices) x = {inner, inner};
+            if ((rc = timeAll(t))) break;
+            for (size_t d = 0; d < t.size(); ++d)
+                for (int ph = 0; ph < 2; ++ph)
+                    if (t[d][ph] < 0.97 * best[d][ph]) {
+                        best[d][ph] = t[d][ph];
+                        keep[d][ph] = inner;
                     }
-                }
-                P.shapes[d][ph] = best;
-                tb += weight * tcur;
-                ta += weight * tbest;
-            }
+        }
+        if (rc) break;
+        P.slices = keep;
+        for (const auto& x : best) ta += weight * (x[0] + x[1]);
     }
-    (void)hipEventDestroy(ea);
-    (void)hipEventDestroy(eb);
     if (rc) return restore(rc);
     if ((rc = RebuildSolveTiles(c))) return restore(rc);
     if (before) *before = tb;
@@ -1867,12 +1984,8 @@ int psp_hip_set_option(psp_hip_ctx* c, int option, int value)
         for (auto& D : c->dev) SetSliceReduce(c, D);
         return PSP_HIP_OK;
     }
-    if (option == PSP_HIP_OPT_SOLVE_PERSIST_GRID) {
+    if (option == PSP_HIP_OPT_SOLVE_PERSIST_GRID) {  // no launch is persistent any more
         if (value < 0) return Fail(c, PSP_HIP_ERR_INVALID, "persistent grid cap must be >= 0");
-        if (c->devReady) (void)hipStreamSynchronize(c->stream);
-        FreeGraphs(c);  // captured launches keep their grid sizes
-        c->mvpGrid = value;
-        for (auto& D : c->dev) D.mvpGrid = value;
         return PSP_HIP_OK;
     }
     if (option == PSP_HIP_OPT_SOLVE_FUSED || option == PSP_HIP_OPT_SOLVE_FUSED_QUEUES ||
@@ -1915,9 +2028,11 @@ int psp_hip_set_option(psp_hip_ctx* c, int option, int value)
             c->plan.maxSplit = value;
         }
         for (int cl = 0; cl < 3; ++cl)
-            if (c->plan.present[cl])
+            if (c->plan.present[cl]) {
                 DefaultSolveShapes(c->plan.cls[cl], c->plan.minTiles, c->plan.maxSplit,
                                    c->plan.wideWg, c->plan.persist);
+                DefaultSlices(c->plan.cls[cl], c->plan.minTiles, c->plan.maxSplit);
+            }
         return RebuildSolveTiles(c);
     }
     return Fail(c, PSP_HIP_ERR_INVALID, "unknown option");
@@ -1934,45 +2049,18 @@ int psp_hip_factor(psp_hip_ctx* c, const double* velocity, int scheme, psp_hip_f
     const double t0 = Now();
     int st = EnsureDevice(c);
     if (st) return st;
-    if ((st = EnsureFactorStorage(c))) return st;
-    // a new factorization invalidates the captured sweeps' results only, not
-    // their launches: the graphs keep reading the same factor arrays
     c->factored = false;
     const int64_t N = (int64_t)c->desc.nx * c->desc.ny * c->desc.nz;
     HIPCHK(c, hipMemcpyAsync(c->vel, velocity, sizeof(double) * N, hipMemcpyHostToDevice,
                              c->stream));
-    // The Schur-complement (U) and inversion (T) scratch lives only while
-    // factoring, so that many factored problems fit in HBM at once.
-    const size_t eb = FrontBytes(c);
-    for (int cl = 0; cl < 3; ++cl) {
-        if (!c->plan.present[cl]) continue;
-        ClassDev& D = c->dev[cl];
-        if ((st = Alloc(c, &D.U, eb * (size_t)D.npanels * D.ustore, c->facAllocs)) ||
-            (st = Alloc(c, &D.T, eb * (size_t)D.npanels * D.tstore, c->facAllocs))) {
-            FreeFactorScratch(c);
-            return st;
-        }
-    }
-    double tf = 0, tl = 0, ti = 0;
-    double tsc = 0;
-    st = c->desc.precision == PSP_HIP_FRONTS_FP32 ? FactorClasses<float>(c, &tf, &tl, &ti, &tsc)
-                                                  : FactorClasses<double>(c, &tf, &tl, &ti, &tsc);
-    if (st) {
-        (void)hipStreamSynchronize(c->stream);
-        for (hipStream_t x : c->side)
-            if (x) (void)hipStreamSynchronize(x);
-        FreeFactorScratch(c);
-        return st;
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    FreeFactorScratch(c);
-    c->factored = true;
+    double t[4] = {0, 0, 0, 0};
+    if ((st = Factor(c, t))) return st;
     if (rep) {
         rep->seconds_total = Now() - t0;
-        rep->seconds_fill = tf;
-        rep->seconds_ldl = tl;
-        rep->seconds_inverse = ti;
-        rep->seconds_schur = tsc;
+        rep->seconds_fill = t[0];
+        rep->seconds_ldl = t[1];
+        rep->seconds_inverse = t[2];
+        rep->seconds_schur = t[3];
         double fl = 0, sc = 0, by = 0;
         int nf = 0;
         for (int cl = 0; cl < 3; ++cl) {
@@ -2083,8 +2171,8 @@ int psp_hip_precondition_noalloc(psp_hip_ctx* c, void* B, int k)
     if (!c->scratch) return Fail(c, PSP_HIP_ERR_STATE, "device scratch not set up");
     const SweepSizes z = SweepBufferSizes(c, k);
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t need = up(z.xp) + up(z.w) + up(z.p) + up(z.g[0]) + up(z.g[1]) + up(z.g[2]) +
-                        up(z.s[0]) + up(z.s[1]) + up(z.s[2]);
+    size_t need = up(z.p) + up(z.xp) + up(z.w);
+    for (int cl = 0; cl < 3; ++cl) need += up(z.v[cl]) + up(z.g[cl]) + up(z.s[cl]);
     if (need > kScratchBytes)
         return Fail(c, PSP_HIP_ERR_INVALID,
                     "precondition_noalloc: the sweep needs " + std::to_string(need) +
@@ -2094,25 +2182,32 @@ int psp_hip_precondition_noalloc(psp_hip_ctx* c, void* B, int k)
     // the slot copies and the vectors' padding rows must read as zero; a
     // fill kernel clears the whole region (no memset node if captured)
     LaunchFillZero(base, (int64_t)need, c->stream);
-    void* keep[6] = {c->Xp, c->W, c->P, c->G[0], c->G[1], c->G[2]};
-    int32_t* keepS[3] = {c->S[0], c->S[1], c->S[2]};
     size_t off = 0;
-    auto take = [&](size_t b) {
-        void* q = b ? base + off : nullptr;
+    auto swap = [&](auto*& p, size_t b) {
+        auto* old = p;
+        p = b ? (decltype(old))(base + off) : nullptr;
         off += up(b);
-        return q;
+        return old;
     };
-    c->Xp = take(z.xp);
-    c->W = take(z.w);
-    c->P = take(z.p);
-    for (int cl = 0; cl < 3; ++cl) c->G[cl] = take(z.g[cl]);
-    for (int cl = 0; cl < 3; ++cl) c->S[cl] = (int32_t*)take(z.s[cl]);
+    void* const p = swap(c->P, z.p);
+    void* const xp = swap(c->Xp, z.xp);
+    void* const w = swap(c->W, z.w);
+    void *v[3], *g[3];
+    int32_t* sy[3];
+    for (int cl = 0; cl < 3; ++cl) {
+        v[cl] = swap(c->vec[cl], z.v[cl]);
+        g[cl] = swap(c->G[cl], z.g[cl]);
+        sy[cl] = swap(c->S[cl], z.s[cl]);
+    }
     SweepEager(c, (c128*)B, k);
-    c->Xp = keep[0];
-    c->W = keep[1];
-    c->P = keep[2];
-    for (int cl = 0; cl < 3; ++cl) c->G[cl] = keep[3 + cl];
-    for (int cl = 0; cl < 3; ++cl) c->S[cl] = keepS[cl];
+    c->P = p;
+    c->Xp = xp;
+    c->W = w;
+    for (int cl = 0; cl < 3; ++cl) {
+        c->vec[cl] = v[cl];
+        c->G[cl] = g[cl];
+        c->S[cl] = sy[cl];
+    }
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return PSP_HIP_OK;

@@ -2,7 +2,9 @@
 #include "symbolic.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <stack>
 
@@ -927,6 +929,494 @@ void BuildQueues(ClassPlan& C, int nqueues, int rows, int cut, int wgPerQueue)
     C.nqueues = nqueues;
 }
 
+// --------------------------------------------------------------------------
+// Merged solves
+// --------------------------------------------------------------------------
+namespace {
+
+// Cost of one launch of the merged solves in seconds: a launch of a few MB
+// takes kLaunchSec, and larger ones stream their factor at kStreamRate
+// (measured on MI355X with launches of 2 to 270 MB: 3 us + bytes / 6.2 TB/s
+// for plain streaming; the index and vector loads before and the stores
+// after add about 3 us).  Composing a merged front's columns costs kFoldRate
+// flops a second (FP64) once per factorization, charged to kFoldSolves solves
+// of the panel, 16 sweeps.  Measured at 100^3 with FP64 fronts, one
+// factorization and one sweep: uncharged 121.9 ms, charged to 64, 32 and 16
+// solves 112.9, 113.1 and 107.7; a solve of 56 FP32 sweeps 579, 589, 579, 603.
+constexpr double kLaunchSec = 6e-6, kStreamRate = 5.5e12, kFoldRate = 3.5e13, kFoldSolves = 32;
+constexpr int kMaxGroup = 6;  // depths merged at most
+
+// Depth groups that minimize the estimated time of a panel solve: merging
+// depths saves launches and adds factor entries (a pivot's column then spans
+// every pivot above it in the group and the top node's update rows).
+std::vector<std::array<int, 2>> MergeGroups(const ClassPlan& C, int entryBytes)
+{
+    const int D = C.maxDepth + 1;
+    std::vector<std::vector<double>> ent(D, std::vector<double>(kMaxGroup, 0.0));
+    std::vector<std::vector<double>> fold(D, std::vector<double>(kMaxGroup, 0.0));
+    for (const Node& n : C.nodes) {
+        // columns of this node in a group whose top depth is n.depth - j
+        const Node* a = &n;
+        double above = 0;
+        for (int j = 0; j < kMaxGroup; ++j) {
+            ent[n.depth][j] += n.size * (n.size + 1.0) / 2 + (double)n.size * (above + a->usize);
+            fold[n.depth][j] +=
+                8.0 * n.size * std::min<double>(above, n.usize) * (a->usize + above / 2);
+            if (a->parent < 0) break;
+            a = &C.nodes[a->parent];
+            above += a->size;
+        }
+    }
+    // (FP32 fronts: half the bytes, twice the rate)
+    const double foldRate = kFoldRate * 16 / entryBytes;
+    std::vector<double> best(D + 1, 0.0);
+    std::vector<int> from(D + 1, 0);
+    for (int d1 = 0; d1 < D; ++d1) {  // best[d1 + 1]: depths 0 .. d1
+        best[d1 + 1] = 1e300;
+        for (int d0 = d1; d0 >= 0 && d1 - d0 < kMaxGroup; --d0) {
+            double e = 0, f = 0;
+            for (int d = d0; d <= d1; ++d) {
+                e += ent[d][d - d0];
+                f += fold[d][d - d0];
+            }
+            const double t = best[d0] + kLaunchSec + e * entryBytes / kStreamRate +
+                             f / foldRate / (2 * kFoldSolves);
+            if (t < best[d1 + 1]) {
+                best[d1 + 1] = t;
+                from[d1 + 1] = d0;
+            }
+        }
+    }
+    std::vector<std::array<int, 2>> g;
+    for (int d = D; d > 0; d = from[d]) g.insert(g.begin(), {from[d], d - 1});
+    return g;
+}
+
+// Merged fronts, solve order, block rows, the vector rows of every update
+// row and the fold's lists for C.groups; false when an update row of a front
+// is touched by more than two of its children.
+bool LayMerged(ClassPlan& C, int tile)
+{
+    const int nn = (int)C.nodes.size();
+    std::vector<int> groupOf(C.maxDepth + 1), top(nn), mcol(nn, 0), first(nn, 0);
+    for (size_t g = 0; g < C.groups.size(); ++g)
+        for (int d = C.groups[g][0]; d <= C.groups[g][1]; ++d) groupOf[d] = (int)g;
+    C.bnodes.clear();
+    C.bnodeOf.assign(nn, -1);
+    C.browBase.clear();
+    C.browLo.clear();
+    std::vector<std::vector<int>> members(nn);
+    for (int t = nn - 1; t >= 0; --t) {
+        const Node& n = C.nodes[t];
+        top[t] = n.depth == C.groups[groupOf[n.depth]][0] ? t : top[n.parent];
+    }
+    for (int t = 0; t < nn; ++t) members[top[t]].push_back(t);
+    int x = 0, w = 0, u0 = 0;
+    int64_t blocks = 0;
+    for (int t = 0; t < nn; ++t) {
+        if (members[t].empty()) continue;
+        BlockNode b;
+        b.top = t;
+        b.group = groupOf[C.nodes[t].depth];
+        for (int f : members[t]) {
+            mcol[f] = b.s;
+            first[f] = b.s;
+            for (int c : C.nodes[f].child)
+                if (c >= 0 && top[c] == t) first[f] = std::min(first[f], first[c]);
+            b.s += C.nodes[f].size;
+        }
+        if (b.s == 0) continue;
+        for (int f : members[t]) C.bnodeOf[f] = (int)C.bnodes.size();
+        b.u = C.nodes[t].usize;
+        b.sb = (int)CeilDiv(b.s, kBlk);
+        b.ub = (int)CeilDiv(b.u, kBlk);
+        b.x0 = x;
+        b.w0 = w;
+        b.u0 = u0;
+        b.br0 = (int)C.browBase.size();
+        x += kBlk * b.sb;
+        w += kBlk * (b.sb + b.ub);
+        u0 += kBlk * b.ub;
+        size_t at = 0;  // the member whose pivots reach the block row
+        for (int r = 0; r < b.sb + b.ub; ++r) {
+            int lo = 0, hi = b.sb;
+            if (r < b.sb) {
+                lo = b.s;
+                hi = r + 1;
+                while (mcol[members[t][at]] + C.nodes[members[t][at]].size <= kBlk * r) ++at;
+                for (size_t i = at; i < members[t].size(); ++i) {
+                    const int f = members[t][i];
+                    if (mcol[f] >= kBlk * (r + 1)) break;
+                    if (C.nodes[f].size > 0) lo = std::min(lo, first[f]);
+                }
+                lo /= kBlk;
+            }
+            C.browBase.push_back((int32_t)(blocks - lo));
+            C.browLo.push_back(lo);
+            blocks += hi - lo;
+        }
+        C.bnodes.push_back(b);
+    }
+    if (blocks > INT32_MAX / 2) return false;
+    C.nblocks = (int)blocks;
+    C.xrows = x;
+    C.wrows = w;
+    // panel-vector row of every padded unknown
+    std::vector<int> xrow(C.n, -1);
+    C.sxy.assign(x, 0);
+    C.sv.assign(x, -1);
+    for (int q = 0; q < C.n; ++q) {
+        const int f = C.qnode[q];
+        xrow[q] = C.bnodes[C.bnodeOf[f]].x0 + mcol[f] + C.qcol[q];
+        C.sxy[xrow[q]] = C.qxy[q];
+        C.sv[xrow[q]] = C.qv[q];
+    }
+    C.udst.assign(u0, 0);
+    C.usrc.assign(u0, C.xrows);
+    const VecRows V(C);
+    // row of unknown q in merged front m: a pivot row, or an update row
+    auto rowIn = [&](int m, int q) {
+        const BlockNode& b = C.bnodes[m];
+        const int f = C.qnode[q];
+        if (C.bnodeOf[f] == m) return mcol[f] + C.qcol[q];
+        const Node& t = C.nodes[b.top];
+        const int* s0 = C.structs.data() + t.ustart;
+        const int* p = std::lower_bound(s0, s0 + t.usize, q);
+        return p != s0 + t.usize && *p == q ? kBlk * b.sb + int(p - s0) : -1;
+    };
+    std::vector<unsigned char> touched(w, 0);
+    for (BlockNode& b : C.bnodes) {
+        const Node& t = C.nodes[b.top];
+        b.parent = t.parent < 0 ? -1 : C.bnodeOf[t.parent];
+        if (b.parent < 0) continue;
+        BlockNode& p = C.bnodes[b.parent];
+        p.leaf = false;
+        for (int a = 0; a < b.u; ++a) {
+            const int q = C.structs[t.ustart + a];
+            const int r = rowIn(b.parent, q);
+            if (r < 0) return false;
+            C.usrc[b.u0 + a] = xrow[q];
+            const int k = touched[p.w0 + r]++;
+            if (k > 1) return false;
+            C.udst[b.u0 + a] = k == 1        ? (int32_t)(V.g1 + p.w0 + r)
+                               : r < p.s     ? p.x0 + r
+                                             : (int32_t)(V.g0 + p.u0 + r - kBlk * p.sb);
+        }
+    }
+    // fold: E = -L_BL Linv per node, top blocks and the tops' E copied,
+    // the other nodes' columns composed from their ancestors'
+    C.foldNodes.assign(nn, FoldNode{});
+    C.packs.clear();
+    C.estore = 0;
+    C.foldE.tileStart = (int)C.tiles.size();
+    for (int t = 0; t < nn; ++t) {
+        const Node& n = C.nodes[t];
+        FoldNode& f = C.foldNodes[t];
+        f.l = n.loff;
+        f.e = C.estore;
+        f.s = n.size;
+        f.u = n.usize;
+        f.urow = -1;
+        if (n.size == 0) continue;
+        const BlockNode& b = C.bnodes[C.bnodeOf[t]];
+        f.mcol = mcol[t];
+        f.br0 = b.br0;
+        f.x0 = b.x0 + mcol[t];
+        if (b.top == t) f.urow = kBlk * b.sb;
+        C.estore += (int64_t)n.size * n.usize;
+        for (int j0 = 0; j0 < n.size; j0 += 32) {
+            for (int i0 = j0; i0 < n.size; i0 += 32) C.packs.push_back({t, i0, j0, 0});
+            if (b.top == t)
+                for (int i0 = 0; i0 < n.usize; i0 += 32) C.packs.push_back({t, n.size + i0, j0, 0});
+        }
+        if (n.usize == 0) continue;
+        const int fs = n.size + n.usize;
+        GemmDesc g{};
+        g.a = n.loff + n.size;
+        g.b = n.loff;
+        g.c = f.e;
+        g.lda = g.ldb = fs;
+        g.ldc = n.usize;
+        g.M = n.usize;
+        g.N = g.K = n.size;
+        g.abuf = g.bbuf = g.dbuf = BUF_L;
+        g.cbuf = BUF_U;
+        g.flags = G_BUNIT | G_NEG | G_BETA0;
+        AddGemmTiles(C, g, tile);
+    }
+    C.foldE.tileCount = (int)C.tiles.size() - C.foldE.tileStart;
+    C.flist.clear();
+    C.fsrc.clear();
+    C.compose.clear();
+    C.fkeys.clear();
+    C.composeTiles.clear();
+    C.composeSteps.clear();
+    std::vector<int> listOf(nn, -1), listLen(nn, 0), at;
+    for (int off = 1; off < kMaxGroup; ++off) {
+        GemmLaunch gl;
+        gl.tileStart = (int)C.composeTiles.size();
+        for (int c = 0; c < nn; ++c) {
+            const Node& n = C.nodes[c];
+            if (n.size == 0 || n.depth - C.nodes[top[c]].depth != off) continue;
+            const int m = C.bnodeOf[c], p = n.parent;
+            const BlockNode& b = C.bnodes[m];
+            if (listOf[p] < 0) {
+                listOf[p] = (int)C.flist.size();
+                for (int a = p;; a = C.nodes[a].parent) {
+                    for (int i = 0; i < C.nodes[a].size; ++i) C.flist.push_back(mcol[a] + i);
+                    if (a == b.top) break;
+                }
+                for (int i = 0; i < b.u; ++i) C.flist.push_back(kBlk * b.sb + i);
+                listLen[p] = (int)C.flist.size() - listOf[p];
+            }
+            at.assign((size_t)kBlk * (b.sb + b.ub), -1);
+            for (int i = 0; i < listLen[p]; ++i) at[C.flist[listOf[p] + i]] = i;
+            ComposeDesc d{};
+            d.e = C.foldNodes[c].e;
+            d.lde = n.usize;
+            d.list = listOf[p];
+            d.rows = listLen[p];
+            d.br0 = b.br0;
+            d.piv = listLen[p] - b.u;
+            d.ccol = mcol[c];
+            d.n = n.size;
+            d.src = (int)C.fsrc.size();
+            C.fsrc.resize(C.fsrc.size() + listLen[p], -1);
+            for (int a = 0; a < n.usize; ++a) {
+                const int r = rowIn(m, C.structs[n.ustart + a]);
+                if (r < 0 || at[r] < 0) return false;
+                C.fsrc[d.src + at[r]] = a;
+            }
+            d.kl = (int)C.fkeys.size();
+            for (int i = 0; i < d.piv; ++i)
+                if (C.fsrc[d.src + i] >= 0)
+                    C.fkeys.push_back({C.flist[d.list + i], i, C.fsrc[d.src + i], 0});
+            d.k = (int)C.fkeys.size() - d.kl;
+            const int di = (int)C.compose.size();
+            C.compose.push_back(d);
+            for (int tn = 0; tn < d.n; tn += tile)
+                for (int tm = 0; tm < d.rows; tm += tile) {
+                    int32_t kend = 0;
+                    while (kend < d.k && C.fkeys[d.kl + kend].pos < tm + tile) ++kend;
+                    C.composeTiles.push_back({di, tm, tn, kend});
+                }
+        }
+        gl.tileCount = (int)C.composeTiles.size() - gl.tileStart;
+        if (gl.tileCount > 0) C.composeSteps.push_back(gl);
+    }
+    return true;
+}
+
+// Output tiles of a merged front: blocks dealt evenly to tiles of at most 4.
+template <class F>
+void ForTiles(int blocks, const F& f)
+{
+    const int nt = (int)CeilDiv(blocks, 4);
+    for (int i = 0, b = 0; i < nt; ++i) {
+        const int n = (blocks - b + nt - i - 1) / (nt - i);
+        f(b, n);
+        b += n;
+    }
+}
+
+// Inner blocks of the tile of output blocks [ob0, ob0 + nob): forward the
+// columns [lo, hi) of its rows, backward the block rows that meet its columns.
+int TileInner(const ClassPlan& C, const BlockNode& b, int ph, int ob0, int nob, int* lo,
+              std::vector<int>* rows)
+{
+    if (ph == 0) {
+        int l = b.sb, h = 0;
+        for (int r = ob0; r < ob0 + nob; ++r) {
+            l = std::min(l, C.browLo[b.br0 + r]);
+            h = std::max(h, std::min(b.sb, r + 1));
+        }
+        *lo = l;
+        return h - l;
+    }
+    int n = 0;
+    for (int r = ob0; r < b.sb + b.ub; ++r)
+        if (C.browLo[b.br0 + r] < ob0 + nob) {
+            if (rows) rows->push_back(r);
+            ++n;
+        }
+    return n;
+}
+
+}  // namespace
+
+void BuildMerged(ClassPlan& C, int entryBytes)
+{
+    constexpr int kTile = 64;  // of the fold's products
+    C.groups = MergeGroups(C, entryBytes);
+    const size_t tiles = C.tiles.size(), gemms = C.gemms.size();
+    if (LayMerged(C, kTile)) return;
+    // one group per depth: every front has at most two children
+    C.tiles.resize(tiles);
+    C.gemms.resize(gemms);
+    C.groups.clear();
+    for (int d = 0; d <= C.maxDepth; ++d) C.groups.push_back({d, d});
+    if (!LayMerged(C, kTile)) C.bnodes.clear();
+}
+
+void DefaultSlices(ClassPlan& C, int minTiles, int maxSplit)
+{
+    // 64 output rows times kMinInner inner blocks is the smallest piece worth
+    // a workgroup: its waves have all their loads in flight at once.
+    constexpr int kMinInner = 8, kMaxInner = 48;
+    C.slices.assign(C.groups.size(), {kMaxInner, kMaxInner});
+    for (size_t g = 0; g < C.groups.size(); ++g)
+        for (int ph = 0; ph < 2; ++ph) {
+            int64_t units = 0;
+            int longest = 0;
+            for (const BlockNode& b : C.bnodes) {
+                if (b.group != (int)g) continue;
+                ForTiles(ph == 0 ? b.sb + b.ub : b.sb, [&](int ob0, int nob) {
+                    int lo;
+                    const int n = TileInner(C, b, ph, ob0, nob, &lo, nullptr);
+                    units += n;
+                    longest = std::max(longest, n);
+                });
+            }
+            const int per = (int)CeilDiv(CeilDiv(units, std::max(1, 2 * minTiles)), 4) * 4;
+            C.slices[g][ph] = std::max((int)CeilDiv(longest, std::max(1, 4 * maxSplit)),
+                                       std::min(kMaxInner, std::max(kMinInner, per)));
+        }
+}
+
+void BuildBlockTiles(ClassPlan& C)
+{
+    const VecRows V(C);
+    C.btiles.clear();
+    C.breds.clear();
+    C.blist.clear();
+    C.bsrc.clear();
+    C.bslots = 0;
+    C.blevels.assign(C.groups.size(), {});
+    for (size_t g = 0; g < C.groups.size(); ++g)
+        for (int ph = 0; ph < 2; ++ph) {
+            ClassPlan::BlockLevel& L = C.blevels[g];
+            const int slice = C.slices[g][ph];
+            L.rstart[ph] = (int)C.breds.size();
+            struct Unit {
+                std::vector<BlockTile> tiles;  // one tile, or the slices of one
+                int work = 0;
+            };
+            std::vector<Unit> units;
+            int slots = 0;
+            std::vector<int> rows;
+            for (const BlockNode& b : C.bnodes) {
+                if (b.group != (int)g) continue;
+                L.vecRows[ph] += 2.0 * b.s + b.u;
+                ForTiles(ph == 0 ? b.sb + b.ub : b.sb, [&](int ob0, int nob) {
+                    BlockTile t{};
+                    t.x0 = b.x0;
+                    t.w0 = b.w0;
+                    t.u0 = b.u0;
+                    t.s = b.s;
+                    t.u = b.u;
+                    t.sb = b.sb;
+                    t.leaf = b.leaf;
+                    t.ob0 = ob0;
+                    t.nob = nob;
+                    t.slot = t.red = -1;
+                    int lo = 0;
+                    rows.clear();
+                    const int n = TileInner(C, b, ph, ob0, nob, &lo, &rows);
+                    if (ph == 0) {
+                        for (int q = 0; q < nob; ++q) {
+                            const int r = ob0 + q;
+                            t.base[q] = C.browBase[b.br0 + r];
+                            t.lo[q] = C.browLo[b.br0 + r];
+                            t.hi[q] = std::min(b.sb, r + 1);
+                        }
+                    } else {
+                        t.lst = (int)(C.blist.size() / 4);
+                        for (int r : rows) {
+                            const int rlo = C.browLo[b.br0 + r], rhi = std::min(b.sb, r + 1);
+                            for (int q = 0; q < 4; ++q) {
+                                const int c = ob0 + q;
+                                C.blist.push_back(q < nob && c >= rlo && c < rhi
+                                                      ? C.browBase[b.br0 + r] + c
+                                                      : C.nblocks);
+                            }
+                            for (int i = 0; i < kBlk; ++i)
+                                C.bsrc.push_back(r < b.sb
+                                                     ? (int32_t)(V.w + b.x0 + kBlk * r + i)
+                                                     : C.usrc[b.u0 + kBlk * (r - b.sb) + i]);
+                        }
+                        lo = 0;
+                    }
+                    Unit un;
+                    un.work = n;
+                    const int ns = std::max(1, (int)CeilDiv(n, slice));
+                    if (ns > 1) {
+                        BlockRed rd{};
+                        rd.x0 = t.x0;
+                        rd.w0 = t.w0;
+                        rd.u0 = t.u0;
+                        rd.s = t.s;
+                        rd.u = t.u;
+                        rd.sb = t.sb;
+                        rd.leaf = t.leaf;
+                        rd.ob0 = ob0;
+                        rd.nob = nob;
+                        rd.slot0 = slots;
+                        rd.nslots = ns;
+                        t.red = (int)C.breds.size();
+                        C.breds.push_back(rd);
+                    }
+                    for (int j = 0, at = 0; j < ns; ++j) {
+                        t.ib0 = lo + at;
+                        t.nib = (n - at + ns - j - 1) / (ns - j);
+                        at += t.nib;
+                        if (ns > 1) t.slot = slots++;
+                        un.tiles.push_back(t);
+                    }
+                    units.push_back(std::move(un));
+                });
+            }
+            for (int d = C.groups[g][0]; d <= C.groups[g][1]; ++d)
+                for (int t : C.levels[d]) {
+                    const Node& n = C.nodes[t];
+                    double above = 0;
+                    int a = t;
+                    for (; C.nodes[a].depth > C.groups[g][0]; above += C.nodes[a].size)
+                        a = C.nodes[a].parent;
+                    L.entries[ph] += n.size * (n.size + 1.0) / 2 +
+                                     (double)n.size * (above + C.nodes[a].usize);
+                }
+            L.rcount[ph] = (int)C.breds.size() - L.rstart[ph];
+            C.bslots = std::max(C.bslots, slots);
+            // Longest first, so that the launch does not end with one long
+            // workgroup.  With slices, workgroup i runs on XCD i % 8 and a
+            // tile's slices go to positions of one residue, each tile to the
+            // residue with the least work so far; free positions are holes
+            // (no output blocks).
+            std::stable_sort(units.begin(), units.end(),
+                             [](const Unit& a, const Unit& b) { return a.work > b.work; });
+            L.start[ph] = (int)C.btiles.size();
+            if (L.rcount[ph] == 0) {
+                for (const Unit& un : units) C.btiles.push_back(un.tiles[0]);
+            } else {
+                std::vector<BlockTile> lane[8];
+                int64_t load[8] = {0};
+                for (const Unit& un : units) {
+                    const int best = (int)(std::min_element(load, load + 8) - load);
+                    lane[best].insert(lane[best].end(), un.tiles.begin(), un.tiles.end());
+                    load[best] += un.work + 4 * (int)un.tiles.size();
+                }
+                size_t len = 0;
+                for (const auto& l : lane) len = std::max(len, l.size());
+                BlockTile hole{};
+                hole.slot = hole.red = -1;
+                for (size_t i = 0; i < len; ++i)
+                    for (const auto& l : lane) C.btiles.push_back(i < l.size() ? l[i] : hole);
+            }
+            L.count[ph] = (int)C.btiles.size() - L.start[ph];
+        }
+    C.bsrc.resize(C.bsrc.size() + kStagePad, 0);
+}
+
 int BuildPlan(const psp_hip_desc& d, Plan& plan, std::string& msg)
 {
     if (d.nx < 1 || d.ny < 1 || d.nz < 1 || d.bz < 1 || d.planesPerPanel < 1 ||
@@ -954,6 +1444,13 @@ int BuildPlan(const psp_hip_desc& d, Plan& plan, std::string& msg)
         Analyse(C, orig);
         AssemblyMeta(plan.geo, C);
         Schedule(plan, C);
+        BuildMerged(C, d.precision == PSP_HIP_FRONTS_FP32 ? 8 : 16);
+        if (C.bnodes.empty()) {
+            msg = "internal error: inconsistent merged fronts";
+            return PSP_HIP_ERR_INVALID;
+        }
+        DefaultSlices(C, plan.minTiles, plan.maxSplit);
+        BuildBlockTiles(C);
         // Every index the kernels dereference must land inside its front.
         for (const Node& n : C.nodes)
             for (int a = 0; a < n.usize; ++a) {

@@ -161,6 +161,87 @@ struct GemmLaunch {
     int32_t tileStart = 0, tileCount = 0;
 };
 
+// ---------------------------------------------------------------------------
+// Merged solves.  The tree levels are cut into groups of consecutive depths;
+// the nodes of one group under a common ancestor (the group's top node) form
+// one merged front, solved with the explicit inverse of its whole pivot
+// block, so a panel solve takes one launch per group and direction instead
+// of one per level.  A merged front's factor F has the group's pivots as
+// columns and, as rows, the same pivots (Linv, unit lower) followed by the
+// top node's update rows (-L_BL Linv), in blocks of 16 x 16.  Blocks are
+// stored once, row of blocks by row of blocks, and serve both directions:
+//   forward   [y; w] = F g          (y scaled by D^-1 for the backward pass)
+//   backward  x = F^T [D^-1 y; x_struct].
+// Pivots keep their post-order, so the pivots under a node are contiguous
+// and row i of F has its entries in one column range: from the first pivot
+// below i's node to i.  Blocks of siblings that do not meet are not stored.
+// ---------------------------------------------------------------------------
+constexpr int kBlk = 16;
+
+struct BlockNode {
+    int top = -1;            // the group's top node (fine tree)
+    int group = 0;
+    int s = 0, u = 0;        // pivots, update rows
+    int sb = 0, ub = 0;      // the same in blocks
+    int x0 = 0;              // first panel-vector row (solve order, multiple of 16)
+    int w0 = 0;              // first work row; rows [0, 16 sb) pivots, then the update rows
+    int u0 = 0;              // first entry of udst / usrc (16 ub entries)
+    int br0 = 0;             // first block row (browBase, browLo); sb + ub of them
+    int parent = -1;         // merged parent
+    bool leaf = true;        // no merged children
+};
+
+// One workgroup of a merged solve: up to 4 output blocks (one per wave) and
+// a range of inner blocks.  128 bytes, read once.
+struct BlockTile {
+    int32_t x0, w0, u0, s;      // of the node
+    int32_t u, sb, leaf, ob0;   // first output block (row of blocks forward, column backward)
+    int32_t nob, ib0, nib, lst; // inner blocks [ib0, ib0 + nib); lst: first entry of blist / bsrc (backward)
+    int32_t slot, red;          // partial-sum slot and reduce item of an inner slice, -1 if none
+    int32_t pad_[2];
+    int32_t base[4];            // forward: block (row ob0 + q, column j) is base[q] + j
+    int32_t lo[4], hi[4];       // forward: its columns [lo, hi)
+    int32_t pad2_[4];
+};
+static_assert(sizeof(BlockTile) == 128, "BlockTile is one 128-byte record");
+
+// A split set of output blocks: the tile's fields with its slots.
+struct BlockRed {
+    int32_t x0, w0, u0, s;
+    int32_t u, sb, leaf, ob0;
+    int32_t nob, slot0, nslots, pad_[5];
+};
+static_assert(sizeof(BlockRed) == 64, "BlockRed is one 64-byte record");
+
+// Fold of one fine node into its merged front.
+struct FoldNode {
+    int64_t l;           // factor offset (BUF_L), (s + u) x s
+    int64_t e;           // E = -L_BL Linv, u x s (in the update scratch)
+    int32_t s, u;
+    int32_t mcol;        // first pivot within the merged front
+    int32_t br0;         // the merged front's first block row
+    int32_t x0;          // panel-vector row of the node's first pivot
+    int32_t urow;        // merged row of the first update row (group tops), -1 otherwise
+};
+
+// Columns of a node below its group's top: F_c = F_A P + ext(E_c), with A the
+// node's ancestors in the group (their columns already folded), P the rows of
+// E_c at their pivots and ext its rows at the top node's update rows.
+// flist[list ..] are the merged rows involved: the pivots of A, nearest
+// ancestor first, then the update rows; F_A is lower triangular in this order.
+// Only the k pivots that E_c has a row for (the node's ring) enter the product.
+struct ComposeDesc {
+    int64_t e;
+    int32_t lde, list, rows, br0;
+    int32_t k, ccol, n;
+    int32_t src;         // fsrc[src ..]: E_c's row at each entry of flist, -1 if none
+    int32_t kl, piv;     // fkeys[kl ..]: the k pivots; entries of flist that are pivots
+};
+struct ComposeKey {      // a pivot of F_A: column of F, entry of flist, E_c's row
+    int32_t col, pos, row, pad_;
+};
+static_assert(sizeof(FoldNode) == 40 && sizeof(ComposeDesc) == 48, "fold records");
+
 struct ClassPlan {
     int cls = 0;
     int vsize = 0;
@@ -251,6 +332,39 @@ struct ClassPlan {
     };
     QueuePhase queue[2];
 
+    // Merged solves (BuildMerged, BuildBlockTiles).
+    std::vector<std::array<int, 2>> groups;  // first and last depth of each group, top group first
+    std::vector<BlockNode> bnodes;
+    std::vector<int> bnodeOf;        // merged front of each fine node (-1: no pivots in it)
+    int xrows = 0;                   // panel-vector rows in solve order, padding included
+    int wrows = 0;                   // work rows
+    int nblocks = 0;                 // 16 x 16 blocks of one panel's factor; block nblocks is zero
+    int64_t estore = 0;              // entries of all E of one panel
+    std::vector<int32_t> sxy, sv;    // qxy, qv per panel-vector row (sv -1: padding)
+    std::vector<int32_t> browBase, browLo;
+    std::vector<int32_t> udst;       // vector row an update row is added into, see VecRows
+    std::vector<int32_t> usrc;       // panel-vector row of an update row (backward input)
+    std::vector<FoldNode> foldNodes;
+    std::vector<TransItem> packs;    // 32 x 32 pieces copied into F: node, row, column of its front
+    std::vector<ComposeDesc> compose;
+    std::vector<ComposeKey> fkeys;
+    std::vector<GemmTile> composeTiles;    // pad_: keys that meet the tile's rows
+    std::vector<GemmLaunch> composeSteps;  // by depth below the group's top, 1, 2, ...
+    std::vector<int32_t> flist, fsrc;
+    GemmLaunch foldE;                // E = -L_BL Linv
+    struct BlockLevel {              // one group: tiles and reduce items per direction
+        int start[2] = {0, 0}, count[2] = {0, 0};
+        int rstart[2] = {0, 0}, rcount[2] = {0, 0};
+        double entries[2] = {0, 0}, vecRows[2] = {0, 0};
+    };
+    std::vector<std::array<int, 2>> slices;  // per group and direction: inner blocks per tile
+    std::vector<BlockLevel> blevels;
+    std::vector<BlockTile> btiles;
+    std::vector<BlockRed> breds;
+    std::vector<int32_t> blist;      // backward: 4 blocks per inner block (nblocks: not stored)
+    std::vector<int32_t> bsrc;       // backward: 16 vector rows per inner block
+    int bslots = 0;
+
     // Algorithmic work per panel.
     double flops = 0, schurFlops = 0, solveFlopsPerRhs = 0;
     double factorEntries = 0;
@@ -275,6 +389,35 @@ struct Plan {
     int fusedWgPerQueue = 64;   // workgroups a queue expects (inner slices are
                                 // cut so a level has about that many tiles)
 };
+
+// Rows (of the solve vector) and entries (of bsrc) a workgroup may read past
+// its tile's inner range, unused.
+constexpr int kStagePad = 256;
+
+// Rows of a class's solve vector, one buffer: the panel vector (xrows rows
+// and 16 zero rows), the forward results (xrows), and two copies of what
+// children add to a front: g0, its update rows (at their u0), and g1, all its
+// work rows (at w0).  A child adds into its parent's pivot rows in place
+// (panel-vector rows) when it is the first to touch them, and to its parent's
+// update rows in g0; the second child to touch a row writes it in g1.  No row
+// is touched by more than two children.
+struct VecRows {
+    int64_t w, g0, g1, total;
+    explicit VecRows(const ClassPlan& C)
+        : w(C.xrows + kBlk), g0(w + C.xrows), g1(g0 + (int64_t)C.udst.size()),
+          total(g1 + C.wrows + kStagePad)
+    {
+    }
+};
+
+// Depth groups of the merged solves, the merged fronts and the fold's work
+// lists.  entryBytes: bytes of a factor entry.
+void BuildMerged(ClassPlan& C, int entryBytes);
+// Inner blocks per tile: as many as give about `minTiles` workgroups a launch,
+// in at most maxSplit slices.
+void DefaultSlices(ClassPlan& C, int minTiles, int maxSplit);
+// (Re)builds the merged solves' tiles from C.slices.
+void BuildBlockTiles(ClassPlan& C);
 
 // Builds everything; returns PSP_HIP_OK or an error code with `msg` set.
 int BuildPlan(const psp_hip_desc& desc, Plan& plan, std::string& msg);

@@ -301,12 +301,10 @@ class DistHelmholtz:
     def set_solve_tiling(self, min_tiles=None, max_split=None, wide_wg=None, persist=None,
                          persist_grid=None, fused=None, fused_queues=None, fused_rows=None,
                          fused_cut=None, fused_wg=None, xcd_reduce=None):
-        """Default front-solve tile shapes: workgroups wanted per launch, the
-        most inner slices per row block, whether levels with few row blocks
-        get 16-wave workgroups instead of slices, and whether the solves run
-        on persistent pipelined workgroups (8 <= k <= 16); rebuilds the solve
-        tiles.  persist_grid caps the workgroups of a persistent launch
-        (0: as many as fit on the device).  fused: the tree levels from the
+        """Default front-solve tiles: workgroups wanted per launch and the
+        most inner slices per tile (in quarters); rebuilds the solve tiles.
+        wide_wg, persist and persist_grid are accepted and change nothing in
+        the merged solves.  fused: the tree levels from the
         cut depth down as one persistent launch per direction (8 <= k <= 16),
         with fused_queues subtree queues (one per XCD; more leave queues the
         last workgroup runs alone), fused_rows output rows per tile and the
