@@ -1517,9 +1517,11 @@ struct BlockShape {
 // Fields of a tile (scalar loads).
 struct TileRec {
     int x0, w0, u0, s, u, sb, leaf, ob0, nob, ib0, nib, lst, slot, red;
-    __device__ explicit TileRec(ConstInts t)
+    int base, lo, hi;  // forward: of wave q's output block
+    __device__ TileRec(ConstInts t, int q)
         : x0(t[0]), w0(t[1]), u0(t[2]), s(t[3]), u(t[4]), sb(t[5]), leaf(t[6]), ob0(t[7]),
-          nob(t[8]), ib0(t[9]), nib(t[10]), lst(t[11]), slot(t[12]), red(t[13])
+          nob(t[8]), ib0(t[9]), nib(t[10]), lst(t[11]), slot(t[12]), red(t[13]),
+          base(t[16 + q]), lo(t[20 + q]), hi(t[24 + q])
     {
     }
 };
@@ -1527,8 +1529,8 @@ struct TileRec {
 // Inner slices of a tile: each wave's partial sums are in P; the slice that
 // arrives last sums the slots in slot order and finishes the rows.
 template <typename T, int PH>
-__device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& a, int k,
-                                          int32_t* redc, const BlockRed* reds)
+__device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& a, int k, int r0,
+                                          int kc, int32_t* redc, const BlockRed* reds)
 {
     __shared__ int arrived;
     const int tid = threadIdx.x;
@@ -1541,8 +1543,8 @@ __device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& 
     if (Uni(arrived) != nslots - 1) return;
     const L2Buf<T> lP(a.P);
     constexpr int kS = 8;  // slots loaded together
-    for (int e = tid; e < t.nob * kBlk * k; e += 256) {
-        const int rl = e / k, r = e % k;
+    for (int e = tid; e < t.nob * kBlk * kc; e += 256) {
+        const int rl = e / kc, r = r0 + e % kc;
         cx<T> v = czero<T>();
         for (int j0 = 0; j0 < nslots; j0 += kS) {
             cx<T> pv[kS];
@@ -1558,7 +1560,98 @@ __device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& 
     if (tid == 0) redc[t.red] = 0;  // no slice of this launch counts any more
 }
 
-// One workgroup on tile tp, up to KB = 8 or 16 right-hand sides (shared by
+// Finish operands of a lane's 4 rows (rows row(lk, p) of output block ob):
+// D^-1 of pivot rows, or where update rows go.
+template <typename T>
+struct FinishOps {
+    cx<T> d[4];
+    int32_t dst[4];
+    __device__ void Load(const BlockBufs<T>& a, const TileRec& t, int ob, int lk)
+    {
+        if (ob < t.sb) {
+            const cx<T>* p = a.dinv + t.x0 + kBlk * ob;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = p[Mfma<T>::row(lk, i)];
+        } else {
+            const int32_t* p = a.udst + t.u0 + kBlk * (ob - t.sb);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i] = p[Mfma<T>::row(lk, i)];
+        }
+    }
+};
+
+// Stores a wave's output block: products of right-hand sides r0 + 8 n + li
+// (li < 8, below r0 + kc), as partial sums of a slice or finished.  The loads
+// of an update block are issued together for each n.
+template <typename T, int PH, int NB>
+__device__ __forceinline__ void StoreBlock(const BlockBufs<T>& a, const TileRec& t, int q, int k,
+                                           int r0, int kc, const FinishOps<T>& fo,
+                                           const typename Mfma<T>::acc (&acc)[NB])
+{
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int ob = t.ob0 + q;
+    cx<T> o[NB][4];
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            o[n][p] = cx<T>{T(acc[n][p]), T(__shfl_xor(acc[n][p], 8, 64))};
+    auto each = [&](auto&& f) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) f(n, p, Mfma<T>::row(lk, p), 8 * n + li);
+    };
+    if (t.slot >= 0) {
+        cx<T>* out = a.P + ((int64_t)t.slot * 64 + kBlk * q) * k + r0;
+        each([&](int n, int p, int row, int r) {
+            if (li < 8 && r < kc) out[row * k + r] = o[n][p];
+        });
+    } else if (PH == PH_B) {
+        cx<T>* out = a.V + (int64_t)(t.x0 + kBlk * ob) * k + r0;
+        each([&](int n, int p, int row, int r) {
+            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = o[n][p];
+        });
+    } else if (ob < t.sb) {
+        cx<T>* out = a.V + (a.w + t.x0 + kBlk * ob) * k + r0;
+        each([&](int n, int p, int row, int r) {
+            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = o[n][p] * fo.d[p];
+        });
+    } else {
+        // an update row: the children's contributions to it and, for a pivot
+        // row of the parent, what that holds
+        const int ru = kBlk * (ob - t.sb);
+        const cx<T>* g0 = a.V + (a.g0 + t.u0 + ru) * k + r0;
+        const cx<T>* g1 = a.V + (a.g1 + t.w0 + kBlk * ob) * k + r0;
+        cx<T>* out[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) out[p] = a.V + (int64_t)fo.dst[p] * k + r0;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const int r = 8 * n + li, rc = min(r, kc - 1);
+            cx<T> x[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) x[p] = out[p][rc];
+            if (!t.leaf) {
+                cx<T> ga[4], gb[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    ga[p] = g0[Mfma<T>::row(lk, p) * k + rc];
+                    gb[p] = g1[Mfma<T>::row(lk, p) * k + rc];
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p) o[n][p] = ga[p] + gb[p] + o[n][p];
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const cx<T> v = fo.dst[p] < a.xrows ? x[p] + o[n][p] : o[n][p];
+                if (li < 8 && r < kc && ru + Mfma<T>::row(lk, p) < t.u) out[p][r] = v;
+            }
+        }
+    }
+}
+
+// One workgroup: up to KB = 8 or 16 right-hand sides of a tile (shared by
 // k_block and k_block_batch).  Reads of the vector and of the index lists may
 // run past the tile's inner range (up to a chunk; the buffers are padded);
 // those rows are not multiplied.
@@ -1571,16 +1664,9 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
     constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT, U = S::U;
     constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
     __shared__ cx<T> vs[CB * kBlk][KB];
-    const ConstInts tw = Const(tp);
-    const TileRec t(tw);
     const int tid = threadIdx.x, lane = tid & 63, q = Uni(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
-    const int ob = t.ob0 + q;
-    const bool own = q < t.nob, top = ob < t.sb;
-    const int base = PH == PH_F ? tw[16 + q] : 0, blo = PH == PH_F ? tw[20 + q] : 0;
-    const int bhi = PH == PH_F ? tw[24 + q] : 0;
-    const int nch = (t.nib + CB - 1) / CB;
-    const int32_t* src = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0);
+    const TileRec t(Const(tp), q);
     const uint32_t loff = PH == PH_F ? lk * kBlk + li : li * kBlk + 4 * lk;
     const uint32_t rk = min(tid % KB, k - 1);           // staged right-hand side
     const uint32_t voff = (tid / KB) * k + rk;
@@ -1598,7 +1684,7 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
         int blk;
         if constexpr (PH == PH_F) {
             const int j = t.ib0 + c * CB + i;
-            blk = j >= blo && j < bhi ? base + j : a.zero;
+            blk = j >= t.lo && j < t.hi ? t.base + j : a.zero;
         } else {
             blk = __builtin_amdgcn_readlane(list, i);
         }
@@ -1609,8 +1695,8 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
     };
     cx<T> sa[SPT], sg[PH == PH_F ? SPT : 1];
     auto stage = [&](int c) {
-        const int row0 = kBlk * (t.ib0 + c * CB);
         if constexpr (PH == PH_F) {
+            const int row0 = kBlk * (t.ib0 + c * CB);
             const cx<T>* x = a.V + (int64_t)(t.x0 + row0) * k;
             const cx<T>* g = a.V + (a.g1 + t.w0 + row0) * k;
 #pragma unroll
@@ -1623,7 +1709,7 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
                 for (int p = 0; p < SPT; ++p) sg[p] = czero<T>();
             }
         } else {
-            const int32_t* ix = src + c * CB * kBlk;
+            const int32_t* ix = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0 + c * CB);
             uint32_t sx[SPT];
 #pragma unroll
             for (int p = 0; p < SPT; ++p) sx[p] = (uint32_t)(ix + p * RP)[tid / KB];
@@ -1643,8 +1729,6 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
         }
     };
     acc_t acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
     // vector operands of the block at inner index i of the chunk
     struct Operand {
         cx<T> v[4][NB];
@@ -1669,21 +1753,6 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
                 acc[n] = Mfma<T>::step(m[u][st].i, b2, acc[n]);
             }
     };
-    // finish operands of this lane's rows: D^-1, or where update rows go
-    const bool fin = own && t.slot < 0 && PH == PH_F;
-    uint32_t dst[4] = {0, 0, 0, 0};
-    cx<T> fd[PH == PH_F ? 4 : 1];
-    if (fin) {
-        if (top) {
-            const cx<T>* d = a.dinv + t.x0 + kBlk * ob;
-#pragma unroll
-            for (int p = 0; p < 4; ++p) fd[PH == PH_F ? p : 0] = d[Mfma<T>::row(lk, p)];
-        } else {
-            const int32_t* d = a.udst + t.u0 + kBlk * (ob - t.sb);
-#pragma unroll
-            for (int p = 0; p < 4; ++p) dst[p] = d[Mfma<T>::row(lk, p)];
-        }
-    }
     // the chunk's products, half a ring at a time (blocks past the range are
     // the zero block), each register group refilled as soon as it is used
     auto run = [&](int c) {
@@ -1706,14 +1775,21 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
             if (i0 + U >= CB) return;
         }
     };
+    // the first loads all go out before the first wait
     loadList(0);
     stage(0);
 #pragma unroll
     for (int u = 0; u < U; ++u) issue(u, 0, u);
-    __builtin_amdgcn_sched_barrier(0);  // all loads go out before the first wait
+    __builtin_amdgcn_sched_barrier(0);
+    const bool own = q < t.nob;
+    FinishOps<T> fo;
+    if (PH == PH_F && own && t.slot < 0) fo.Load(a, t, t.ob0 + q, lk);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
     put();
     LdsBarrier();
     run(0);
+    const int nch = (t.nib + CB - 1) / CB;
     for (int c = 1; c < nch; ++c) {
         loadList(c);
         stage(c);
@@ -1722,102 +1798,52 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
         LdsBarrier();
         run(c);
     }
-    if (own) {
-        cx<T> o[NB][4];
-#pragma unroll
-        for (int n = 0; n < NB; ++n)
-#pragma unroll
-            for (int p = 0; p < 4; ++p)
-                o[n][p] = cx<T>{T(acc[n][p]), T(__shfl_xor(acc[n][p], 8, 64))};
-        // element (n, p): row kBlk ob + row(lk, p), right-hand side 8 n + li
-        const int ru = kBlk * (ob - t.sb);  // first update row
-        auto each = [&](auto&& f) {
-#pragma unroll
-            for (int n = 0; n < NB; ++n)
-#pragma unroll
-                for (int p = 0; p < 4; ++p) f(n, p, Mfma<T>::row(lk, p), 8 * n + li);
-        };
-        if (t.slot >= 0) {
-            cx<T>* out = a.P + ((int64_t)t.slot * 64 + kBlk * q) * k;
-            each([&](int n, int p, int row, int r) {
-                if (li < 8 && r < k) out[row * k + r] = o[n][p];
-            });
-        } else if (PH == PH_B) {
-            cx<T>* out = a.V + (int64_t)(t.x0 + kBlk * ob) * k;
-            each([&](int n, int p, int row, int r) {
-                if (li < 8 && r < k && kBlk * ob + row < t.s) out[row * k + r] = o[n][p];
-            });
-        } else if (top) {
-            cx<T>* out = a.V + (a.w + t.x0 + kBlk * ob) * k;
-            each([&](int n, int p, int row, int r) {
-                if (li < 8 && r < k && kBlk * ob + row < t.s)
-                    out[row * k + r] = o[n][p] * fd[PH == PH_F ? p : 0];
-            });
-        } else {
-            // an update row: the children's contributions to it and, for a
-            // pivot row of the parent, what that holds
-            const cx<T>* g0 = a.V + (a.g0 + t.u0 + ru) * k;
-            const cx<T>* g1 = a.V + (a.g1 + t.w0 + kBlk * ob) * k;
-#pragma unroll
-            for (int n = 0; n < NB; ++n) {
-                const int r = 8 * n + li, rc = min(r, k - 1);
-                cx<T> x[4];
-#pragma unroll
-                for (int p = 0; p < 4; ++p) x[p] = a.V[dst[p] * (uint32_t)k + rc];
-                if (!t.leaf) {
-                    cx<T> ga[4], gb[4];
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) {
-                        ga[p] = g0[Mfma<T>::row(lk, p) * k + rc];
-                        gb[p] = g1[Mfma<T>::row(lk, p) * k + rc];
-                    }
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) o[n][p] = ga[p] + gb[p] + o[n][p];
-                }
-#pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const cx<T> v = (int)dst[p] < a.xrows ? x[p] + o[n][p] : o[n][p];
-                    if (li < 8 && r < k && ru + Mfma<T>::row(lk, p) < t.u)
-                        a.V[dst[p] * (uint32_t)k + r] = v;
-                }
-            }
-        }
-    }
-    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, redc, reds);
+    if (own) StoreBlock<T, PH, NB>(a, t, q, k, 0, k, fo, acc);
+    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, 0, k, redc, reds);
 }
 
-// The same for wide blocks of right-hand sides: passes of up to KB = 32 or 64
-// over the tile, CB inner blocks at a time in two LDS buffers; the vector and
-// factor loads of the next chunks are in flight while a chunk is multiplied.
+// The same for one pass (right-hand sides KB pass .. + KB) of a wide block.
+// Bound by the matrix cores and by waiting for loads, so the vector and the
+// factor blocks of the next two chunks of CB inner blocks are in flight, each in
+// its own registers, while one is multiplied from LDS (two buffers), and blocks
+// that a tile does not have are skipped.  The passes are workgroups of one
+// launch: a loop over them in one workgroup, on one staged chunk ahead, took
+// 41.7 ms a sweep at 100^3 k = 64 FP32 and 66.0 in FP64 (29.2 and 52.5 so);
+// 15.8 ms at 120 x 96 x 60 k = 32 FP32 (11.9).  CB = 4 and three workgroups a CU
+// spill registers and were slower.
 template <typename T, int KB>
 struct WideShape {
     static constexpr int NB = KB / 8;
-    static constexpr int CB = sizeof(T) == 4 && KB == 32 ? 4 : 2;
+    static constexpr int CB = 2;
     static constexpr int SPT = CB * kBlk * KB / 256;  // staged elements per thread
 };
 
 template <typename T, int PH, int KB>
 __device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBufs<T>& a, int k,
-                                              int32_t* redc, const BlockRed* reds)
+                                              int pass, int32_t* redc, const BlockRed* reds)
 {
     typedef typename Mfma<T>::acc acc_t;
     typedef WideShape<T, KB> S;
     constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT;
     __shared__ cx<T> vs[2][CB * kBlk][KB];
-    const ConstInts tw = Const(tp);
-    const TileRec t(tw);
     const int tid = threadIdx.x, lane = tid & 63, q = Uni(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
-    const int ob = t.ob0 + q;
-    const int base = PH == PH_F ? tw[16 + q] : 0, blo = PH == PH_F ? tw[20 + q] : 0;
-    const int bhi = PH == PH_F ? tw[24 + q] : 0;
-    const ConstInts bl = Const(a.blist) + 4 * (int64_t)(t.lst + t.ib0) + q;
-    const int32_t* src = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0);
     const uint32_t loff = PH == PH_F ? lk * kBlk + li : li * kBlk + 4 * lk;
-    const int nch = (t.nib + CB - 1) / CB;
     struct Chunk {
+        int blk[CB];  // wave-uniform
         cx<T> m[CB][4];
     };
+    const int r0 = KB * pass, kc = min(KB, k - r0);
+    constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
+    const int rr = r0 + min(tid % KB, kc - 1);
+    const uint32_t voff = (tid / KB) * k + rr;
+    struct Stage {
+        cx<T> a[SPT], g[PH == PH_F ? SPT : 1];
+    };
+    const TileRec t(Const(tp), q);
+    const ConstInts bl = Const(a.blist) + 4 * (int64_t)(t.lst + t.ib0) + q;
+    const int32_t* src = a.bsrc + (int64_t)kBlk * (t.lst + t.ib0);
+    const int nch = (t.nib + CB - 1) / CB;
     auto factor = [&](int c, Chunk& d) {
 #pragma unroll
         for (int b = 0; b < CB; ++b) {
@@ -1826,125 +1852,111 @@ __device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBu
             if (i < t.nib) {
                 if constexpr (PH == PH_F) {
                     const int j = t.ib0 + i;
-                    if (j >= blo && j < bhi) blk = base + j;
+                    if (j >= t.lo && j < t.hi) blk = t.base + j;
                 } else {
                     blk = bl[4 * i];
                 }
             }
+            if (q >= t.nob) blk = a.zero;
+            d.blk[b] = blk;
             const cx<T>* p = a.F + (int64_t)blk * (kBlk * kBlk);
 #pragma unroll
             for (int st = 0; st < 4; ++st) d.m[b][st] = (p + (PH == PH_F ? 4 * kBlk * st : st))[loff];
         }
     };
-    for (int r0 = 0; r0 < k; r0 += KB) {
-        const int kc = min(KB, k - r0);
-        acc_t acc[NB];
+    acc_t acc[NB];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
-        constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
-        const int rr = r0 + min(tid % KB, kc - 1);
-        const uint32_t voff = (tid / KB) * k + rr;
-        // (stages past the end read the last chunk again, unused)
-        int32_t sx[PH == PH_B ? SPT : 1];
-        auto indices = [&](int c) {
-            if constexpr (PH == PH_B) {
-                const int32_t* ix = src + min(c, nch - 1) * CB * kBlk;
+    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
+    // (stages past the end read the last chunk again, unused)
+    int32_t sx[PH == PH_B ? SPT : 1];
+    auto indices = [&](int c) {
+        if constexpr (PH == PH_B) {
+            const int32_t* ix = src + min(c, nch - 1) * CB * kBlk;
 #pragma unroll
-                for (int p = 0; p < SPT; ++p) sx[p] = (ix + p * RP)[tid / KB];
-            }
-        };
-        cx<T> sa[SPT], sg[PH == PH_F ? SPT : 1];
-        auto stage = [&](int c) {
-            if constexpr (PH == PH_F) {
-                const int row0 = kBlk * (t.ib0 + min(c, nch - 1) * CB);
-                const cx<T>* x = a.V + (int64_t)(t.x0 + row0) * k;
-                const cx<T>* g = a.V + (a.g1 + t.w0 + row0) * k;
+            for (int p = 0; p < SPT; ++p) sx[p] = (ix + p * RP)[tid / KB];
+        }
+    };
+    auto stage = [&](int c, Stage& d) {
+        if constexpr (PH == PH_F) {
+            const int row0 = kBlk * (t.ib0 + min(c, nch - 1) * CB);
+            const cx<T>* x = a.V + (int64_t)(t.x0 + row0) * k;
+            const cx<T>* g = a.V + (a.g1 + t.w0 + row0) * k;
 #pragma unroll
-                for (int p = 0; p < SPT; ++p) sa[p] = (x + p * RP * k)[voff];
-                if (!t.leaf) {
+            for (int p = 0; p < SPT; ++p) d.a[p] = (x + p * RP * k)[voff];
+            if (!t.leaf) {
 #pragma unroll
-                    for (int p = 0; p < SPT; ++p) sg[p] = (g + p * RP * k)[voff];
-                } else {
-#pragma unroll
-                    for (int p = 0; p < SPT; ++p) sg[p] = czero<T>();
-                }
+                for (int p = 0; p < SPT; ++p) d.g[p] = (g + p * RP * k)[voff];
             } else {
 #pragma unroll
-                for (int p = 0; p < SPT; ++p) sa[p] = a.V[(int64_t)sx[p] * k + rr];
+                for (int p = 0; p < SPT; ++p) d.g[p] = czero<T>();
             }
-        };
-        auto put = [&](int buf) {
+        } else {
 #pragma unroll
-            for (int p = 0; p < SPT; ++p) {
-                const int c = tid / KB + RP * p;
-                const int row = PH == PH_F ? c : (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3);
-                cx<T> v = sa[p];
-                if constexpr (PH == PH_F) v = v + sg[p];
-                vs[buf][row][tid % KB] = mk(v.r, v.i);
-            }
-        };
-        Chunk d0, d1;
-        indices(0);
-        stage(0);
-        indices(1);
-        factor(0, d0);
-        factor(1, d1);
-        auto step = [&](int c, Chunk& d) {
-            put(c & 1);
-            stage(c + 1);
-            indices(c + 2);
-            LdsBarrier();
-#pragma unroll
-            for (int b = 0; b < CB; ++b)
-#pragma unroll
-                for (int st = 0; st < 4; ++st)
-#pragma unroll
-                    for (int n = 0; n < NB; ++n) {
-                        const cx<T> v = vs[c & 1][kBlk * b + 4 * st + lk][8 * n + (li & 7)];
-                        const T b1 = li < 8 ? v.r : v.i;
-                        const T b2 = li < 8 ? -v.i : v.r;
-                        acc[n] = Mfma<T>::step(d.m[b][st].r, b1, acc[n]);
-                        acc[n] = Mfma<T>::step(d.m[b][st].i, b2, acc[n]);
-                    }
-            factor(c + 2, d);
-        };
-        for (int c = 0; c < nch; c += 2) {
-            step(c, d0);
-            if (c + 1 >= nch) break;
-            step(c + 1, d1);
+            for (int p = 0; p < SPT; ++p) d.a[p] = a.V[(int64_t)sx[p] * k + rr];
         }
-        if (q < t.nob) {
+    };
+    auto put = [&](int buf, const Stage& d) {
 #pragma unroll
-            for (int n = 0; n < NB; ++n) {
+        for (int p = 0; p < SPT; ++p) {
+            const int c = tid / KB + RP * p;
+            const int row = PH == PH_F ? c : (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3);
+            cx<T> v = d.a[p];
+            if constexpr (PH == PH_F) v = v + d.g[p];
+            vs[buf][row][tid % KB] = mk(v.r, v.i);
+        }
+    };
+    Chunk d0, d1;
+    Stage s0, s1;
+    indices(0);
+    stage(0, s0);
+    indices(1);
+    stage(1, s1);
+    indices(2);
+    factor(0, d0);
+    factor(1, d1);
+    auto step = [&](int c, Chunk& d, Stage& sv) {
+        put(c & 1, sv);
+        stage(c + 2, sv);
+        indices(c + 3);
+        LdsBarrier();
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const T val = acc[n][p];
-                    const T other = __shfl_xor(val, 8, 64);
-                    const int rl = Mfma<T>::row(lk, p), rr = 8 * n + li;
-                    if (li >= 8 || rr >= kc) continue;
-                    const cx<T> v{val, other};
-                    if (t.slot >= 0)
-                        a.P[((int64_t)t.slot * 64 + kBlk * q + rl) * k + r0 + rr] = v;
-                    else
-                        BlockFinish<T, PH>(a, t.x0, t.w0, t.u0, t.s, t.u, t.sb, t.leaf,
-                                           kBlk * ob + rl, r0 + rr, k, v);
+        for (int b = 0; b < CB; ++b) {
+            if (d.blk[b] == a.zero) continue;
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                    const cx<T> v = vs[c & 1][kBlk * b + 4 * st + lk][8 * n + (li & 7)];
+                    const T b1 = li < 8 ? v.r : v.i;
+                    const T b2 = li < 8 ? -v.i : v.r;
+                    acc[n] = Mfma<T>::step(d.m[b][st].r, b1, acc[n]);
+                    acc[n] = Mfma<T>::step(d.m[b][st].i, b2, acc[n]);
                 }
-            }
         }
-        LdsBarrier();  // the next pass overwrites the staged chunks
+        factor(c + 2, d);
+    };
+    for (int c = 0; c < nch; c += 2) {
+        step(c, d0, s0);
+        if (c + 1 >= nch) break;
+        step(c + 1, d1, s1);
     }
-    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, redc, reds);
+    if (q < t.nob) {
+        FinishOps<T> fo;
+        if (PH == PH_F && t.slot < 0) fo.Load(a, t, t.ob0 + q, lk);
+        StoreBlock<T, PH, NB>(a, t, q, k, r0, kc, fo, acc);
+    }
+    if (redc != nullptr && t.slot >= 0) SumSlices<T, PH>(t, a, k, r0, kc, redc, reds);
 }
 
-// KB right-hand sides per pass: 8 and 16 one pass, 32 and 64 as many as k needs.
+// One tile, right-hand sides KB pass .. + KB (KB 8 and 16: one pass).
 template <typename T, int PH, int KB>
 __device__ __forceinline__ void BlockWork(const BlockTile* tp, const BlockBufs<T>& a, int k,
-                                          int32_t* redc, const BlockRed* reds)
+                                          int pass, int32_t* redc, const BlockRed* reds)
 {
     if constexpr (KB <= 16)
         BlockTileWork<T, PH, KB>(tp, a, k, redc, reds);
     else
-        BlockTileWide<T, PH, KB>(tp, a, k, redc, reds);
+        BlockTileWide<T, PH, KB>(tp, a, k, pass, redc, reds);
 }
 
 // Workgroups per CU the register budget allows for (the most without spills).
@@ -1952,16 +1964,29 @@ template <typename T, int PH, int KB>
 constexpr int BlockOccupancy()
 {
     if (KB > 16) return 2;
-    return PH == PH_B ? 6 : 4;
+    const int wide = KB == 16, f64 = sizeof(T) == 8;
+    return PH == PH_B ? 6 - f64 - wide : 4 - wide;
 }
 
+// Workgroup g of a launch of `count` tiles and `passes` passes: the passes of
+// a tile are 8 workgroups apart, so they run on one XCD at about the same time
+// and the later ones find the factor blocks in its L2.  redc: counters, one
+// set of nreds per pass.
 template <typename T, int PH, int KB>
 __global__ __launch_bounds__(256, (BlockOccupancy<T, PH, KB>())) void k_block(
-    const BlockTile* tiles, BlockBufs<T> a, int k, int32_t* redc, const BlockRed* reds)
+    const BlockTile* tiles, BlockBufs<T> a, int k, int count, int passes, int32_t* redc, int nreds,
+    const BlockRed* reds)
 {
-    const BlockTile* tp = tiles + blockIdx.x;
+    int tile = blockIdx.x, pass = 0;
+    if (KB > 16) {
+        tile = blockIdx.x / (8 * passes) * 8 + blockIdx.x % 8;
+        pass = blockIdx.x / 8 % passes;
+        if (tile >= count) return;
+        if (redc != nullptr) redc += pass * nreds;
+    }
+    const BlockTile* tp = tiles + tile;
     if (Const(tp)[8] <= 0) return;  // a hole of the XCD placement
-    BlockWork<T, PH, KB>(tp, a, k, redc, reds);
+    BlockWork<T, PH, KB>(tp, a, k, pass, redc, reds);
 }
 
 // Sum of the slices of one tile in slot order, then the finish (where the
@@ -2115,7 +2140,7 @@ __global__ __launch_bounds__(256, (BlockOccupancy<T, PH, KB>())) void k_block_ba
     const BlockTile* tp = (const BlockTile*)bb.item;
     const BatchSolveSeg sg = segs[bb.seg];
     if (!active[bb.problem] || Const(tp)[8] <= 0) return;
-    BlockWork<T, PH, KB>(tp, SegBufs<T>(sg), sg.k, nullptr, nullptr);
+    BlockWork<T, PH, KB>(tp, SegBufs<T>(sg), sg.k, bb.blk, nullptr, nullptr);
 }
 
 template <typename T, int PH>
@@ -2749,26 +2774,30 @@ void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, 
                             vr.g1,
                             c.xrows,
                             plan.nblocks};
-    // the partial sums are read through a buffer of at most 4 GiB
-    const bool pfits = (int64_t)sizeof(cx<T>) * k * 64 * plan.bslots < ((int64_t)1 << 32);
+    // the partial sums are read through a buffer of at most 4 GiB, and each
+    // pass needs counters of its own
+    const bool pfits = (int64_t)sizeof(cx<T>) * k * 64 * plan.bslots < ((int64_t)1 << 32) &&
+                       k <= kPassRhs * kMaxPasses;
     int32_t* rc = pfits ? c.bredc : nullptr;
     auto go = [&](auto ph, int g) {
         constexpr int PH = decltype(ph)::value;
         const ClassPlan::BlockLevel& L = plan.blevels[g];
         if (L.count[PH] <= 0) return;
         auto run = [&](auto kb) {
-            hipLaunchKernelGGL((k_block<T, PH, decltype(kb)::value>), dim3(L.count[PH]), dim3(256),
-                               0, s, c.btiles + L.start[PH], bufs, k, rc, c.breds);
+            constexpr int KB = decltype(kb)::value;
+            const int passes = KB <= 16 ? 1 : (k + KB - 1) / KB;
+            const int grid = KB <= 16 ? L.count[PH] : (L.count[PH] + 7) / 8 * 8 * passes;
+            hipLaunchKernelGGL((k_block<T, PH, KB>), dim3(grid), dim3(256), 0, s,
+                               c.btiles + L.start[PH], bufs, k, L.count[PH], passes, rc, c.nbreds,
+                               c.breds);
         };
         ProfBegin(prof, s);
         if (k <= 8)
             run(std::integral_constant<int, 8>());
         else if (k <= 16)
             run(std::integral_constant<int, 16>());
-        else if (k <= 32)
-            run(std::integral_constant<int, 32>());
         else
-            run(std::integral_constant<int, 64>());
+            run(std::integral_constant<int, kPassRhs>());
         ProfEnd(prof, s, sizeof(cx<T>) * (L.entries[PH] + L.vecRows[PH] * k),
                 8.0 * L.entries[PH] * k);
         if (L.rcount[PH] > 0 && !rc)
@@ -2947,10 +2976,8 @@ void LaunchSolveBatch(int ph, int kb, const BatchBlock* blocks, int nblocks,
             run(std::integral_constant<int, 8>());
         else if (kb <= 16)
             run(std::integral_constant<int, 16>());
-        else if (kb <= 32)
-            run(std::integral_constant<int, 32>());
         else
-            run(std::integral_constant<int, 64>());
+            run(std::integral_constant<int, kPassRhs>());
     };
     if (ph == PH_F)
         go(std::integral_constant<int, PH_F>());

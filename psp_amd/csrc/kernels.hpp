@@ -100,8 +100,10 @@ struct ClassDev {
     // merged solves
     BlockTile* btiles = nullptr;
     BlockRed* breds = nullptr;
-    int32_t* bredcBuf = nullptr;    // one arrival counter per reduce item (zero between launches)
+    int32_t* bredcBuf = nullptr;    // one arrival counter per reduce item and pass over the
+                                    // right-hand sides (zero between launches)
     int32_t* bredc = nullptr;       // bredcBuf when slices are summed in the launch
+    int nbreds = 0;
     int32_t *blist = nullptr, *bsrc = nullptr, *udst = nullptr;
     int32_t *sxy = nullptr, *sv = nullptr;
     int32_t xrows = 0;
@@ -116,6 +118,10 @@ struct ClassDev {
     ComposeKey* fkeys = nullptr;
     GemmTile* composeTiles = nullptr;
 };
+
+// Right-hand sides per pass of the product launches for k > 16, and the most
+// passes (k <= 256).
+constexpr int kPassRhs = 32, kMaxPasses = 8;
 
 // Rows of a panel vector and the unknowns they hold (v < 0: padding).
 struct PanelMap {
@@ -234,7 +240,7 @@ void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* 
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,
                         int32_t* sync = nullptr, int nsync = 0);
 // Batched launches over nblocks BatchBlocks: products of phase ph with up to
-// kb (8, 16, 32 or 64) right-hand sides per pass, reduce items, or panel
+// kb (8, 16 or kPassRhs) right-hand sides per pass, reduce items, or panel
 // copies (op).
 template <typename T>
 void LaunchSolveBatch(int ph, int kb, const BatchBlock* blocks, int nblocks,

@@ -647,12 +647,13 @@ int UploadTiles(psp_hip_ctx* c, int cl)
     int st;
     if ((st = ReUpload(c, &D.btiles, P.btiles)) || (st = ReUpload(c, &D.breds, P.breds)) ||
         (st = ReUpload(c, &D.blist, P.blist)) || (st = ReUpload(c, &D.bsrc, P.bsrc)) ||
-        (st = ReUpload(c, &D.bredcBuf, ReduceCounters(P.breds.size()))) ||
+        (st = ReUpload(c, &D.bredcBuf, ReduceCounters(P.breds.size() * kMaxPasses))) ||
         (st = ReUpload(c, &D.mv, fused ? SolveTiles(P, P.mv) : std::vector<SolveTile>{})) ||
         (st = ReUpload(c, &D.mvred, fused ? SolveTiles(P, P.mvred) : std::vector<SolveTile>{})) ||
         (st = ReUpload(c, &D.redcBuf, ReduceCounters(fused ? P.mvred.size() : 0))) ||
         (st = UploadQueues(c, cl)))
         return st;
+    D.nbreds = (int)P.breds.size();
     SetSliceReduce(c, D);
     return PSP_HIP_OK;
 }
@@ -1224,7 +1225,7 @@ int RunSolve(psp_hip_ctx* c, void* B, int k, int m, double relTol, int maxIts, i
 // leaves (level d at step D - d, D the deepest level over all problems, so
 // the roots line up) and the backward phase from the roots.
 // A step's products go in one launch per number of right-hand sides a pass
-// covers (8, 16, 32 or 64).  Each problem's kernels see the tiles, factors and
+// covers (8, 16 or kPassRhs).  Each problem's kernels see the tiles, factors and
 // buffers of its own single-problem sweep, in the same order.
 struct BatchSweep {
     enum Kind { PRODUCTS = 0, REDUCE = 1, COPY = 2 };
@@ -1263,14 +1264,16 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
     // stage key: sweep direction (0 forward, 1 backward), panel step,
     // sub-step (0: first copy; 1 .. 1 + D: forward phase, level D + 1 - sub;
     // 2 + D .. 2 + 2D: backward phase, level sub - 2 - D; 3 + 2D: copy-out),
-    // part (0 products, 1 reduce), right-hand sides per pass (8, 16, 32, 64;
-    // 0 for copies and reduces); a level is a depth group of the merged solves
+    // part (0 products, 1 reduce), right-hand sides per pass (8, 16 or
+    // kPassRhs; 0 for copies and reduces); a level is a depth group of the
+    // merged solves
     using Key = std::array<int, 5>;
     struct Entry {
         int problem, seg;
         const char* items;
-        int stride;  // bytes per item
-        int count;   // tiles / reduce items; copies: workgroups
+        int stride;      // bytes per item
+        int count;       // tiles / reduce items; copies: workgroups
+        int passes = 1;  // workgroups per tile
     };
     std::map<Key, std::vector<Entry>> stages;
     int dmax = 0;
@@ -1336,7 +1339,8 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             const ClassPlan& plan = c->plan.cls[cl];
             const ClassDev& D = c->dev[cl];
             const int seg = solveSeg(p);
-            const int kb = k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : 64;
+            const int kb = k <= 16 ? (k <= 8 ? 8 : 16) : kPassRhs;
+            const int passes = k <= 16 ? 1 : (k + kPassRhs - 1) / kPassRhs;
             for (int ph = 0; ph < 2; ++ph)
                 for (int d = 0; d < (int)plan.blevels.size(); ++d) {
                     const ClassPlan::BlockLevel& lv = plan.blevels[d];
@@ -1344,7 +1348,7 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
                     if (lv.count[ph] > 0)
                         stages[Key{dir, t, sub, 0, kb}].push_back(
                             Entry{i, seg, (const char*)(D.btiles + lv.start[ph]),
-                                  (int)sizeof(BlockTile), lv.count[ph]});
+                                  (int)sizeof(BlockTile), lv.count[ph], passes});
                     if (lv.rcount[ph] > 0)
                         stages[Key{dir, t, sub, 1, 0}].push_back(
                             Entry{i, seg, (const char*)(D.breds + lv.rstart[ph]),
@@ -1377,14 +1381,15 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
         L.kb = key[4];
         L.blk0 = (int64_t)bs.blocks.size();
         for (const Entry& e : kv.second)
-            for (int j = 0; j < e.count; ++j) {
-                BatchBlock b{};
-                b.item = copy ? nullptr : e.items + (size_t)j * e.stride;
-                b.seg = e.seg;
-                b.problem = e.problem;
-                b.blk = j;
-                bs.blocks.push_back(b);
-            }
+            for (int j = 0; j < e.count; ++j)
+                for (int p = 0; p < e.passes; ++p) {
+                    BatchBlock b{};
+                    b.item = copy ? nullptr : e.items + (size_t)j * e.stride;
+                    b.seg = e.seg;
+                    b.problem = e.problem;
+                    b.blk = copy ? j : p;
+                    bs.blocks.push_back(b);
+                }
         L.nblocks = (int)((int64_t)bs.blocks.size() - L.blk0);
         bs.launches.push_back(L);
     }
