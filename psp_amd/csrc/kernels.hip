@@ -2208,8 +2208,10 @@ __global__ __launch_bounds__(256, (BlockOccupancy<T, PH, KB>())) void k_block_ba
     const BatchBlock bb = blocks[blockIdx.x];
     const BlockTile* tp = (const BlockTile*)bb.item;
     const BatchSolveSeg sg = segs[bb.seg];
-    if (!active[bb.problem] || Const(tp)[8] <= 0) return;
-    BlockWork<T, PH, KB>(tp, SegBufs<T>(sg), sg.k, bb.blk, nullptr, nullptr);
+    // (holes of the XCD placement: no tile, or one without output blocks)
+    if (!active[bb.problem] || tp == nullptr || Const(tp)[8] <= 0) return;
+    int32_t* redc = sg.redc == nullptr ? nullptr : sg.redc + bb.blk * sg.nreds;
+    BlockWork<T, PH, KB>(tp, SegBufs<T>(sg), sg.k, bb.blk, redc, sg.reds);
 }
 
 template <typename T, int PH>
@@ -2826,6 +2828,15 @@ static void ProfEnd(MvProfile* prof, hipStream_t s, double bytes, double flops)
     prof->flops += flops;
 }
 
+int32_t* SliceCounters(const ClassDev& c, const ClassPlan& plan, int k, int entryBytes)
+{
+    // the partial sums are read through a buffer of at most 4 GiB, and each
+    // pass needs counters of its own
+    const bool fits = (int64_t)entryBytes * k * 64 * plan.bslots < ((int64_t)1 << 32) &&
+                      k <= kPassRhs * kMaxPasses;
+    return fits ? c.bredc : nullptr;
+}
+
 template <typename T>
 void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, void* P, int k,
                       hipStream_t s, MvProfile* prof, int onlyGroup, int onlyPhase)
@@ -2843,11 +2854,7 @@ void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, 
                             vr.g1,
                             c.xrows,
                             plan.nblocks};
-    // the partial sums are read through a buffer of at most 4 GiB, and each
-    // pass needs counters of its own
-    const bool pfits = (int64_t)sizeof(cx<T>) * k * 64 * plan.bslots < ((int64_t)1 << 32) &&
-                       k <= kPassRhs * kMaxPasses;
-    int32_t* rc = pfits ? c.bredc : nullptr;
+    int32_t* rc = SliceCounters(c, plan, k, sizeof(cx<T>));
     auto go = [&](auto ph, int g) {
         constexpr int PH = decltype(ph)::value;
         const ClassPlan::BlockLevel& L = plan.blevels[g];

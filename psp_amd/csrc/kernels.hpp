@@ -148,7 +148,9 @@ struct BatchSolveSeg {
     void *V, *P;
     const int32_t *bsrc, *blist, *udst;
     int64_t w, g0, g1;       // VecRows
-    int32_t xrows, zero, k;
+    int32_t xrows, zero, k, nreds;
+    int32_t* redc;           // slices summed in the launch: counters (nreds per pass), else null
+    const BlockRed* reds;
 };
 enum BatchCopyOp : int { BATCH_COPY_IN = 0, BATCH_COPY_OUT = 1, BATCH_ZERO_SET_PLANE = 2 };
 constexpr int kBatchCopyThreads = 256;  // elements per workgroup of a batched copy
@@ -196,6 +198,10 @@ struct MvProfile {
     int launches = 0;
     double seconds = 0, bytes = 0, flops = 0;
 };
+
+// The counters with which a class's product launches sum their slices
+// themselves, null if a reduce launch does (after each product launch).
+int32_t* SliceCounters(const ClassDev& c, const ClassPlan& plan, int k, int entryBytes);
 
 // Solve of one panel (batch entry b of class c) on the class's solve vector V
 // (VecRows, k right-hand sides interleaved); P: partial sums (bslots x 64

@@ -1331,6 +1331,9 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             s.xrows = D.xrows;
             s.zero = c->plan.cls[cl].nblocks;
             s.k = k;
+            s.nreds = D.nbreds;
+            s.redc = SliceCounters(D, c->plan.cls[cl], k, (int)eb);
+            s.reds = D.breds;
             bs.solveSegs.push_back(s);
             return (int)bs.solveSegs.size() - 1;
         };
@@ -1349,7 +1352,7 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
                         stages[Key{dir, t, sub, 0, kb}].push_back(
                             Entry{i, seg, (const char*)(D.btiles + lv.start[ph]),
                                   (int)sizeof(BlockTile), lv.count[ph], passes});
-                    if (lv.rcount[ph] > 0)
+                    if (lv.rcount[ph] > 0 && bs.solveSegs[seg].redc == nullptr)
                         stages[Key{dir, t, sub, 1, 0}].push_back(
                             Entry{i, seg, (const char*)(D.breds + lv.rstart[ph]),
                                   (int)sizeof(BlockRed), lv.rcount[ph]});
@@ -1380,16 +1383,20 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
                                : BATCH_COPY_OUT;
         L.kb = key[4];
         L.blk0 = (int64_t)bs.blocks.size();
+        // Workgroup i runs on XCD i % 8 and a tile's slices are 8 apart in its
+        // list: a list's passes take turns every 8 workgroups (with several,
+        // filled up by holes), so that the slices of a pass stay 8 apart.
         for (const Entry& e : kv.second)
-            for (int j = 0; j < e.count; ++j)
-                for (int p = 0; p < e.passes; ++p) {
-                    BatchBlock b{};
-                    b.item = copy ? nullptr : e.items + (size_t)j * e.stride;
-                    b.seg = e.seg;
-                    b.problem = e.problem;
-                    b.blk = copy ? j : p;
-                    bs.blocks.push_back(b);
-                }
+            for (int j0 = 0; j0 < e.count; j0 += 8)
+                for (int p = 0; p < e.passes; ++p)
+                    for (int j = j0; j < j0 + 8 && (j < e.count || e.passes > 1); ++j) {
+                        BatchBlock b{};
+                        b.item = copy || j >= e.count ? nullptr : e.items + (size_t)j * e.stride;
+                        b.seg = e.seg;
+                        b.problem = e.problem;
+                        b.blk = copy ? j : p;
+                        bs.blocks.push_back(b);
+                    }
         L.nblocks = (int)((int64_t)bs.blocks.size() - L.blk0);
         bs.launches.push_back(L);
     }

@@ -31,3 +31,23 @@ def test_passes_match_oracle(torch_cuda, k, tiling):
         h.Precondition(xd)
         torch.cuda.synchronize()
         assert _rel(xd.cpu().numpy()[l2n], ref) < tol
+
+
+@pytest.mark.parametrize("off", [(), (1,), (0, 1, 2)])
+def test_merged_batch_of_sliced_passes(torch_cuda, off):
+    # sliced tiles of one and several passes in merged launches, members `off`
+    # with their sums in a reduce launch: each equals its own solve
+    import psp_amd
+    from test_gpu_batch_merged import _alone, _batch, _sources
+    torch = torch_cuda
+    helms, Bs = [], []
+    for j, (nx, ny, nz, k) in enumerate([(15, 13, 24, 70), (16, 14, 22, 33), (12, 11, 26, 5)]):
+        disc, vel = _problem(nx, ny, nz)
+        h = psp_amd.DistHelmholtz(disc)
+        h.set_solve_tiling(min_tiles=4096, max_split=16, xcd_reduce=0 if j in off else 1)
+        h.Initialize(vel)
+        helms.append(h)
+        Bs.append(_sources(nx, ny, nz, k, 170 + j))
+    ref = [_alone(torch, h, B, 1e-9) for h, B in zip(helms, Bs)]
+    for (x, r), (xr, rr) in zip(zip(*_batch(torch, helms, Bs, 1e-9)), ref):
+        assert r.iterations == rr.iterations and torch.equal(x, xr)
