@@ -2450,33 +2450,73 @@ __device__ __forceinline__ void ZeroSetPlaneElem(int64_t e, int n, int k, const 
 // --------------------------------------------------------------------------
 // Multiply (solve.hpp:613-679) in natural order: y = A x or y = b - A x.
 // --------------------------------------------------------------------------
-// I: index type, uint32_t when every element index (and the grid's last
-// thread) fits, which keeps the index divisions 32-bit; int64_t otherwise.
-template <typename I>
+// Bound by memory: a block is read and written once if its neighbours in y and
+// z are found in L2.  Workgroups in the order of memory go to the 8 XCDs in turn,
+// so each XCD's L2 fetched the lines of its neighbours too.  Order of the work
+// here: strips of `rows` lines of y, in each all planes z, so that a plane of a
+// strip, read as z + 1, is still in L2 as z and z - 1; workgroup b takes place
+// b / 8 in the part b % 8 of that order, so an XCD has its own part.
+// kStripBytes: 128 KiB, 256 KiB and no strips were up to 7, 4 and 13% slower.  us
+// a call on blocks that no cache holds, before and after: 100^3 k = 8 137 -> 129,
+// k = 64 915 -> 745; 144 x 128 x 80 k = 16 355 -> 308; 120 x 96 x 60 k = 32
+// 336 -> 276; 61 x 47 x 83 k = 5 38.6 -> 36.5.  Now the L1s' loads bound it (seven
+// of 16 bytes for each 32 moved).
+struct SpmvOrder {
+    int rows, strips, per;   // lines per strip, strips, workgroups per strip plane
+    int64_t part;            // workgroups per part
+};
+constexpr int kStripBytes = 512 << 10;
+constexpr unsigned kSpmvGrid = 1u << 22;  // most workgroups of a launch (more: several turns)
+
+// V: right-hand sides of a point per thread (V divides k), which share its
+// stencil row (four needed more registers: 15% slower than two).
+// LOOP: more workgroups than a launch takes.
+template <int V, bool LOOP>
 __global__ __launch_bounds__(kThreads) void k_spmv(StencilArgs st, const double* vel,
                                                     const c128* X, const c128* Bv, c128* Y, int k,
-                                                    int mode)
+                                                    int mode, SpmvOrder o)
 {
-    const I e = (I)blockIdx.x * (I)blockDim.x + (I)threadIdx.x;
-    const I nx = (I)st.nx, ny = (I)st.ny, kk = (I)k;
-    const I plane = nx * ny;
-    if (e >= plane * (I)st.nz * kk) return;
-    const I p = e / kk;
-    const I py = p / nx;
-    const int x = (int)(p - py * nx);
-    const int y = (int)(py % ny);
-    const int z = (int)(py / ny);
-    const int v = st.nz - 1 - z;
-    c128 c[7];
-    GlobalRowFast(st, vel[p], x, y, v, c);
-    c128 acc = X[e] * c[0];
-    if (x > 0) acc = cfma(c[1], X[e - kk], acc);
-    if (x + 1 < st.nx) acc = cfma(c[2], X[e + kk], acc);
-    if (y > 0) acc = cfma(c[3], X[e - nx * kk], acc);
-    if (y + 1 < st.ny) acc = cfma(c[4], X[e + nx * kk], acc);
-    if (v > 0) acc = cfma(c[5], X[e + plane * kk], acc);
-    if (v + 1 < st.nz) acc = cfma(c[6], X[e - plane * kk], acc);
-    Y[e] = mode == 0 ? acc : (Bv[e] - acc);
+    for (int64_t i = blockIdx.x >> 3; LOOP ? i < o.part : true; i += gridDim.x >> 3) {
+        const int64_t g = (int64_t)(blockIdx.x & 7) * o.part + i;
+        const int64_t sp = g / o.per;
+        const int strip = (int)(sp / st.nz), z = (int)(sp - (int64_t)strip * st.nz);
+        if (strip >= o.strips) return;
+        const int y0 = strip * o.rows, rows = min(o.rows, st.ny - y0);
+        const uint32_t nx = st.nx, kk = k / V;
+        const uint32_t t = (uint32_t)(g - sp * o.per) * kThreads + threadIdx.x;
+        if (t >= rows * nx * kk) {
+            if (LOOP) continue;
+            return;
+        }
+        const uint32_t q = t / kk, r = (t - q * kk) * V, yl = q / nx;
+        const int x = (int)(q - yl * nx), y = y0 + (int)yl, v = st.nz - 1 - z;
+        const int64_t p = ((int64_t)z * st.ny + y0) * nx + q;
+        const int64_t line = (int64_t)st.nx * k, plane = line * st.ny;
+        const c128* Xe = X + p * k + r;
+        c128 c[7];
+        GlobalRowFast(st, vel[p], x, y, v, c);
+        c128 acc[V];
+        auto term = [&](bool on, int64_t d, int j) {
+            if (on) {
+#pragma unroll
+                for (int n = 0; n < V; ++n) acc[n] = cfma(c[j], Xe[d + n], acc[n]);
+            }
+        };
+#pragma unroll
+        for (int n = 0; n < V; ++n) acc[n] = Xe[n] * c[0];
+        term(x > 0, -k, 1);
+        term(x + 1 < st.nx, k, 2);
+        term(y > 0, -line, 3);
+        term(y + 1 < st.ny, line, 4);
+        term(v > 0, plane, 5);
+        term(v + 1 < st.nz, -plane, 6);
+#pragma unroll
+        for (int n = 0; n < V; ++n) {
+            const int64_t e = p * k + r + n;
+            Y[e] = mode == 0 ? acc[n] : (Bv[e] - acc[n]);
+        }
+        if (!LOOP) return;
+    }
 }
 
 // dL/dm_i = sum_s Re(omega^2 s1 s2 s3 lambda_s(i) u_s(i)).
@@ -3086,13 +3126,26 @@ void LaunchCopyBatch(int op, const BatchBlock* blocks, int nblocks, const BatchC
 void LaunchSpmv(const StencilArgs& st, const double* vel, const c128* x, const c128* b, c128* y,
                 int k, int mode, hipStream_t s)
 {
-    const int64_t n = (int64_t)st.nx * st.ny * st.nz * k;
-    if ((int64_t)Blocks(n) * kThreads <= (int64_t)UINT32_MAX)
-        hipLaunchKernelGGL((k_spmv<uint32_t>), dim3(Blocks(n)), dim3(kThreads), 0, s, st, vel, x,
-                           b, y, k, mode);
+    auto run = [&](auto vc) {
+        constexpr int V = decltype(vc)::value;
+        SpmvOrder o;
+        const int64_t line = (int64_t)st.nx * k * (int64_t)sizeof(c128);
+        o.rows = (int)std::min<int64_t>(st.ny, std::max<int64_t>(1, kStripBytes / line));
+        o.strips = (st.ny + o.rows - 1) / o.rows;
+        o.per = (int)Blocks((int64_t)o.rows * st.nx * (k / V));
+        o.part = ((int64_t)o.strips * st.nz * o.per + 7) / 8;
+        const unsigned grid = (unsigned)std::min<int64_t>(8 * o.part, kSpmvGrid);
+        if (8 * o.part <= kSpmvGrid)
+            hipLaunchKernelGGL((k_spmv<V, false>), dim3(grid), dim3(kThreads), 0, s, st, vel, x, b,
+                               y, k, mode, o);
+        else
+            hipLaunchKernelGGL((k_spmv<V, true>), dim3(grid), dim3(kThreads), 0, s, st, vel, x, b,
+                               y, k, mode, o);
+    };
+    if (k % 2 == 0)
+        run(std::integral_constant<int, 2>());
     else
-        hipLaunchKernelGGL((k_spmv<int64_t>), dim3(Blocks(n)), dim3(kThreads), 0, s, st, vel, x, b,
-                           y, k, mode);
+        run(std::integral_constant<int, 1>());
 }
 
 int ReducePartials(int64_t npoints)
