@@ -77,7 +77,6 @@ struct ClassDev {
     int32_t* redc = nullptr;        // redcBuf when split row blocks are summed in the launch
     TransItem* trans = nullptr;     // LT[:, :s] blocks
     TransItem* foldBack = nullptr;  // L_BL / diagonal blocks
-    int32_t* ginv = nullptr;
     int ninv = 0, ntrans = 0, nfold = 0;
     int32_t* panelVOff = nullptr;   // per batch entry: panel vOffset
     c128* s3art = nullptr;          // per batch entry: vsize + 2 profile values

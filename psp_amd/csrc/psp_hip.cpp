@@ -392,7 +392,7 @@ int EnsureDevice(psp_hip_ctx* c)
             (st = Upload(c, &D.foldNodes, P.foldNodes)) || (st = Upload(c, &D.packs, P.packs)) ||
             (st = Upload(c, &D.compose, P.compose)) || (st = Upload(c, &D.fkeys, P.fkeys)) ||
             (st = Upload(c, &D.composeTiles, P.composeTiles)) ||
-            (st = Upload(c, &D.trans, P.trans)) || (st = Upload(c, &D.ginv, P.ginv)) ||
+            (st = Upload(c, &D.trans, P.trans)) ||
             (st = Upload(c, &D.foldBack, P.foldBack)) ||
             (st = Upload(c, &D.panelVOff, vOff)))
             return st;

@@ -6,7 +6,9 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <future>
 #include <stack>
+#include <system_error>
 
 namespace psp_amd {
 
@@ -241,10 +243,14 @@ void AssemblyMeta(const Geometry& g, ClassPlan& C)
     C.qnode.assign(n, -1);
     C.qcol.assign(n, 0);
     C.qrows.assign((size_t)n * 6, -1);
+    std::vector<int> index(n);  // (x, y, v), x fastest
+    auto at = [&](int x, int y, int v) -> int& {
+        return index[x + (size_t)nx * (y + (size_t)ny * v)];
+    };
     for (int v = 0; v < vs; ++v)
         for (int y = 0; y < ny; ++y)
             for (int x = 0; x < nx; ++x) {
-                const int q = NestedIndex(x, y, v, nx, ny, vs, cut);
+                const int q = at(x, y, v) = NestedIndex(x, y, v, nx, ny, vs, cut);
                 C.qxy[q] = x | (y << 16);
                 C.qv[q] = v;
             }
@@ -266,7 +272,7 @@ void AssemblyMeta(const Geometry& g, ClassPlan& C)
             if (nbx[e] < 0 || nbx[e] >= nx || nby[e] < 0 || nby[e] >= ny || nbv[e] < 0 ||
                 nbv[e] >= vs)
                 continue;
-            const int ni = NestedIndex(nbx[e], nby[e], nbv[e], nx, ny, vs, cut);
+            const int ni = at(nbx[e], nby[e], nbv[e]);
             if (ni <= q) continue;
             int row;
             if (ni < nd.off + nd.size) {
@@ -546,16 +552,6 @@ void Schedule(const Plan& plan, ClassPlan& C)
 
     // Solve schedule.
     {
-        C.ginv.assign((size_t)2 * C.wstore, -1);
-        for (const Node& n : C.nodes)
-            for (int k = 0; k < 2; ++k) {
-                if (n.child[k] < 0) continue;
-                const Node& ch = C.nodes[n.child[k]];
-                for (int a = 0; a < ch.usize; ++a) {
-                    const int r = C.relinds[ch.ustart + a];
-                    C.ginv[(size_t)2 * (n.woff + r) + k] = (int32_t)(ch.woff + ch.size + a);
-                }
-            }
         DefaultSolveShapes(C, plan.minTiles, plan.maxSplit, plan.wideWg, plan.persist);
         BuildSolveTiles(C);
         BuildQueues(C, plan.fused ? plan.fusedQueues : 0, plan.fusedRows, plan.fusedCut,
@@ -1433,8 +1429,15 @@ int BuildPlan(const psp_hip_desc& d, Plan& plan, std::string& msg)
         msg = "The domain is very shallow. Please run a sparse-direct factorization instead.";
         return st;
     }
-    for (int c = 0; c < 3; ++c) {
-        if (c == 1 && !plan.geo.haveLeftover) continue;
+    // The classes' plans are independent and take tens of ms each at 100^3: one
+    // thread a class, the largest (2) on this one.
+    struct Result {
+        int st = PSP_HIP_OK;
+        std::string msg;
+    };
+    auto build = [&](int c) -> Result {
+        Result res;
+        res.st = PSP_HIP_ERR_INVALID;
         ClassPlan& C = plan.cls[c];
         C.cls = c;
         C.vsize = plan.geo.classVSize(c);
@@ -1446,8 +1449,8 @@ int BuildPlan(const psp_hip_desc& d, Plan& plan, std::string& msg)
         Schedule(plan, C);
         BuildMerged(C, d.precision == PSP_HIP_FRONTS_FP32 ? 8 : 16);
         if (C.bnodes.empty()) {
-            msg = "internal error: inconsistent merged fronts";
-            return PSP_HIP_ERR_INVALID;
+            res.msg = "internal error: inconsistent merged fronts";
+            return res;
         }
         DefaultSlices(C, plan.minTiles, plan.maxSplit);
         BuildBlockTiles(C);
@@ -1457,16 +1460,41 @@ int BuildPlan(const psp_hip_desc& d, Plan& plan, std::string& msg)
                 const int64_t e = n.ustart + a;
                 if (C.structs[e] < 0 || C.structs[e] >= C.n ||
                     (n.parent >= 0 && C.relinds[e] < 0)) {
-                    msg = "internal error: inconsistent front structure";
-                    return PSP_HIP_ERR_INVALID;
+                    res.msg = "internal error: inconsistent front structure";
+                    return res;
                 }
             }
         for (int q = 0; q < C.n; ++q)
             if (C.qnode[q] < 0) {
-                msg = "internal error: unknown without a front";
-                return PSP_HIP_ERR_INVALID;
+                res.msg = "internal error: unknown without a front";
+                return res;
             }
         plan.present[c] = true;
+        res.st = PSP_HIP_OK;
+        return res;
+    };
+    std::future<Result> other[2];
+    bool here[2] = {false, false};
+    for (int c = 0; c < 2; ++c) {
+        if (c == 1 && !plan.geo.haveLeftover) continue;
+        try {
+            other[c] = std::async(std::launch::async, build, c);
+        } catch (const std::system_error&) {  // no thread to be had
+            here[c] = true;
+        }
+    }
+    const Result last = build(2);
+    for (int c = 0; c < 2; ++c) {
+        if (!other[c].valid() && !here[c]) continue;
+        const Result r = here[c] ? build(c) : other[c].get();
+        if (r.st != PSP_HIP_OK) {
+            msg = r.msg;
+            return r.st;
+        }
+    }
+    if (last.st != PSP_HIP_OK) {
+        msg = last.msg;
+        return last.st;
     }
     return PSP_HIP_OK;
 }

@@ -289,8 +289,6 @@ struct ClassPlan {
 
     // Solve schedule.  Per depth: forward product (F) and backward product
     // (B).
-    // ginv[2*r + c]: row of child c's work vector feeding front row r (or -1).
-    std::vector<int32_t> ginv;
     std::vector<MvTile> mv;
     std::vector<MvTile> mvred;  // reduce items of split row blocks
     int maxSlots = 0;           // partial slots of the largest (level, phase)
