@@ -2403,6 +2403,95 @@ __global__ __launch_bounds__(kThreads) void k_zero_set_plane(int n, int k, const
     ZeroSetPlaneElem<T>(e, n, k, qxy, qv, st, vel, B, Xp, v2, vlLast);
 }
 
+// A panel's copy out, with its coupling, and the next panel's copy in as one
+// launch: both are small (5 us each, mostly latency, and a sweep of P panels had
+// 4 P - 2 of them; now 2 P), and a value that couples stays in a register.  A
+// thread owns a column (x, y, r) of both panels, so it has read every row of the
+// old vector that it writes in the new one.  The arithmetic is CopyOutElem's,
+// CopyInElem's and ZeroSetPlaneElem's.  Bound by its chain of loads (6 us at 24 x
+// 20, k = 3), so the first U planes of both panels are loaded together.  ms a
+// sweep, before and after: 100^3 k = 8 FP32 8.87 -> 8.68, k = 16 11.26 -> 10.9,
+// k = 64 28.4 -> 27.6; 120 x 96 x 60 k = 32 FP32 11.4 -> 11.15; 24 x 20 x 26 and
+// 40^3 as before.
+template <typename T, int U>
+__global__ __launch_bounds__(kThreads) void k_pass_on(StencilArgs st, const double* vel, c128* B,
+                                                       int k, PassPanel o, PassPanel i, int mode,
+                                                       int dir)
+{
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t plane = (int64_t)st.nx * st.ny;
+    if (e >= plane * k) return;
+    const int xy = (int)(e / k), r = (int)(e - (int64_t)xy * k);
+    const int y = xy / st.nx, x = xy - y * st.nx;
+    // grid point of (x, y) on plane vl of a panel
+    auto at = [&](const PassPanel& p, int vl) {
+        return xy + plane * (st.nz - 1 - (p.vOffset + vl));
+    };
+    const cx<T>* Xo = (const cx<T>*)o.X;
+    cx<T>* Xi = (cx<T>*)i.X;
+    const int edgeIn = dir == 0 ? 0 : i.depth - 1;
+    const double velIn = vel[at(i, i.padding + edgeIn)];
+    int32_t ro[U], ri[U];
+    cx<T> v[U];
+    c128 bo[U], bi[U];
+    auto rows = [&](const PassPanel& p, int j0, int32_t (&row)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            row[u] = p.row[(p.padding + min(j0 + u, p.depth - 1)) * plane + xy];
+    };
+    auto outs = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u] = Xo[(int64_t)ro[u] * k + r];
+            if (mode != 0) bo[u] = B[at(o, o.padding + min(j0 + u, o.depth - 1)) * k + r];
+        }
+    };
+    auto ins = [&](int j0) {
+        if (dir == 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                bi[u] = B[at(i, i.padding + min(j0 + u, i.depth - 1)) * k + r];
+        }
+    };
+    rows(o, 0, ro);
+    rows(i, 0, ri);
+    ins(0);
+    outs(0);
+    const int edgeOut = dir == 0 ? o.depth - 1 : 0;  // the plane that couples
+    c128 ev{0.0, 0.0};
+    for (int j0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + u >= o.depth) break;
+            const c128 w = cvt<double>(v[u]);
+            const c128 out = mode == 0 ? w : bo[u] + w;
+            B[at(o, o.padding + j0 + u) * k + r] = out;
+            if (j0 + u == edgeOut) ev = out;
+        }
+        if ((j0 += U) >= o.depth) break;
+        rows(o, j0, ro);
+        outs(j0);
+    }
+    for (int vl = 0; vl < i.padding; ++vl)
+        Xi[(int64_t)i.row[vl * plane + xy] * k + r] = czero<T>();
+    // row (x, y, v) couples to the plane below with c[5], above with c[6]
+    c128 c[7];
+    GlobalRowFast(st, velIn, x, y, i.vOffset + i.padding + edgeIn, c);
+    for (int j0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + u;
+            if (j >= i.depth) break;
+            c128 in = dir == 0 ? bi[u] : c128{0.0, 0.0};
+            if (j == edgeIn) in = dir == 0 ? in - c[5] * ev : -(c[6] * ev);
+            Xi[(int64_t)ri[u] * k + r] = cvt<T>(in);
+        }
+        if ((j0 += U) >= i.depth) break;
+        rows(i, j0, ri);
+        ins(j0);
+    }
+}
+
 // One batched panel copy: op BATCH_COPY_IN, BATCH_COPY_OUT (mode and
 // coupling plane v1 per segment) or BATCH_ZERO_SET_PLANE, with the segment's
 // elements split into whole workgroups (BatchBlock.item unused, blk: the
@@ -3068,6 +3157,21 @@ void LaunchCopyOut(const PanelMap& m, c128* B, const void* Xp, int k, int nx, in
 }
 
 template <typename T>
+void LaunchPassOn(const StencilArgs& st, const double* vel, c128* B, int k, const PassPanel& o,
+                  const PassPanel& i, int mode, int dir, hipStream_t s)
+{
+    // few columns: small workgroups, so that they are on more CUs, and more
+    // loads at a time
+    const int64_t n = (int64_t)st.nx * st.ny * k;
+    if (n < 256 * kThreads)
+        hipLaunchKernelGGL((k_pass_on<T, 8>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, st,
+                           vel, B, k, o, i, mode, dir);
+    else
+        hipLaunchKernelGGL((k_pass_on<T, 4>), dim3(Blocks(n)), dim3(kThreads), 0, s, st, vel, B, k,
+                           o, i, mode, dir);
+}
+
+template <typename T>
 void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* vel,
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,
                         int32_t* sync, int nsync)
@@ -3234,6 +3338,8 @@ void LaunchAdjointGrad(const StencilArgs& st, const c128* u, const c128* lam, in
     template void LaunchCopyOut<T>(const PanelMap&, c128*, const void*, int, int, int, int, int,  \
                                    int, int, hipStream_t, const StencilArgs*, const double*,      \
                                    int);                                                          \
+    template void LaunchPassOn<T>(const StencilArgs&, const double*, c128*, int,                  \
+                                  const PassPanel&, const PassPanel&, int, int, hipStream_t);     \
     template void LaunchZeroSetPlane<T>(const PanelMap&, const StencilArgs&, const double*,       \
                                         const c128*, void*, int, int, int, hipStream_t, int32_t*, \
                                         int);                                                     \

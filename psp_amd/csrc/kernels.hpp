@@ -104,7 +104,7 @@ struct ClassDev {
     int32_t* bredc = nullptr;       // bredcBuf when slices are summed in the launch
     int nbreds = 0;
     int32_t *blist = nullptr, *bsrc = nullptr, *udst = nullptr;
-    int32_t *sxy = nullptr, *sv = nullptr;
+    int32_t *sxy = nullptr, *sv = nullptr, *srow = nullptr;
     int32_t xrows = 0;
     int64_t fentries = 0;           // entries of one panel's F
     void* F = nullptr;              // npanels * fentries
@@ -240,6 +240,21 @@ void LaunchCopyOut(const PanelMap& m, c128* B, const void* Xp, int k, int nx, in
                    const StencilArgs* st = nullptr, const double* vel = nullptr, int v1 = -1);
 // Backward sweep, one pass: Xp = 0 except the superdiagonal coupling on the
 // panel's last local plane (MultiplySuperdiagonal, solve.hpp:725-733).
+// A panel's vector X in a pass from panel to panel: row[(v ny + y) nx + x] is
+// its row of (x, y, v), planes [padding, padding + depth) are the panel's own.
+struct PassPanel {
+    const int32_t* row;
+    void* X;
+    int vOffset, padding, depth;
+};
+// The copy out of panel o (mode 0 stores, 1 adds) and the copy in of panel i: dir
+// 0, i is the panel above o, copied with o's subdiagonal coupling; dir 1, i is the
+// panel below o, zero but for the superdiagonal coupling.  The vectors may share
+// their memory.
+template <typename T>
+void LaunchPassOn(const StencilArgs& st, const double* vel, c128* B, int k, const PassPanel& o,
+                  const PassPanel& i, int mode, int dir, hipStream_t s);
+
 template <typename T>
 void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* vel,
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,

@@ -368,6 +368,11 @@ int EnsureDevice(psp_hip_ctx* c)
             const int x = P.qxy[q] & 0xffff, y = P.qxy[q] >> 16;
             nat2q[x + y * d.nx + P.qv[q] * d.nx * d.ny] = q;
         }
+        // panel-vector row of (x, y, v)
+        std::vector<int32_t> srow(P.n);
+        for (int q = 0; q < P.xrows; ++q)
+            if (P.sv[q] >= 0)
+                srow[(P.sxy[q] & 0xffff) + (size_t)d.nx * ((P.sxy[q] >> 16) + (size_t)d.ny * P.sv[q])] = q;
         std::vector<int32_t> vOff(D.npanels);
         std::vector<zd> s3a((size_t)D.npanels * (P.vsize + 2));
         for (int b = 0; b < D.npanels; ++b) {
@@ -387,6 +392,7 @@ int EnsureDevice(psp_hip_ctx* c)
             (st = Upload(c, &D.ldl, P.ldl)) || (st = Upload(c, &D.gemms, P.gemms)) ||
             (st = Upload(c, &D.tiles, P.tiles)) || (st = Upload(c, &D.inv, P.inv)) ||
             (st = Upload(c, &D.sxy, P.sxy)) || (st = Upload(c, &D.sv, P.sv)) ||
+            (st = Upload(c, &D.srow, srow)) ||
             (st = Upload(c, &D.browBase, P.browBase)) || (st = Upload(c, &D.udst, P.udst)) ||
             (st = Upload(c, &D.flist, P.flist)) || (st = Upload(c, &D.fsrc, P.fsrc)) ||
             (st = Upload(c, &D.foldNodes, P.foldNodes)) || (st = Upload(c, &D.packs, P.packs)) ||
@@ -912,9 +918,38 @@ template <typename T>
 void Sweep(psp_hip_ctx* c, c128* B, int k, MvProfile* prof = nullptr)
 {
     const Geometry& g = c->plan.geo;
-    for (int i = 0; i < g.numPanels - 1; ++i) PanelForward<T>(c, B, k, i, prof, g.panelV(i + 1));
-    PanelForward<T>(c, B, k, g.numPanels - 1, prof);
-    for (int i = g.numPanels - 2; i >= 0; --i) PanelBackward<T>(c, B, k, i, prof);
+    bool fused = false;
+    for (int cl = 0; cl < 3; ++cl)
+        if (c->plan.present[cl]) fused = fused || PanelSolver<T>(c, cl, k).fused;
+    if (fused) {
+        for (int i = 0; i < g.numPanels - 1; ++i)
+            PanelForward<T>(c, B, k, i, prof, g.panelV(i + 1));
+        PanelForward<T>(c, B, k, g.numPanels - 1, prof);
+        for (int i = g.numPanels - 2; i >= 0; --i) PanelBackward<T>(c, B, k, i, prof);
+        return;
+    }
+    // PanelForward and PanelBackward of all panels, a panel's copy out and the
+    // next one's copy in as one launch
+    const int last = g.numPanels - 1;
+    const StencilArgs st = Stencil(c);
+    auto panel = [&](int p) {
+        const int cl = g.cls(p);
+        return PassPanel{c->dev[cl].srow, c->vec[cl], g.vOffset(p), g.padding(p), g.depth(p)};
+    };
+    auto solve = [&](int p) { PanelSolver<T>(c, g.cls(p), k).Solve(c->panelBatch[p], prof); };
+    const PanelSolver<T> first(c, g.cls(0), k);
+    LaunchCopyIn<T>(first.map, B, first.x, k, g.nx, g.ny, g.nz, g.vOffset(0), g.padding(0),
+                    c->stream);
+    for (int i = 0; i <= last; ++i) {
+        solve(i);
+        if (i < last) LaunchPassOn<T>(st, c->vel, B, k, panel(i), panel(i + 1), 0, 0, c->stream);
+    }
+    for (int i = last - 1; i >= 0; --i) {
+        LaunchPassOn<T>(st, c->vel, B, k, panel(i + 1), panel(i), i + 1 < last, 1, c->stream);
+        solve(i);
+    }
+    LaunchCopyOut<T>(first.map, B, first.x, k, g.nx, g.ny, g.nz, g.vOffset(0), g.padding(0),
+                     last > 0, c->stream);
 }
 
 void SweepEager(psp_hip_ctx* c, c128* B, int k)
