@@ -29,7 +29,7 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-TRAFFIC_PROFILE = "k_mvp_k_mvm_front_solves_bumps100_8rhs.md"
+TRAFFIC_PROFILE = "k_block_front_solves_bumps100_8rhs.md"
 
 
 def measured_traffic():
@@ -436,7 +436,7 @@ def main():
     # the sweep from a hipGraph, whose kernels cannot be bracketed singly).
     launches, ksec, kbytes, kflops = h32.ProfileSweep(Bsrc.clone())
     achieved = kbytes / ksec / 1e9
-    kname = ("k_mvp/k_mvm" if k <= 16 else "k_mvm") if 8 <= k < 32 else ("k_mmw" if k >= 32 else "k_mv")
+    kname = "k_mvq, k_mvm" if args.fused and 8 <= k <= 16 else "k_block"
     traffic = measured_traffic() if (k == 8 and args.workload == "bumps100") else None
     roofline = {"bound": "hbm", "achieved": achieved, "peak": 8000.0, "unit": "GB/s",
                 "frac": achieved / 8000.0,
@@ -524,7 +524,8 @@ def main():
         "config": {"workload": wl.name, "grid": [disc.nx, disc.ny, disc.nz], "rhs": k,
                    "gmres_m": args.m, "rel_tol": args.tol, "omega": disc.omega,
                    "sigma": disc.sigmax, "max_its": args.max_its,
-                   "sweep_launches": "fused below the cut" if args.fused else "one per level"},
+                   "sweep_launches": "fused below the cut" if args.fused else
+                                     "one per group of tree depths"},
         "status": "ok" if value is not None else
                   "not converged: value is null (a timed solve ended above rel_tol)",
         "roofline": roofline,
