@@ -2769,6 +2769,149 @@ __global__ __launch_bounds__(kThreads) void k_coldot_final(const c128* part, int
     if (threadIdx.x == 0) out[r] = sh[0];
 }
 
+// Modified Gram-Schmidt with two passes over the basis.  Step by step it is
+// h_a = v_a^H (w - sum_{b<a} h_b v_b) = d_a - sum_{b<a} (v_a^H v_b) h_b, so all
+// d_a = v_a^H w and the Gram row v_a^H v_j of the newest vector come from one
+// pass (k_arnoldi_dots), h from a triangular solve with the Gram rows of the
+// cycle (k_arnoldi_solve), and w - V h with its norm from a second pass
+// (k_arnoldi_update): 2.25 j vectors moved instead of 4 j, 4 launches instead of
+// 2 j + 4.  The rounding error is that of the steps one by one.  Bound by memory
+// for wide blocks.  ms a solve, before and after: 120 x 96 x 60 k = 32 501 -> 465,
+// 44 x 36 x 48 k = 16 with its adjoint 141 -> 137, 61 x 47 x 83 k = 5 57.4 -> 56.8,
+// 40^3 k = 1 19.9 -> 19.5.  Cycles past 64 (the solve is one wave) go step by step.
+constexpr int kDotGroup = 8;  // basis vectors per workgroup (16 sums in registers)
+
+// Block partials of group blockIdx.y: part[(q grid.x + block) k + r], q = i for
+// v_i^H w and j + 1 + i for v_i^H v_j.
+__global__ __launch_bounds__(kThreads) void k_arnoldi_dots(const c128* __restrict__ V, int64_t n,
+                                                            int j, const c128* __restrict__ W,
+                                                            int64_t np, int k,
+                                                            c128* __restrict__ part)
+{
+    __shared__ c128 sh[kThreads];
+    const int lanes = (kThreads / k) * k, per = kThreads / k;
+    const int t = threadIdx.x, i0 = blockIdx.y * kDotGroup, cnt = min(kDotGroup, j + 1 - i0);
+    const int64_t chunk = (np + gridDim.x - 1) / gridDim.x;
+    const int64_t p0 = (int64_t)blockIdx.x * chunk, p1 = min(np, p0 + chunk);
+    const c128 *Vi = V + i0 * n, *Vj = V + j * n;
+    c128 acc[2 * kDotGroup];
+#pragma unroll
+    for (int u = 0; u < 2 * kDotGroup; ++u) acc[u] = c128{0.0, 0.0};
+    auto add = [](c128& s, const c128& v, const c128& w) {  // s += conj(v) w
+        s.r = fma(v.r, w.r, s.r);
+        s.r = fma(v.i, w.i, s.r);
+        s.i = fma(v.r, w.i, s.i);
+        s.i = fma(-v.i, w.r, s.i);
+    };
+    if (t < lanes) {
+        const int r = t % k;
+        for (int64_t p = p0 + t / k; p < p1; p += per) {
+            const int64_t e = p * k + r;
+            const c128 w = W[e], vj = Vj[e];
+            c128 v[kDotGroup];
+#pragma unroll
+            for (int u = 0; u < kDotGroup; ++u)
+                if (u < cnt) v[u] = Vi[u * n + e];
+#pragma unroll
+            for (int u = 0; u < kDotGroup; ++u)
+                if (u < cnt) {
+                    add(acc[2 * u], v[u], w);
+                    add(acc[2 * u + 1], v[u], vj);
+                }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2 * kDotGroup; ++u) {
+        if (u / 2 >= cnt) break;
+        sh[t] = acc[u];
+        __syncthreads();
+        if (t < k) {
+            c128 s = {0.0, 0.0};
+            for (int q = 0; q < per; ++q) s = s + sh[t + q * k];
+            const int64_t q = (u & 1) * (j + 1) + i0 + u / 2;
+            part[(q * gridDim.x + blockIdx.x) * k + t] = s;
+        }
+        __syncthreads();
+    }
+}
+
+// Column r = blockIdx.x: sums the partials (a wave per sum, in a fixed order),
+// stores the Gram row j, gram[(j m + i) k + r] = v_j^H v_i, and solves for h.
+constexpr int kSolveThreads = 512, kMaxGram = 64;  // the longest cycle this form takes
+__global__ __launch_bounds__(kSolveThreads) void k_arnoldi_solve(const c128* part, int nblk, int j,
+                                                                  int m, int k, c128* gram, c128* h)
+{
+    __shared__ c128 d[kMaxGram], row[kMaxGram];
+    const int r = blockIdx.x, lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < 2 * (j + 1); q += kSolveThreads / 64) {
+        c128 s = {0.0, 0.0};
+        for (int b = lane; b < nblk; b += 64) s = s + part[((int64_t)q * nblk + b) * k + r];
+        for (int o = 32; o > 0; o >>= 1) {
+            s.r += __shfl_xor(s.r, o, 64);
+            s.i += __shfl_xor(s.i, o, 64);
+        }
+        if (lane == 0) {
+            if (q <= j)
+                d[q] = s;
+            else
+                row[q - j - 1] = c128{s.r, -s.i};  // v_j^H v_i
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    // one wave: lane a holds row a (j < kMaxGram = 64)
+    if (lane < j) gram[((int64_t)j * m + lane) * k + r] = row[lane];
+    c128 da = lane <= j ? d[lane] : c128{0.0, 0.0};
+    for (int b = 0; b < j; ++b) {
+        const c128 hb{__shfl(da.r, b, 64), __shfl(da.i, b, 64)};
+        if (lane > b && lane <= j) {
+            const c128 g = lane == j ? row[b] : gram[((int64_t)lane * m + b) * k + r];
+            da = cfms(g, hb, da);
+        }
+    }
+    if (lane <= j) h[lane * k + r] = da;
+}
+
+// W -= V h, and the partial sums of its norms (k_colnorm_part's partition).
+__global__ __launch_bounds__(kThreads) void k_arnoldi_update(const c128* __restrict__ V, int64_t n,
+                                                              int j, const c128* __restrict__ h,
+                                                              c128* __restrict__ W, int64_t np,
+                                                              int k, double* __restrict__ part)
+{
+    __shared__ double sh[kThreads];
+    const int lanes = (kThreads / k) * k, per = kThreads / k;
+    const int t = threadIdx.x;
+    const int64_t chunk = (np + gridDim.x - 1) / gridDim.x;
+    const int64_t p0 = (int64_t)blockIdx.x * chunk, p1 = min(np, p0 + chunk);
+    double acc = 0.0;
+    if (t < lanes) {
+        const int r = t % k;
+        for (int64_t p = p0 + t / k; p < p1; p += per) {
+            const int64_t e = p * k + r;
+            c128 w = W[e];
+            int i = 0;
+            for (; i + 4 <= j + 1; i += 4) {
+                c128 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = V[(i + u) * n + e];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w = cfms(h[(i + u) * k + r], v[u], w);
+            }
+            for (; i <= j; ++i) w = cfms(h[i * k + r], V[i * n + e], w);
+            W[e] = w;
+            acc = fma(w.r, w.r, acc);
+            acc = fma(w.i, w.i, acc);
+        }
+    }
+    sh[t] = acc;
+    __syncthreads();
+    if (t < k) {
+        double s = 0.0;
+        for (int i = 0; i < per; ++i) s += sh[t + i * k];
+        part[(int64_t)blockIdx.x * k + t] = s;
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void k_axpy_cols(const c128* alpha, int sign,
                                                          const c128* V, c128* W, int64_t n, int k)
 {
@@ -3270,6 +3413,41 @@ void LaunchColDot(const c128* v, const c128* w, int64_t np, int k, c128* part, c
     const int g = ReducePartials(np);
     hipLaunchKernelGGL(k_coldot_part, dim3(g), dim3(kThreads), 0, s, v, w, np, k, part);
     hipLaunchKernelGGL(k_coldot_final, dim3(k), dim3(kThreads), 0, s, part, g, k, out);
+}
+
+int64_t ArnoldiPartials(int64_t np, int k, int m)
+{
+    return 2 * (int64_t)std::min(m, kMaxGram) * ReducePartials(np) * k;
+}
+
+int64_t ArnoldiGram(int k, int m)
+{
+    const int64_t g = std::min(m, kMaxGram);
+    return g * g * k;
+}
+
+void LaunchArnoldi(const c128* V, int j, int m, c128* w, int64_t np, int k, c128* part, c128* gram,
+                   double* npart, c128* h, double* norms, hipStream_t s)
+{
+    const int64_t n = np * k;
+    const int g = ReducePartials(np);
+    if (m <= kMaxGram) {
+        hipLaunchKernelGGL(k_arnoldi_dots, dim3(g, (j + kDotGroup) / kDotGroup), dim3(kThreads), 0, s,
+                           V, n, j, w, np, k, part);
+        hipLaunchKernelGGL(k_arnoldi_solve, dim3(k), dim3(kSolveThreads), 0, s, part, g, j, m, k,
+                           gram, h);
+        hipLaunchKernelGGL(k_arnoldi_update, dim3(g), dim3(kThreads), 0, s, V, n, j, h, w, np, k,
+                           npart);
+    } else {
+        // step i's update of w and step i + 1's dot product share a pass
+        LaunchColDot(V, w, np, k, part, h, s);
+        for (int i = 0; i < j; ++i)
+            LaunchAxpyDot(h + (int64_t)i * k, V + i * n, V + (i + 1) * n, w, np, k, part,
+                          h + (int64_t)(i + 1) * k, s);
+        LaunchAxpyCols(h + (int64_t)j * k, -1, V + j * n, w, np, k, s);
+        hipLaunchKernelGGL(k_colnorm_part, dim3(g), dim3(kThreads), 0, s, w, np, k, npart);
+    }
+    hipLaunchKernelGGL(k_colnorm_final, dim3(k), dim3(kThreads), 0, s, npart, g, k, norms);
 }
 
 void LaunchAxpyDot(const c128* alpha, const c128* v, const c128* vn, c128* w, int64_t np, int k,

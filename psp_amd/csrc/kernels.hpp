@@ -278,6 +278,16 @@ void LaunchSpmv(const StencilArgs& st, const double* vel, const c128* x, const c
 
 // Column reductions over N x k interleaved blocks (deterministic two-pass).
 int ReducePartials(int64_t npoints);
+// Step j of a cycle of m: w := w - V_{0..j} h by modified Gram-Schmidt (in two
+// passes up to m = 64, step by step beyond), h (j + 1 rows of k) and the norms of
+// the columns of w.  part: ArnoldiPartials, gram: ArnoldiGram entries, enough for
+// every shorter cycle too (the cycle's
+// products of basis vectors; steps 0 .. j - 1 filled their rows), npart: the
+// partial sums of a norm.
+int64_t ArnoldiPartials(int64_t npoints, int k, int m);
+int64_t ArnoldiGram(int k, int m);
+void LaunchArnoldi(const c128* V, int j, int m, c128* w, int64_t npoints, int k, c128* part,
+                   c128* gram, double* npart, c128* h, double* norms, hipStream_t s);
 void LaunchColNorm2(const c128* x, int64_t npoints, int k, double* part, double* out,
                     hipStream_t s);  // out[r] = ||x_r||_2
 void LaunchColDot(const c128* v, const c128* w, int64_t npoints, int k, c128* part,

@@ -66,7 +66,7 @@ struct psp_hip_ctx {
     int32_t* S[3] = {nullptr, nullptr, nullptr};  // per class: fused-launch state (counters)
     c128 *V = nullptr, *x = nullptr, *x0 = nullptr, *w = nullptr, *b = nullptr;
     double *partD = nullptr, *normD = nullptr;
-    c128 *partC = nullptr, *Hcol = nullptr, *ydev = nullptr;
+    c128 *partC = nullptr, *gram = nullptr, *Hcol = nullptr, *ydev = nullptr;
     // captured sweeps, keyed on (block pointer, k)
     bool useGraph = true;
     bool xcdReduce = true;  // split row blocks summed in the product launch (option)
@@ -578,8 +578,10 @@ int EnsureWorkspace(psp_hip_ctx* c, int k, int m)
     const int g = ReducePartials(N);
     if ((st = Alloc(c, &p, sizeof(double) * g * k, c->wsAllocs))) return st;
     c->partD = (double*)p;
-    if ((st = Alloc(c, &p, sizeof(c128) * g * k, c->wsAllocs))) return st;
+    if ((st = Alloc(c, &p, sizeof(c128) * ArnoldiPartials(N, k, m), c->wsAllocs))) return st;
     c->partC = (c128*)p;
+    if ((st = Alloc(c, &p, sizeof(c128) * ArnoldiGram(k, m), c->wsAllocs))) return st;
+    c->gram = (c128*)p;
     if ((st = Alloc(c, &p, sizeof(double) * k, c->wsAllocs))) return st;
     c->normD = (double*)p;
     if ((st = Alloc(c, &p, sizeof(c128) * (m + 1) * k, c->wsAllocs))) return st;
@@ -1135,15 +1137,11 @@ int Gmres(psp_hip_ctx* c, int k, int m, double relTol, int maxIts, int steps, do
             HIPCHK(c, hipEventRecord(ev.e[1], s));
             if ((rc = Precondition(c, c->w, k))) return rc;
             HIPCHK(c, hipEventRecord(ev.e[2], s));
-            // Arnoldi by modified Gram-Schmidt (solve.hpp:382-399): step i's
-            // update of w and step i + 1's dot product share one pass
-            LaunchColDot(c->V, c->w, N, k, c->partC, c->Hcol, s);
-            for (int i = 0; i < j; ++i)
-                LaunchAxpyDot(c->Hcol + (int64_t)i * k, c->V + (int64_t)i * n,
-                              c->V + (int64_t)(i + 1) * n, c->w, N, k, c->partC,
-                              c->Hcol + (int64_t)(i + 1) * k, s);
-            LaunchAxpyCols(c->Hcol + (int64_t)j * k, -1, c->V + (int64_t)j * n, c->w, N, k, s);
-            if ((rc = Norms(c, c->w, k, delta))) return rc;
+            // Arnoldi by modified Gram-Schmidt (solve.hpp:382-399)
+            LaunchArnoldi(c->V, j, m, c->w, N, k, c->partC, c->gram, c->partD, c->Hcol, c->normD, s);
+            delta.resize(k);
+            HIPCHK(c, hipMemcpyAsync(delta.data(), c->normD, sizeof(double) * k,
+                                     hipMemcpyDeviceToHost, s));
             HIPCHK(c, hipMemcpyAsync(hc.data(), c->Hcol, sizeof(c128) * (j + 1) * k,
                                      hipMemcpyDeviceToHost, s));
             HIPCHK(c, hipEventRecord(ev.e[3], s));
@@ -1662,15 +1660,12 @@ int GmresBatch(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>& ks, 
             for (int i = 0; i < np; ++i) {
                 if (!P[i].active) continue;
                 psp_hip_ctx* c = cs[i];
-                const int64_t N = P[i].N, n = P[i].n;
+                const int64_t N = P[i].N;
                 const int k = P[i].k;
-                LaunchColDot(c->V, c->w, N, k, c->partC, c->Hcol, s);
-                for (int l = 0; l < j; ++l)
-                    LaunchAxpyDot(c->Hcol + (int64_t)l * k, c->V + (int64_t)l * n,
-                                  c->V + (int64_t)(l + 1) * n, c->w, N, k, c->partC,
-                                  c->Hcol + (int64_t)(l + 1) * k, s);
-                LaunchAxpyCols(c->Hcol + (int64_t)j * k, -1, c->V + (int64_t)j * n, c->w, N, k, s);
-                if ((rc = norms(i))) return rc;
+                LaunchArnoldi(c->V, j, m, c->w, N, k, c->partC, c->gram, c->partD, c->Hcol, c->normD,
+                              s);
+                HIPCHK(c, hipMemcpyAsync(P[i].nrm, c->normD, sizeof(double) * k,
+                                         hipMemcpyDeviceToHost, s));
                 HIPCHK(c, hipMemcpyAsync(P[i].hc, c->Hcol, sizeof(c128) * (j + 1) * k,
                                          hipMemcpyDeviceToHost, s));
             }
