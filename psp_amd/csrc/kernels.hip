@@ -1464,7 +1464,6 @@ struct BlockBufs {
     const int32_t* bsrc;
     const int32_t* blist;
     const int32_t* udst;
-    const cx<T>* dinv;   // one panel's D^-1, by panel-vector row
     cx<T>* P;            // partial sums, 64 rows per slot
     int64_t w, g0, g1;   // VecRows
     int32_t xrows, zero; // zero: a block of zeros in F
@@ -1495,7 +1494,7 @@ __device__ __forceinline__ void BlockFinish(const BlockBufs<T>& a, int x0, int w
     if (PH == PH_B) {
         if (row < s) a.V[(int64_t)(x0 + row) * k + r] = v;
     } else if (row < s) {
-        a.V[(a.w + x0 + row) * k + r] = v * a.dinv[x0 + row];
+        a.V[(a.w + x0 + row) * k + r] = v;
     } else if (row >= kBlk * sb && row - kBlk * sb < u) {
         const int ur = u0 + row - kBlk * sb, dst = a.udst[ur];
         a.V[(int64_t)dst * k + r] = UpdateBase(a, ur, w0 + row, leaf, dst, r, k) + v;
@@ -1511,6 +1510,11 @@ struct BlockShape {
     // inner blocks per chunk of the staged vector
     static constexpr int CB = 16 / (KB / 8) / (sizeof(T) == 8 ? 2 : 1);
     static constexpr int SPT = CB * kBlk * KB / 256;  // staged elements per thread
+    // accumulators that a block's products are dealt to (BlockSum)
+    static constexpr int NA = KB == 8 ? (sizeof(T) == 4 ? 4 : 2) : 1;
+    // steps whose vector operands are read ahead: a whole block of them would
+    // take 64 more registers in FP64 with KB = 16
+    static constexpr int OS = sizeof(T) == 4 ? 4 : 2;
     static_assert(CB % U == 0 || U % CB == 0, "chunk shape");
 };
 
@@ -1541,9 +1545,7 @@ struct SliceElement {
             const int row = kBlk * t.ob0 + rl, ur = row - kBlk * t.sb;
             dst = 0;
             ga = gb = czero<T>();
-            if (ur < 0) {
-                x = a.dinv[t.x0 + row];
-            } else {
+            if (ur >= 0) {
                 dst = a.udst[t.u0 + ur];
                 if (!t.leaf) {
                     ga = a.V[(a.g0 + t.u0 + ur) * k + r];
@@ -1559,7 +1561,7 @@ struct SliceElement {
         if constexpr (PH == PH_B) {
             if (row < t.s) a.V[(int64_t)(t.x0 + row) * k + r] = v;
         } else if (row < t.s) {
-            a.V[(a.w + t.x0 + row) * k + r] = v * x;
+            a.V[(a.w + t.x0 + row) * k + r] = v;
         } else if (row >= kBlk * t.sb && row - kBlk * t.sb < t.u) {
             cx<T> g = czero<T>();
             if (!t.leaf) g = ga + gb;
@@ -1626,42 +1628,38 @@ __device__ __forceinline__ void SumSlices(const TileRec& t, const BlockBufs<T>& 
     if (tid == 0) redc[t.red] = 0;  // no slice of this launch counts any more
 }
 
-// Finish operands of a lane's 4 rows (rows row(lk, p) of output block ob):
-// D^-1 of pivot rows, or where update rows go.
+// Where a lane's 4 rows (rows row(lk, p) of output block ob) go, if they are
+// update rows.
 template <typename T>
 struct FinishOps {
-    cx<T> d[4];
     int32_t dst[4];
     __device__ void Load(const BlockBufs<T>& a, const TileRec& t, int ob, int lk)
     {
-        if (ob < t.sb) {
-            const cx<T>* p = a.dinv + t.x0 + kBlk * ob;
+        if (ob < t.sb) return;
+        const int32_t* p = a.udst + t.u0 + kBlk * (ob - t.sb);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) d[i] = p[Mfma<T>::row(lk, i)];
-        } else {
-            const int32_t* p = a.udst + t.u0 + kBlk * (ob - t.sb);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) dst[i] = p[Mfma<T>::row(lk, i)];
-        }
+        for (int i = 0; i < 4; ++i) dst[i] = p[Mfma<T>::row(lk, i)];
     }
 };
 
 // Stores a wave's output block: products of right-hand sides r0 + 8 n + li
 // (li < 8, below r0 + kc), as partial sums of a slice or finished.  The loads
 // of an update block are issued together for each n.
-template <typename T, int PH, int NB>
+template <typename T, int PH, int NB, class SUM>
 __device__ __forceinline__ void StoreBlock(const BlockBufs<T>& a, const TileRec& t, int q, int k,
                                            int r0, int kc, const FinishOps<T>& fo,
-                                           const typename Mfma<T>::acc (&acc)[NB])
+                                           const SUM (&sum)[NB])
 {
+    typedef typename SUM::real S;
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int ob = t.ob0 + q;
-    cx<T> o[NB][4];
+    cx<S> o[NB][4];
 #pragma unroll
-    for (int n = 0; n < NB; ++n)
+    for (int n = 0; n < NB; ++n) {
+        const typename SUM::vec v = sum[n].Value();
 #pragma unroll
-        for (int p = 0; p < 4; ++p)
-            o[n][p] = cx<T>{T(acc[n][p]), T(__shfl_xor(acc[n][p], 8, 64))};
+        for (int p = 0; p < 4; ++p) o[n][p] = cx<S>{S(v[p]), S(__shfl_xor(v[p], 8, 64))};
+    }
     auto each = [&](auto&& f) {
 #pragma unroll
         for (int n = 0; n < NB; ++n)
@@ -1671,17 +1669,17 @@ __device__ __forceinline__ void StoreBlock(const BlockBufs<T>& a, const TileRec&
     if (t.slot >= 0) {
         cx<T>* out = a.P + ((int64_t)t.slot * 64 + kBlk * q) * k + r0;
         each([&](int n, int p, int row, int r) {
-            if (li < 8 && r < kc) out[row * k + r] = o[n][p];
+            if (li < 8 && r < kc) out[row * k + r] = cvt<T>(o[n][p]);
         });
     } else if (PH == PH_B) {
         cx<T>* out = a.V + (int64_t)(t.x0 + kBlk * ob) * k + r0;
         each([&](int n, int p, int row, int r) {
-            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = o[n][p];
+            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = cvt<T>(o[n][p]);
         });
     } else if (ob < t.sb) {
         cx<T>* out = a.V + (a.w + t.x0 + kBlk * ob) * k + r0;
         each([&](int n, int p, int row, int r) {
-            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = o[n][p] * fo.d[p];
+            if (li < 8 && r < kc && kBlk * ob + row < t.s) out[row * k + r] = cvt<T>(o[n][p]);
         });
     } else {
         // an update row: the children's contributions to it and, for a pivot
@@ -1706,16 +1704,61 @@ __device__ __forceinline__ void StoreBlock(const BlockBufs<T>& a, const TileRec&
                     gb[p] = g1[Mfma<T>::row(lk, p) * k + rc];
                 }
 #pragma unroll
-                for (int p = 0; p < 4; ++p) o[n][p] = ga[p] + gb[p] + o[n][p];
+                for (int p = 0; p < 4; ++p) o[n][p] = cvt<S>(ga[p]) + cvt<S>(gb[p]) + o[n][p];
             }
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
-                const cx<T> v = fo.dst[p] < a.xrows ? x[p] + o[n][p] : o[n][p];
+                const cx<T> v = cvt<T>(fo.dst[p] < a.xrows ? cvt<S>(x[p]) + o[n][p] : o[n][p]);
                 if (li < 8 && r < kc && ru + Mfma<T>::row(lk, p) < t.u) out[p][r] = v;
             }
         }
     }
 }
+
+// The sum of an output block over the inner blocks.  A block's products run
+// through accumulators of their own, from zero, and are added here: one
+// accumulator through a whole slice (up to 768 columns) rounds two to four times
+// as much as the sums need, and GMRES with FP32 fronts then stalls before its
+// tolerance (40^3, k = 1, to 1e-5: 21 steps, 18 so).  TWICE: in twice the
+// precision of T (FP64: a value and what its additions rounded off, by the
+// Moller-Knuth sum of two numbers), for few right-hand sides, where nothing else
+// of a launch takes the time.  What a sweep of u + v differs from those of u and
+// of v by, the rounding of its vectors and sums, k = 1, with one accumulator and
+// so: 40^3 FP32 3.7e-7 and 1.2e-7, FP64 7.0e-16 and 2.5e-16; 61 x 47 x 83 FP32
+// 5.4e-7 and 1.1e-7, FP64 8.4e-16 and 2.5e-16; k = 32 at 100^3 FP32 7.2e-7 and
+// 2.1e-7, FP64 1.3e-15 and 4.0e-16.
+template <typename T, bool TWICE>
+struct BlockSum {
+    typedef typename Mfma<T>::acc vec;
+    typedef T real;
+    vec v{0, 0, 0, 0};
+    __device__ __forceinline__ void Add(const vec& z) { v += z; }
+    __device__ __forceinline__ vec Value() const { return v; }
+};
+template <>
+struct BlockSum<float, true> {
+    typedef Mfma<double>::acc vec;
+    typedef double real;
+    vec v{0, 0, 0, 0};
+    __device__ __forceinline__ void Add(const Mfma<float>::acc& z)
+    {
+        v += __builtin_convertvector(z, vec);
+    }
+    __device__ __forceinline__ vec Value() const { return v; }
+};
+template <>
+struct BlockSum<double, true> {
+    typedef Mfma<double>::acc vec;
+    typedef double real;
+    vec v{0, 0, 0, 0}, off{0, 0, 0, 0};
+    __device__ __forceinline__ void Add(const vec& z)
+    {
+        const vec s = v + z, d = s - v;
+        off += (v - (s - d)) + (z - d);
+        v = s;
+    }
+    __device__ __forceinline__ vec Value() const { return v + off; }
+};
 
 // One workgroup: up to KB = 8 or 16 right-hand sides of a tile (shared by
 // k_block and k_block_batch).  Reads of the vector and of the index lists may
@@ -1727,7 +1770,7 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
 {
     typedef typename Mfma<T>::acc acc_t;
     typedef BlockShape<T, KB> S;
-    constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT, U = S::U;
+    constexpr int NB = S::NB, CB = S::CB, SPT = S::SPT, U = S::U, NA = S::NA, OS = S::OS;
     constexpr int RP = 256 / KB;  // rows staged by one load of the workgroup
     __shared__ cx<T> vs[CB * kBlk][KB];
     const int tid = threadIdx.x, lane = tid & 63, q = Uni(tid >> 6);
@@ -1796,29 +1839,51 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
             vs[row][tid % KB] = mk(v.r, v.i);
         }
     };
-    acc_t acc[NB];
-    // vector operands of the block at inner index i of the chunk
-    struct Operand {
-        cx<T> v[4][NB];
+    acc_t acc[NA][NB];
+    BlockSum<T, KB == 8> sum[NB];
+    auto clear = [&]() {
+#pragma unroll
+        for (int h = 0; h < NA; ++h)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[h][n] = acc_t{0, 0, 0, 0};
     };
-    auto operand = [&](int i) {
+    auto fold = [&]() {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            if constexpr (NA == 4)
+                sum[n].Add((acc[0][n] + acc[1][n]) + (acc[2][n] + acc[3][n]));
+            else if constexpr (NA == 2)
+                sum[n].Add(acc[0][n] + acc[1][n]);
+            else
+                sum[n].Add(acc[0][n]);
+        }
+        clear();
+    };
+    // vector operands of OS steps from step st of the block at inner index i of
+    // the chunk
+    struct Operand {
+        cx<T> v[OS][NB];
+    };
+    auto operand = [&](int i, int st) {
         Operand o;
 #pragma unroll
-        for (int st = 0; st < 4; ++st)
+        for (int j = 0; j < OS; ++j)
 #pragma unroll
-            for (int n = 0; n < NB; ++n) o.v[st][n] = vs[kBlk * i + 4 * st + lk][8 * n + (li & 7)];
+            for (int n = 0; n < NB; ++n)
+                o.v[j][n] = vs[kBlk * i + 4 * (st + j) + lk][8 * n + (li & 7)];
         return o;
     };
-    auto multiply = [&](int u, const Operand& o) {
+    auto multiply = [&](int u, int st, const Operand& o) {
 #pragma unroll
-        for (int st = 0; st < 4; ++st)
+        for (int j = 0; j < OS; ++j)
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
-                const cx<T> v = o.v[st][n];
+                const cx<T> v = o.v[j][n];
                 const T b1 = li < 8 ? v.r : v.i;
                 const T b2 = li < 8 ? -v.i : v.r;
-                acc[n] = Mfma<T>::step(m[u][st].r, b1, acc[n]);
-                acc[n] = Mfma<T>::step(m[u][st].i, b2, acc[n]);
+                const int h1 = NA == 4 ? 2 * ((st + j) & 1) : 0, h2 = NA > 1 ? h1 + 1 : 0;
+                acc[h1][n] = Mfma<T>::step(m[u][st + j].r, b1, acc[h1][n]);
+                acc[h2][n] = Mfma<T>::step(m[u][st + j].i, b2, acc[h2][n]);
             }
     };
     // the chunk's products, half a ring at a time, each register group refilled
@@ -1827,15 +1892,25 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
     auto run = [&](int c) {
         const int left = t.nib - c * CB;
         constexpr int H = U / 2;
-        Operand o = operand(0);
+        Operand o = operand(0, 0);
         for (int i0 = 0;; i0 += U) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
                 for (int u = H * h; u < H * h + H; ++u) {
-                    const Operand o1 = operand(min(i0 + u + 1, CB - 1));
-                    if (id[u] != a.zero) multiply(u, o);
-                    o = o1;
+                    const int i1 = min(i0 + u + 1, CB - 1);
+                    if (id[u] == a.zero) {
+                        o = operand(i1, 0);
+                        continue;
+                    }
+#pragma unroll
+                    for (int st = 0; st < 4; st += OS) {
+                        const Operand o1 =
+                            st + OS < 4 ? operand(i0 + u, st + OS) : operand(i1, 0);
+                        multiply(u, st, o);
+                        o = o1;
+                    }
+                    fold();
                 }
                 if (i0 + H * h + H >= left) return;
 #pragma unroll
@@ -1853,8 +1928,7 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
     const bool own = q < t.nob;
     FinishOps<T> fo;
     if (PH == PH_F && own && t.slot < 0) fo.Load(a, t, t.ob0 + q, lk);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
+    clear();
     put();
     LdsBarrier();
     run(0);
@@ -1867,7 +1941,7 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
         LdsBarrier();
         run(c);
     }
-    if (own) StoreBlock<T, PH, NB>(a, t, q, k, 0, k, fo, acc);
+    if (own) StoreBlock<T, PH, NB>(a, t, q, k, 0, k, fo, sum);
     if (redc != nullptr && t.slot >= 0) SumSlices<T, PH, KB>(t, a, k, 0, k, redc, reds);
 }
 
@@ -1933,9 +2007,7 @@ __device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBu
             for (int st = 0; st < 4; ++st) d.m[b][st] = (p + (PH == PH_F ? 4 * kBlk * st : st))[loff];
         }
     };
-    acc_t acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = acc_t{0, 0, 0, 0};
+    BlockSum<T, false> sum[NB];
     // (stages past the end read the last chunk again, unused)
     int32_t sx[PH == PH_B ? SPT : 1];
     auto indices = [&](int c) {
@@ -1992,15 +2064,18 @@ __device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBu
         for (int b = 0; b < CB; ++b) {
             if (d.blk[b] == a.zero) continue;
 #pragma unroll
-            for (int st = 0; st < 4; ++st)
+            for (int n = 0; n < NB; ++n) {
+                acc_t acc{0, 0, 0, 0};
 #pragma unroll
-                for (int n = 0; n < NB; ++n) {
+                for (int st = 0; st < 4; ++st) {
                     const cx<T> v = vs[c & 1][kBlk * b + 4 * st + lk][8 * n + (li & 7)];
                     const T b1 = li < 8 ? v.r : v.i;
                     const T b2 = li < 8 ? -v.i : v.r;
-                    acc[n] = Mfma<T>::step(d.m[b][st].r, b1, acc[n]);
-                    acc[n] = Mfma<T>::step(d.m[b][st].i, b2, acc[n]);
+                    acc = Mfma<T>::step(d.m[b][st].r, b1, acc);
+                    acc = Mfma<T>::step(d.m[b][st].i, b2, acc);
                 }
+                sum[n].Add(acc);
+            }
         }
         factor(c + 2, d);
     };
@@ -2012,7 +2087,7 @@ __device__ __forceinline__ void BlockTileWide(const BlockTile* tp, const BlockBu
     if (q < t.nob) {
         FinishOps<T> fo;
         if (PH == PH_F && t.slot < 0) fo.Load(a, t, t.ob0 + q, lk);
-        StoreBlock<T, PH, NB>(a, t, q, k, r0, kc, fo, acc);
+        StoreBlock<T, PH, NB>(a, t, q, k, r0, kc, fo, sum);
     }
     if (redc != nullptr && t.slot >= 0) SumSlices<T, PH, KB>(t, a, k, r0, kc, redc, reds);
 }
@@ -2083,7 +2158,9 @@ __global__ __launch_bounds__(kThreads) void k_block_reduce(const BlockRed* reds,
 // --------------------------------------------------------------------------
 // Fold: the merged fronts' F from the factored fine fronts (L after the
 // selective inversion: Linv below the diagonal, D on it, L_BL below; E =
-// -L_BL Linv from a batched product).
+// -L_BL Linv from a batched product).  Pivot rows are scaled by D^-1/2, so that F
+// serves both directions without a product by D^-1 between them, whose rounding
+// would come on top of theirs.
 // --------------------------------------------------------------------------
 // Address of (row, column) of a merged front in F.
 __device__ __forceinline__ int64_t BlockAt(int browBase, int row, int col)
@@ -2091,15 +2168,23 @@ __device__ __forceinline__ int64_t BlockAt(int browBase, int row, int col)
     return (int64_t)(browBase + (col >> 4)) * (kBlk * kBlk) + (col & 15) * kBlk + (row & 15);
 }
 
-// Copies a 32 x 32 piece of a node's front: its own lower triangle (with the
-// unit diagonal; D^-1 goes to dinv), or rows of E of a group's top node.
+// A square root of z, by the half-angle formulas (F's scale is used twice, so
+// either root will do).
+__device__ __forceinline__ c128 csqrt(c128 z)
+{
+    const double m = sqrt(0.5 * (hypot(z.r, z.i) + fabs(z.r)));
+    const double o = m > 0.0 ? 0.5 * fabs(z.i) / m : 0.0;
+    return z.r >= 0.0 ? c128{m, z.i < 0.0 ? -o : o} : c128{o, z.i < 0.0 ? -m : m};
+}
+
+// Copies a 32 x 32 piece of a node's front: its own lower triangle (row i of the
+// unit lower Linv times D_i^-1/2), or rows of E of a group's top node.
 // Entries of F outside every piece stay zero from its allocation.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_pack(const TransItem* items, const FoldNode* nodes,
                                                    const int32_t* browBase, const cx<T>* L,
                                                    int64_t fstore, const cx<T>* E, int64_t estride,
-                                                   cx<T>* F, int64_t fentries, cx<T>* dinv,
-                                                   int xrows)
+                                                   cx<T>* F, int64_t fentries)
 {
     const TransItem it = items[blockIdx.x];
     const FoldNode f = nodes[it.node];
@@ -2111,18 +2196,17 @@ __global__ __launch_bounds__(kThreads) void k_pack(const TransItem* items, const
     if (i >= (own ? f.s : fs)) return;
     const int row = own ? f.mcol + i : f.urow + i - f.s;
     const int bb = browBase[f.br0 + (row >> 4)];
+    c128 scale{1.0, 0.0};
+    if (own) scale = csqrt(cinv(cvt<double>(Lf[i + (int64_t)i * fs])));
     for (int j = it.j0 + (threadIdx.x >> 5); j < min(it.j0 + 32, f.s); j += 8) {
         if (own && i < j) break;
         cx<T> v;
-        if (!own) {
+        if (!own)
             v = Ef[i - f.s + (int64_t)j * f.u];
-        } else {
-            v = Lf[i + (int64_t)j * fs];
-            if (i == j) {
-                dinv[(int64_t)blockIdx.y * xrows + f.x0 + i] = cinv(v);
-                v = cx<T>{T(1), T(0)};
-            }
-        }
+        else if (i == j)
+            v = cvt<T>(scale);
+        else
+            v = cvt<T>(scale * cvt<double>(Lf[i + (int64_t)j * fs]));
         Fp[BlockAt(bb, row, f.mcol + j)] = v;
     }
 }
@@ -2196,7 +2280,7 @@ template <typename T>
 __device__ __forceinline__ BlockBufs<T> SegBufs(const BatchSolveSeg& sg)
 {
     return BlockBufs<T>{(const cx<T>*)sg.F, (cx<T>*)sg.V, sg.bsrc, sg.blist, sg.udst,
-                        (const cx<T>*)sg.dinv, (cx<T>*)sg.P, sg.w, sg.g0, sg.g1, sg.xrows,
+                        (cx<T>*)sg.P, sg.w, sg.g0, sg.g1, sg.xrows,
                         sg.zero};
 }
 
@@ -3119,7 +3203,6 @@ void LaunchPanelSolve(const ClassDev& c, const ClassPlan& plan, int b, void* V, 
                             c.bsrc,
                             c.blist,
                             c.udst,
-                            (const cx<T>*)c.dinv + (int64_t)b * c.xrows,
                             (cx<T>*)P,
                             vr.w,
                             vr.g0,
@@ -3251,7 +3334,7 @@ void LaunchPack(const ClassDev& c, hipStream_t s)
     if (c.npacks <= 0) return;
     hipLaunchKernelGGL((k_pack<T>), dim3(c.npacks, c.npanels), dim3(kThreads), 0, s, c.packs,
                        c.foldNodes, c.browBase, (const cx<T>*)c.L, c.fstore, (const cx<T>*)c.U,
-                       c.ustore, (cx<T>*)c.F, c.fentries, (cx<T>*)c.dinv, c.xrows);
+                       c.ustore, (cx<T>*)c.F, c.fentries);
 }
 
 template <typename T>

@@ -108,7 +108,6 @@ struct ClassDev {
     int32_t xrows = 0;
     int64_t fentries = 0;           // entries of one panel's F
     void* F = nullptr;              // npanels * fentries
-    void* dinv = nullptr;           // npanels * xrows
     int32_t *browBase = nullptr, *flist = nullptr, *fsrc = nullptr;
     FoldNode* foldNodes = nullptr;
     TransItem* packs = nullptr;
@@ -143,7 +142,7 @@ struct BatchBlock {
 // One problem's panel solve in a batched product or reduce launch (front
 // precision erased: the kernels cast to their cx<T>).
 struct BatchSolveSeg {
-    const void *F, *dinv;    // this panel's factor
+    const void* F;           // this panel's factor
     void *V, *P;
     const int32_t *bsrc, *blist, *udst;
     int64_t w, g0, g1;       // VecRows

@@ -416,8 +416,8 @@ int EnsureDevice(psp_hip_ctx* c)
 }
 
 // Factor storage, allocated by the first Initialize after construction or
-// Finalize and kept until Finalize: L (the factorization), F and D^-1 (the
-// merged solves) and, for the fused subtree launches, LT.
+// Finalize and kept until Finalize: L (the factorization), F (the merged
+// solves) and, for the fused subtree launches, LT.
 int EnsureFactorStorage(psp_hip_ctx* c)
 {
     const size_t eb = FrontBytes(c);
@@ -438,14 +438,10 @@ int EnsureFactorStorage(psp_hip_ctx* c)
             HIPCHK(c, hipMemsetAsync((char*)D.L + body, 0, fb - body, c->stream));
         }
         if (!D.F) {
-            // entries of F and D^-1 that no fold writes (padding of the
-            // blocks) stay zero
+            // entries of F that no fold writes (padding of the blocks) stay zero
             const size_t f = eb * (size_t)D.npanels * D.fentries;
-            const size_t v = eb * (size_t)D.npanels * D.xrows;
             if ((st = Alloc(c, &D.F, f, c->facStore))) return st;
             HIPCHK(c, hipMemsetAsync(D.F, 0, std::max<size_t>(f, 16), c->stream));
-            if ((st = Alloc(c, &D.dinv, v, c->facStore))) return st;
-            HIPCHK(c, hipMemsetAsync(D.dinv, 0, std::max<size_t>(v, 16), c->stream));
         }
         if (c->plan.fused && !D.LT) {
             // the fold writes every entry of LT
@@ -464,7 +460,6 @@ void FreeFactorStorage(psp_hip_ctx* c)
         c->dev[cl].L = nullptr;
         c->dev[cl].LT = nullptr;
         c->dev[cl].F = nullptr;
-        c->dev[cl].dinv = nullptr;
     }
     c->factored = false;
     c->facFused = false;
@@ -1352,7 +1347,6 @@ void BuildBatchSweep(const std::vector<psp_hip_ctx*>& cs, const std::vector<int>
             const VecRows vr(c->plan.cls[cl]);
             BatchSolveSeg s{};
             s.F = (const char*)D.F + eb * b * D.fentries;
-            s.dinv = (const char*)D.dinv + eb * b * D.xrows;
             s.V = c->vec[cl];
             s.P = c->P;
             s.bsrc = D.bsrc;

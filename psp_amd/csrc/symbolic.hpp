@@ -167,11 +167,11 @@ struct GemmLaunch {
 // one merged front, solved with the explicit inverse of its whole pivot
 // block, so a panel solve takes one launch per group and direction instead
 // of one per level.  A merged front's factor F has the group's pivots as
-// columns and, as rows, the same pivots (Linv, unit lower) followed by the
-// top node's update rows (-L_BL Linv), in blocks of 16 x 16.  Blocks are
+// columns and, as rows, the same pivots (D^-1/2 Linv, lower triangular) followed
+// by the top node's update rows (-L_BL Linv), in blocks of 16 x 16.  Blocks are
 // stored once, row of blocks by row of blocks, and serve both directions:
-//   forward   [y; w] = F g          (y scaled by D^-1 for the backward pass)
-//   backward  x = F^T [D^-1 y; x_struct].
+//   forward   [y; w] = F g
+//   backward  x = F^T [y; x_struct].
 // Pivots keep their post-order, so the pivots under a node are contiguous
 // and row i of F has its entries in one column range: from the first pivot
 // below i's node to i.  Blocks of siblings that do not meet are not stored.
