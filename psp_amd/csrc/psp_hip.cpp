@@ -90,6 +90,7 @@ namespace {
     do {                                                                               \
         hipError_t e_ = (expr);                                                        \
         if (e_ != hipSuccess) {                                                        \
+            (void)hipGetLastError(); /* reported here, not by a later call's check */  \
             (ctx)->err = std::string(#expr) + ": " + hipGetErrorString(e_);            \
             return e_ == hipErrorOutOfMemory ? PSP_HIP_ERR_MEMORY : PSP_HIP_ERR_HIP;   \
         }                                                                              \
@@ -415,12 +416,31 @@ int EnsureDevice(psp_hip_ctx* c)
     return PSP_HIP_OK;
 }
 
+// Frees the factor storage allocated after the first `keep` arrays.
+void FreeFactorStorageFrom(psp_hip_ctx* c, size_t keep)
+{
+    for (; c->facStore.size() > keep; c->facStore.pop_back()) {
+        void* const p = c->facStore.back();
+        for (ClassDev& D : c->dev)
+            for (void** q : {&D.L, &D.F, &D.LT})
+                if (*q == p) *q = nullptr;
+        (void)hipFree(p);
+    }
+}
+
 // Factor storage, allocated by the first Initialize after construction or
 // Finalize and kept until Finalize: L (the factorization), F (the merged
 // solves) and, for the fused subtree launches, LT.
 int EnsureFactorStorage(psp_hip_ctx* c)
 {
     const size_t eb = FrontBytes(c);
+    // the first `body` bytes are not cleared
+    auto add = [&](void** q, size_t body, size_t bytes) -> int {
+        int st = Alloc(c, q, bytes, c->facStore);
+        if (st) return st;
+        if (bytes > body) HIPCHK(c, hipMemsetAsync((char*)*q + body, 0, bytes - body, c->stream));
+        return PSP_HIP_OK;
+    };
     for (int cl = 0; cl < 3; ++cl) {
         if (!c->plan.present[cl]) continue;
         ClassDev& D = c->dev[cl];
@@ -431,36 +451,20 @@ int EnsureFactorStorage(psp_hip_ctx* c)
         const size_t body = eb * (size_t)D.npanels * D.fstore;
         const size_t fb = body + eb * (size_t)kSolvePad * maxFs;
         int st;
-        if (!D.L) {
-            // only the padding needs zeroing here: every factorization
-            // zeroes L before assembly
-            if ((st = Alloc(c, &D.L, fb, c->facStore))) return st;
-            HIPCHK(c, hipMemsetAsync((char*)D.L + body, 0, fb - body, c->stream));
-        }
-        if (!D.F) {
-            // entries of F that no fold writes (padding of the blocks) stay zero
-            const size_t f = eb * (size_t)D.npanels * D.fentries;
-            if ((st = Alloc(c, &D.F, f, c->facStore))) return st;
-            HIPCHK(c, hipMemsetAsync(D.F, 0, std::max<size_t>(f, 16), c->stream));
-        }
-        if (c->plan.fused && !D.LT) {
-            // the fold writes every entry of LT
-            if ((st = Alloc(c, &D.LT, fb, c->facStore))) return st;
-            HIPCHK(c, hipMemsetAsync((char*)D.LT + body, 0, fb - body, c->stream));
-        }
+        // only the padding needs zeroing here: every factorization zeroes L
+        // before assembly
+        if (!D.L && (st = add(&D.L, body, fb))) return st;
+        // entries of F that no fold writes (padding of the blocks) stay zero
+        if (!D.F && (st = add(&D.F, 0, eb * (size_t)D.npanels * D.fentries))) return st;
+        // the fold writes every entry of LT
+        if (c->plan.fused && !D.LT && (st = add(&D.LT, body, fb))) return st;
     }
     return PSP_HIP_OK;
 }
 
 void FreeFactorStorage(psp_hip_ctx* c)
 {
-    for (void* p : c->facStore) (void)hipFree(p);
-    c->facStore.clear();
-    for (int cl = 0; cl < 3; ++cl) {
-        c->dev[cl].L = nullptr;
-        c->dev[cl].LT = nullptr;
-        c->dev[cl].F = nullptr;
-    }
+    FreeFactorStorageFrom(c, 0);
     c->factored = false;
     c->facFused = false;
 }
@@ -801,23 +805,25 @@ int FactorClasses(psp_hip_ctx* c, double* tFill, double* tLdl, double* tInv, dou
 // (fill, LDL, inversion and fold, Schur GEMMs).
 int Factor(psp_hip_ctx* c, double t[4])
 {
+    const size_t storage = c->facStore.size();
     int st = EnsureFactorStorage(c);
-    if (st) return st;
-    // a new factorization invalidates the captured sweeps' results only, not
-    // their launches: the graphs keep reading the same factor arrays
-    c->factored = false;
     // The Schur-complement (U) and inversion (T) scratch lives only while
     // factoring, so that many factored problems fit in HBM at once.
     const size_t eb = FrontBytes(c);
     for (int cl = 0; cl < 3; ++cl) {
-        if (!c->plan.present[cl]) continue;
+        if (st || !c->plan.present[cl]) continue;
         ClassDev& D = c->dev[cl];
-        if ((st = Alloc(c, &D.U, eb * (size_t)D.npanels * D.ustore, c->facAllocs)) ||
-            (st = Alloc(c, &D.T, eb * (size_t)D.npanels * D.tstore, c->facAllocs))) {
-            FreeFactorScratch(c);
-            return st;
-        }
+        st = Alloc(c, &D.U, eb * (size_t)D.npanels * D.ustore, c->facAllocs);
+        if (!st) st = Alloc(c, &D.T, eb * (size_t)D.npanels * D.tstore, c->facAllocs);
     }
+    if (st) {  // the factors of an earlier call stay as they are
+        FreeFactorScratch(c);
+        FreeFactorStorageFrom(c, storage);
+        return st;
+    }
+    // a new factorization invalidates the captured sweeps' results only, not
+    // their launches: the graphs keep reading the same factor arrays
+    c->factored = false;
     st = c->desc.precision == PSP_HIP_FRONTS_FP32
              ? FactorClasses<float>(c, &t[0], &t[1], &t[2], &t[3])
              : FactorClasses<double>(c, &t[0], &t[1], &t[2], &t[3]);
