@@ -64,11 +64,14 @@ enum {
     PSP_HIP_OPT_SOLVE_FUSED = 7,       /* 1: for 8 <= k <= 16, the tree levels from
                                           the cut depth down run as one persistent
                                           launch per direction, a subtree queue per
-                                          XCD, on factors in their own layout (made
-                                          by the next factorization, or from the
-                                          same velocity by the next solve); 0
-                                          (default): merged solves, one launch per
-                                          depth group and direction */
+                                          XCD, on factors in their own layout: made
+                                          by the next factorization, or by the next
+                                          solve or sweep of 8 <= k <= 16, which
+                                          factors the same velocity once more (with
+                                          the memory for it; otherwise, and in
+                                          psp_hip_precondition_noalloc until then,
+                                          merged solves); 0 (default): merged solves,
+                                          one launch per depth group and direction */
     PSP_HIP_OPT_SOLVE_FUSED_QUEUES = 8, /* queues of the fused launches (default 8,
                                           one per XCD; more leaves queues that the
                                           last workgroup runs alone) */

@@ -496,38 +496,38 @@ void FreeWorkspace(psp_hip_ctx* c)
     c->wsK = c->wsM = 0;
 }
 
-int64_t NeededSlots(const psp_hip_ctx* c)
+int64_t NeededSlots(const psp_hip_ctx* c, bool fused)
 {
     int64_t maxs = 1;
     for (int cl = 0; cl < 3; ++cl)
         if (c->plan.present[cl]) {
             maxs = std::max<int64_t>(maxs, c->plan.cls[cl].bslots);
-            if (c->plan.fused) maxs = std::max<int64_t>(maxs, c->plan.cls[cl].maxSlots);
+            if (fused) maxs = std::max<int64_t>(maxs, c->plan.cls[cl].maxSlots);
         }
     return maxs;
 }
 
 // Byte sizes of the sweep's buffers for k right-hand sides: per panel class
 // the solve vector (VecRows; the rows nothing writes must read as zero) and
-// the partial sums P.  The fused launches add the padded panel vector Xp, the
-// node work vectors W and per class the two slot copies G of the children's
+// the partial sums P.  The fused launches (fused) add the padded panel vector Xp,
+// the node work vectors W and per class the two slot copies G of the children's
 // update rows, each ending in kSolvePad + 2 rows that must read as zero (the
 // kernels read past a tile's rows), and their launch state.
 struct SweepSizes {
     size_t v[3] = {0, 0, 0}, p = 0, xp = 0, w = 0, g[3] = {0, 0, 0}, s[3] = {0, 0, 0};
 };
 
-SweepSizes SweepBufferSizes(const psp_hip_ctx* c, int k)
+SweepSizes SweepBufferSizes(const psp_hip_ctx* c, int k, bool fused)
 {
     const size_t eb = FrontBytes(c);
     const size_t padRows = (size_t)kSolvePad + 2;
     SweepSizes z;
-    z.p = eb * NeededSlots(c) * 64 * k;
+    z.p = eb * NeededSlots(c, fused) * 64 * k;
     for (int cl = 0; cl < 3; ++cl) {
         if (!c->plan.present[cl]) continue;
         const ClassPlan& C = c->plan.cls[cl];
         z.v[cl] = eb * (size_t)VecRows(C).total * k;
-        if (!c->plan.fused) continue;
+        if (!fused) continue;
         z.xp = std::max(z.xp, eb * ((size_t)C.n + padRows) * k);
         z.w = std::max(z.w, eb * ((size_t)C.wstore + padRows) * k);
         z.g[cl] = eb * (2 * (size_t)C.wstore + padRows) * k;
@@ -538,10 +538,11 @@ SweepSizes SweepBufferSizes(const psp_hip_ctx* c, int k)
 
 int EnsureWorkspace(psp_hip_ctx* c, int k, int m)
 {
-    if (c->wsK == k && c->wsM >= m && c->wsSlots >= NeededSlots(c)) return PSP_HIP_OK;
+    const bool fused = c->plan.fused;
+    if (c->wsK == k && c->wsM >= m && c->wsSlots >= NeededSlots(c, fused)) return PSP_HIP_OK;
     FreeWorkspace(c);
     const int64_t N = (int64_t)c->desc.nx * c->desc.ny * c->desc.nz;
-    const SweepSizes z = SweepBufferSizes(c, k);
+    const SweepSizes z = SweepBufferSizes(c, k, fused);
     int st;
     void* p;
     if ((st = Alloc(c, &c->P, z.p, c->wsAllocs))) return st;
@@ -553,12 +554,12 @@ int EnsureWorkspace(psp_hip_ctx* c, int k, int m)
         HIPCHK(c, hipMemsetAsync(*q, 0, bytes, c->stream));
         return PSP_HIP_OK;
     };
-    if (c->plan.fused && ((st = zeroed(&c->Xp, z.xp)) || (st = zeroed(&c->W, z.w)))) return st;
+    if (fused && ((st = zeroed(&c->Xp, z.xp)) || (st = zeroed(&c->W, z.w)))) return st;
     for (int cl = 0; cl < 3; ++cl) {
         c->vec[cl] = c->G[cl] = nullptr;
         if (!c->plan.present[cl]) continue;
         if ((st = zeroed(&c->vec[cl], z.v[cl]))) return st;
-        if (!c->plan.fused) continue;
+        if (!fused) continue;
         if ((st = zeroed(&c->G[cl], z.g[cl]))) return st;
         void* sp = nullptr;
         if ((st = Alloc(c, &sp, z.s[cl], c->wsAllocs))) return st;
@@ -589,7 +590,7 @@ int EnsureWorkspace(psp_hip_ctx* c, int k, int m)
     c->ydev = (c128*)p;
     c->wsK = k;
     c->wsM = m;
-    c->wsSlots = NeededSlots(c);
+    c->wsSlots = NeededSlots(c, fused);
     return PSP_HIP_OK;
 }
 
@@ -841,13 +842,26 @@ int Factor(psp_hip_ctx* c, double t[4])
     return PSP_HIP_OK;
 }
 
-// The fused launches were switched on after Initialize: factor once more, with
-// their layout.
-int EnsureFusedFactors(psp_hip_ctx* c)
+// Whether class cl's panel solves for k right-hand sides are the fused launches'
+// (given factors in their layout).
+bool FusedClass(const psp_hip_ctx* c, int cl, int k)
 {
-    if (!c->plan.fused || c->facFused) return PSP_HIP_OK;
+    return c->plan.fused && c->plan.present[cl] &&
+           FusedApplies(c->dev[cl], c->plan.cls[cl], k, (int64_t)FrontBytes(c));
+}
+
+// Before a sweep of k right-hand sides: where it would use the fused launches and
+// they were switched on after Initialize, factors once more, with their layout.
+// Without the memory for that the merged solves serve, as the factors stand.
+int EnsureFusedFactors(psp_hip_ctx* c, int k)
+{
+    if (c->facFused || !(FusedClass(c, 0, k) || FusedClass(c, 1, k) || FusedClass(c, 2, k)))
+        return PSP_HIP_OK;
     double t[4];
-    return Factor(c, t);
+    const int st = Factor(c, t);
+    if (st == PSP_HIP_ERR_MEMORY && c->factored) return PSP_HIP_OK;
+    if (st == PSP_HIP_OK) FreeGraphs(c);  // captured sweeps of merged solves
+    return st;
 }
 
 // ---------------------------------------------------------------------------
@@ -868,7 +882,7 @@ struct PanelSolver {
     int32_t* sync;
     PanelSolver(psp_hip_ctx* c_, int cl_, int k_)
         : c(c_), cl(cl_), k(k_), D(c_->dev[cl_]),
-          fused(c_->plan.fused && FusedApplies(D, c_->plan.cls[cl_], k_, sizeof(cx<T>))),
+          fused(c_->facFused && FusedClass(c_, cl_, k_)),
           map(fused ? PanelMap{D.n, D.qxy, D.qv} : PanelMap{D.xrows, D.sxy, D.sv}),
           x(fused ? c_->Xp : c_->vec[cl_]), sync(fused ? c_->S[cl_] : nullptr)
     {
@@ -1208,7 +1222,7 @@ int CheckSolveArgs(psp_hip_ctx* c, const void* B, int k, int m)
     if (!B) return Fail(c, PSP_HIP_ERR_INVALID, "null right-hand side");
     if (k < 1 || k > 256) return Fail(c, PSP_HIP_ERR_INVALID, "number of RHS must be in [1, 256]");
     if (m < 1) return Fail(c, PSP_HIP_ERR_INVALID, "GMRES restart length must be >= 1");
-    return EnsureFusedFactors(c);
+    return PSP_HIP_OK;
 }
 
 int RunSolve(psp_hip_ctx* c, void* B, int k, int m, double relTol, int maxIts, int flags,
@@ -1217,7 +1231,7 @@ int RunSolve(psp_hip_ctx* c, void* B, int k, int m, double relTol, int maxIts, i
     int rc = CheckSolveArgs(c, B, k, m);
     if (rc) return rc;
     const double t0 = Now();
-    if ((rc = EnsureWorkspace(c, k, m))) return rc;
+    if ((rc = EnsureFusedFactors(c, k)) || (rc = EnsureWorkspace(c, k, m))) return rc;
     const int64_t n = (int64_t)c->desc.nx * c->desc.ny * c->desc.nz * k;
     const bool dev = flags & PSP_HIP_DEVICE_POINTER;
     // PullRightHandSides: natural order is the working order on the GPU.
@@ -2199,7 +2213,9 @@ int psp_hip_precondition(psp_hip_ctx* c, void* B, int k)
 {
     int rc = CheckSolveArgs(c, B, k, 1);
     if (rc) return rc;
-    if ((rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1)))) return rc;
+    if ((rc = EnsureFusedFactors(c, k)) ||
+        (rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1))))
+        return rc;
     if ((rc = Precondition(c, (c128*)B, k))) return rc;
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -2211,7 +2227,7 @@ int psp_hip_precondition_noalloc(psp_hip_ctx* c, void* B, int k)
     int rc = CheckSolveArgs(c, B, k, 1);
     if (rc) return rc;
     if (!c->scratch) return Fail(c, PSP_HIP_ERR_STATE, "device scratch not set up");
-    const SweepSizes z = SweepBufferSizes(c, k);
+    const SweepSizes z = SweepBufferSizes(c, k, c->plan.fused && c->facFused);
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     size_t need = up(z.p) + up(z.xp) + up(z.w);
     for (int cl = 0; cl < 3; ++cl) need += up(z.v[cl]) + up(z.g[cl]) + up(z.s[cl]);
@@ -2269,7 +2285,9 @@ int psp_hip_profile_sweep(psp_hip_ctx* c, void* B, int k, psp_hip_kernel_stats* 
     int rc = CheckSolveArgs(c, B, k, 1);
     if (rc) return rc;
     if (!stats) return Fail(c, PSP_HIP_ERR_INVALID, "null stats");
-    if ((rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1)))) return rc;
+    if ((rc = EnsureFusedFactors(c, k)) ||
+        (rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1))))
+        return rc;
     MvProfile prof;
     HIPCHK(c, hipEventCreate(&prof.a));
     HIPCHK(c, hipEventCreate(&prof.b));
@@ -2295,7 +2313,9 @@ int psp_hip_solve_panel(psp_hip_ctx* c, void* B, int k, int panel)
     if (rc) return rc;
     if (panel < 0 || panel >= c->plan.geo.numPanels)
         return Fail(c, PSP_HIP_ERR_INVALID, "panel index out of range");
-    if ((rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1)))) return rc;
+    if ((rc = EnsureFusedFactors(c, k)) ||
+        (rc = EnsureWorkspace(c, k, std::max(1, c->wsK == k ? c->wsM : 1))))
+        return rc;
     if (c->desc.precision == PSP_HIP_FRONTS_FP32)
         PanelForward<float>(c, (c128*)B, k, panel);
     else

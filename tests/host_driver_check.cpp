@@ -1,9 +1,12 @@
 // The host side of the C ABI (psp_amd/csrc/psp_hip.cpp) against a HIP runtime
 // made of host memory, without a GPU:
-//   host_driver_check retry nx ny nz [precision]
+//   host_driver_check fused|oom|retry nx ny nz [precision]
 // The kernels' launch wrappers here compute nothing; they check that every
 // array they are given lies in live memory and is as large as the kernel needs,
 // and count.
+//  fused: which calls factor, allocate and run which panel solves when the
+//         fused launches are switched on after Initialize;
+//  oom:   the same without the memory for their layout;
 //  retry: Initialize after a first one whose n-th allocation failed, for
 //         every n.
 #include <sys/mman.h>
@@ -325,6 +328,70 @@ static Counts Of(const char* what, psp_hip_ctx* c, const F& call)
     return {factorizations - t.f, merged - t.m, fusedSolves - t.q, allocs - t.a, frees - t.r};
 }
 
+static void fused()
+{
+    psp_hip_ctx* c = Context();
+    need(Factor(c) == PSP_HIP_OK, "Initialize");
+    const int solves = 2 * psp_hip_num_panels(c) - 1;
+    const long once = factorizations;
+    psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 1);
+    void* B = block.data();
+    Counts n = Of("noalloc", c, [&] { return psp_hip_precondition_noalloc(c, B, 8); });
+    need(n.f == 0 && n.a == 0 && n.r == 0 && n.m == solves && n.q == 0, "noalloc", n.f, n.a);
+    n = Of("Multiply", c, [&] { return psp_hip_multiply(c, B, B, 8); });
+    need(n.f == 0 && n.a == 0, "Multiply", n.f, n.a);
+    n = Of("gradient", c, [&] { return psp_hip_adjoint_gradient(c, B, B, 8, vel.data(), 0); });
+    need(n.f == 0 && n.a == 0, "gradient", n.f, n.a);
+    for (int k : {3, 7, 17}) {  // the fused launches take 8 to 16
+        n = Of("sweep", c, [&] { return psp_hip_precondition(c, B, k); });
+        need(n.f == 0 && n.m == solves && n.q == 0, "sweep without fused launches", n.f, n.q);
+    }
+    n = Of("first fused sweep", c, [&] { return psp_hip_precondition(c, B, 8); });
+    need(n.f == once && n.q > 0, "factors in the fused layout", n.f, n.q);
+    n = Of("fused sweep", c, [&] { return psp_hip_precondition(c, B, 12); });
+    need(n.f == 0 && n.q > 0, "kept", n.f, n.q);
+    n = Of("noalloc", c, [&] { return psp_hip_precondition_noalloc(c, B, 8); });
+    need(n.f == 0 && n.a == 0 && n.r == 0 && n.q > 0, "noalloc, fused", n.a, n.q);
+    psp_hip_destroy(c);
+}
+
+static void oom()
+{
+    // (the workspace's are smaller without slices)
+    const size_t big = block.size() * sizeof(block[0]) * (desc.precision ? 1 : 2);
+    for (int n = 0;; ++n) {
+        psp_hip_ctx* c = Context();
+        psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_MAX_SPLIT, 1);
+        psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_MIN_TILES, 1);
+        psp_hip_set_option(c, PSP_HIP_OPT_SWEEP_GRAPH, 0);
+        need(Factor(c) == PSP_HIP_OK, "Initialize");
+        const int solves = 2 * psp_hip_num_panels(c) - 1;
+        const size_t resident = used;
+        psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 1);
+        void* B = block.data();
+        smallest = big;
+        failAt = n;
+        Counts t = Of("panel solve", c, [&] { return psp_hip_solve_panel(c, B, 9, 1); });
+        const bool failed = failAt < 0;
+        failAt = -1;
+        smallest = 0;
+        if (failed) {
+            need(t.f == 0 && t.m == 1 && t.q == 0, "merged solves serve", n, t.f);
+            t = Of("noalloc", c, [&] { return psp_hip_precondition_noalloc(c, B, 8); });
+            need(t.f == 0 && t.m == solves, "noalloc", n);
+            t = Of("Multiply", c, [&] { return psp_hip_multiply(c, B, B, 9); });
+            psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 0);  // frees the workspace
+            need(used == resident, "memory given back", n, (long)(used - resident));
+            psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 1);
+        }
+        t = Of("sweep", c, [&] { return psp_hip_precondition(c, B, 9); });
+        need((t.f > 0) == failed && t.q > 0, "fused solves with the memory back", n, t.f);
+        psp_hip_destroy(c);
+        if (!failed) break;
+        need(n < 20, "big allocations");
+    }
+}
+
 static void retry()
 {
     for (int n = 0;; ++n) {
@@ -362,7 +429,11 @@ int main(int argc, char** argv)
     vel.assign(N, 2.0);
     block.assign(N * 32, {1.0, 0.0});
     const std::string mode = argv[1];
-    if (mode == "retry")
+    if (mode == "fused")
+        fused();
+    else if (mode == "oom")
+        oom();
+    else if (mode == "retry")
         retry();
     else
         return 2;

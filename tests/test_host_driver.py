@@ -1,8 +1,10 @@
 """The host side of the C ABI (psp_amd/csrc/psp_hip.cpp) without a GPU, by
 tests/host_driver_check.cpp: built here with the address and undefined sanitizers
 against a HIP runtime of host memory, whose kernels compute nothing and check
-that their arrays are live and large enough.  Initialize after one that ran out of memory at any
-of its allocations."""
+that their arrays are live and large enough.  Which calls factor and allocate
+when the fused launches are switched on after Initialize, with the memory for
+their layout and without it, and Initialize after one that ran out of memory at
+any of its allocations."""
 import os
 import subprocess
 
@@ -28,7 +30,8 @@ def checker(tmp_path_factory):
 
 # mode nx ny nz [precision]
 @pytest.mark.parametrize("args", [
-    "retry 14 13 24", "retry 9 13 27 1",
+    "fused 24 22 30", "fused 40 40 24 1", "oom 24 22 30", "oom 24 22 30 1", "retry 14 13 24",
+    "retry 9 13 27 1",
 ])
 def test_host_driver(checker, args):
     out = subprocess.run([checker] + args.split(), capture_output=True, text=True, timeout=300)
