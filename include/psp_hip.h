@@ -58,8 +58,8 @@ enum {
                                         as many (default 256) */
     PSP_HIP_OPT_SOLVE_MAX_SPLIT = 3, /* most inner slices a tile is cut into, in
                                         quarters (default 8: 32 slices) */
-    PSP_HIP_OPT_SOLVE_WIDE_WG = 4,   /* accepted, without effect on the merged solves */
-    PSP_HIP_OPT_SOLVE_PERSIST = 5,   /* accepted, without effect on the merged solves */
+    PSP_HIP_OPT_SOLVE_WIDE_WG = 4,   /* accepted, without effect */
+    PSP_HIP_OPT_SOLVE_PERSIST = 5,   /* accepted, without effect */
     PSP_HIP_OPT_SOLVE_PERSIST_GRID = 6, /* accepted (>= 0), without effect */
     PSP_HIP_OPT_SOLVE_FUSED = 7,       /* 1: for 8 <= k <= 16, the tree levels from
                                           the cut depth down run as one persistent

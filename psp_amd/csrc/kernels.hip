@@ -623,8 +623,7 @@ __global__ void k_xcc_probe(int32_t* out)
 // Without redc a reduce launch follows.  Tiles with no rows are holes in that
 // placement and exit at once.
 //
-// MvmTile is the work of one workgroup on tile tl (nrows > 0); k_mvm runs it
-// on one panel solve's tiles, k_mvm_batch on the tiles of many.
+// MvmTile is the work of one workgroup on tile tl (nrows > 0).
 template <typename T, int PH, int RT, int KB>
 __device__ __forceinline__ void MvmTile(const SolveTile tl, const int32_t* structs,
                                         const Slots<T> gs, const cx<T>* L, const cx<T>* LT,

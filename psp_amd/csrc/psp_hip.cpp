@@ -2040,6 +2040,8 @@ int psp_hip_set_option(psp_hip_ctx* c, int option, int value)
         for (auto& D : c->dev) SetSliceReduce(c, D);
         return PSP_HIP_OK;
     }
+    if (option == PSP_HIP_OPT_SOLVE_WIDE_WG || option == PSP_HIP_OPT_SOLVE_PERSIST)
+        return PSP_HIP_OK;  // every workgroup has 4 waves and one tile
     if (option == PSP_HIP_OPT_SOLVE_PERSIST_GRID) {  // no launch is persistent any more
         if (value < 0) return Fail(c, PSP_HIP_ERR_INVALID, "persistent grid cap must be >= 0");
         return PSP_HIP_OK;
@@ -2068,13 +2070,8 @@ int psp_hip_set_option(psp_hip_ctx* c, int option, int value)
         }
         return RebuildSolveTiles(c);
     }
-    if (option == PSP_HIP_OPT_SOLVE_MIN_TILES || option == PSP_HIP_OPT_SOLVE_MAX_SPLIT ||
-        option == PSP_HIP_OPT_SOLVE_WIDE_WG || option == PSP_HIP_OPT_SOLVE_PERSIST) {
-        if (option == PSP_HIP_OPT_SOLVE_WIDE_WG) {
-            c->plan.wideWg = value != 0;
-        } else if (option == PSP_HIP_OPT_SOLVE_PERSIST) {
-            c->plan.persist = value != 0;
-        } else if (option == PSP_HIP_OPT_SOLVE_MIN_TILES) {
+    if (option == PSP_HIP_OPT_SOLVE_MIN_TILES || option == PSP_HIP_OPT_SOLVE_MAX_SPLIT) {
+        if (option == PSP_HIP_OPT_SOLVE_MIN_TILES) {
             if (value < 1 || value > (1 << 20))
                 return Fail(c, PSP_HIP_ERR_INVALID, "solve min tiles out of range");
             c->plan.minTiles = value;
@@ -2085,8 +2082,7 @@ int psp_hip_set_option(psp_hip_ctx* c, int option, int value)
         }
         for (int cl = 0; cl < 3; ++cl)
             if (c->plan.present[cl]) {
-                DefaultSolveShapes(c->plan.cls[cl], c->plan.minTiles, c->plan.maxSplit,
-                                   c->plan.wideWg, c->plan.persist);
+                DefaultSolveShapes(c->plan.cls[cl], c->plan.minTiles, c->plan.maxSplit);
                 DefaultSlices(c->plan.cls[cl], c->plan.minTiles, c->plan.maxSplit);
             }
         return RebuildSolveTiles(c);

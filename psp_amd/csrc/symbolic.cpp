@@ -552,7 +552,7 @@ void Schedule(const Plan& plan, ClassPlan& C)
 
     // Solve schedule.
     {
-        DefaultSolveShapes(C, plan.minTiles, plan.maxSplit, plan.wideWg, plan.persist);
+        DefaultSolveShapes(C, plan.minTiles, plan.maxSplit);
         BuildSolveTiles(C);
         BuildQueues(C, plan.fused ? plan.fusedQueues : 0, plan.fusedRows, plan.fusedCut,
                     plan.fusedWgPerQueue);
@@ -634,23 +634,19 @@ int64_t RowBlocks(const ClassPlan& C, int d, int ph, int rows)
 
 }  // namespace
 
-void DefaultSolveShapes(ClassPlan& C, int minTiles, int maxSplit, bool wideWg, bool persist)
+void DefaultSolveShapes(ClassPlan& C, int minTiles, int maxSplit)
 {
     C.shapes.assign(C.maxDepth + 1, {});
     for (int d = 0; d <= C.maxDepth; ++d)
         for (int ph = 0; ph < 2; ++ph) {
-            SolveShape sh{16, 1, 4, persist ? 1 : 0};
+            SolveShape sh{16, 1};
             for (int cand : {64, 32, 16}) {
                 sh.rows = cand;
                 if (RowBlocks(C, d, ph, cand) >= minTiles) break;
             }
             const int64_t t = RowBlocks(C, d, ph, sh.rows);
-            if (t > 0 && t < minTiles) {
-                if (wideWg && !persist)
-                    sh.waves = 16;
-                else
-                    sh.split = (int)std::min<int64_t>(maxSplit, CeilDiv(minTiles, t));
-            }
+            if (t > 0 && t < minTiles)
+                sh.split = (int)std::min<int64_t>(maxSplit, CeilDiv(minTiles, t));
             C.shapes[d][ph] = sh;
         }
 }
@@ -670,8 +666,6 @@ void BuildSolveTiles(ClassPlan& C)
     auto build = [&](int d, int ph, ClassPlan::Range& rg) {
         const SolveShape sh = C.shapes[d][ph];
         rg.rows = sh.rows;
-        rg.waves = sh.waves;
-        rg.persist = sh.persist;
         rg.start = (int)C.mv.size();
         rg.rstart = (int)C.mvred.size();
         int slots = 0;
@@ -725,7 +719,7 @@ void BuildSolveTiles(ClassPlan& C)
     // positions a residue leaves free are holes (tiles with no rows).
     auto place = [&](ClassPlan::Range& rg) {
         rg.xcd = 0;
-        if (rg.persist || rg.rcount <= 0) return;
+        if (rg.rcount <= 0) return;
         std::vector<std::vector<MvTile>> lane(8);
         for (int i = rg.start; i < rg.start + rg.count;) {
             int j = i + 1;

@@ -303,8 +303,8 @@ class DistHelmholtz:
                          fused_cut=None, fused_wg=None, xcd_reduce=None):
         """Default front-solve tiles: workgroups wanted per launch and the
         most inner slices per tile (in quarters); rebuilds the solve tiles.
-        wide_wg, persist and persist_grid are accepted and change nothing in
-        the merged solves.  fused: the tree levels from the
+        wide_wg, persist and persist_grid are accepted and change nothing.
+        fused: the tree levels from the
         cut depth down as one persistent launch per direction (8 <= k <= 16),
         with fused_queues subtree queues (one per XCD; more leave queues the
         last workgroup runs alone), fused_rows output rows per tile and the

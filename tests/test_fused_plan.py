@@ -40,3 +40,12 @@ def test_fused_work_lists(checker, args):
     assert out.returncode == 0, out.stdout + out.stderr
     assert "class 0: cut" in out.stdout and "levels placed per XCD" in out.stdout
     assert "class 0: updates in two regions" in out.stdout
+
+
+@pytest.mark.parametrize("args", ["100 100 100", "40 40 24 8 32 -1 64 1 16"])
+def test_split_levels_are_placed_by_default(checker, args):
+    # the levels above the cut sum their slices in the product launch
+    out = subprocess.run([checker] + args.split(), capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    placed = [int(line.split()[2]) for line in out.stdout.splitlines() if "placed per XCD" in line]
+    assert placed and min(placed) > 0

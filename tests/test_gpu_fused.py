@@ -123,3 +123,21 @@ def test_fused_solve_matches_oracle(torch_cuda):
     rep = h.Solve(Bd, 20, 1e-8)
     assert rep.status == 0 and rep.iterations == rep_o.iterations
     assert _rel(Bd.cpu().numpy(), xo) < 1e-10
+
+
+@pytest.mark.parametrize("k", [8, 13, 16])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_levels_above_the_cut_sum_their_slices(torch_cuda, precision, k):
+    """Row blocks cut into slices at the levels above the cut: summed in the
+    product launch, bitwise as by the reduce launch."""
+    torch = torch_cuda
+    disc, vel = _problem(40, 40, 24)
+    X = rand_block(np.random.default_rng(160 + k), disc.nx * disc.ny * disc.nz, k)
+    tiling = dict(min_tiles=4096, max_split=16, fused_cut=5)
+    on = _sweep(torch, _helm(disc, vel, precision, **tiling), X)
+    off = _sweep(torch, _helm(disc, vel, precision, xcd_reduce=0, **tiling), X)
+    assert np.array_equal(on, off)
+    if precision == "fp64":
+        o = _oracle(disc, vel)
+        l2n = o.local_to_natural()
+        assert _rel(on[l2n], o.precondition(X[l2n])) < 1e-10
