@@ -3328,10 +3328,10 @@ void LaunchPanelSolveFused(const ClassDev& c, const ClassPlan& plan, int b, void
 }
 
 template <typename T>
-void LaunchPack(const ClassDev& c, hipStream_t s)
+void LaunchPack(const ClassDev& c, int start, int count, hipStream_t s)
 {
-    if (c.npacks <= 0) return;
-    hipLaunchKernelGGL((k_pack<T>), dim3(c.npacks, c.npanels), dim3(kThreads), 0, s, c.packs,
+    if (count <= 0) return;
+    hipLaunchKernelGGL((k_pack<T>), dim3(count, c.npanels), dim3(kThreads), 0, s, c.packs + start,
                        c.foldNodes, c.browBase, (const cx<T>*)c.L, c.fstore, (const cx<T>*)c.U,
                        c.ustore, (cx<T>*)c.F, c.fentries);
 }
@@ -3589,7 +3589,7 @@ void LaunchAdjointGrad(const StencilArgs& st, const c128* u, const c128* lam, in
                                       hipStream_t, MvProfile*, int, int);                         \
     template void LaunchPanelSolveFused<T>(const ClassDev&, const ClassPlan&, int, void*, void*,  \
                                            void*, void*, int, hipStream_t, MvProfile*, int32_t*); \
-    template void LaunchPack<T>(const ClassDev&, hipStream_t);                                    \
+    template void LaunchPack<T>(const ClassDev&, int, int, hipStream_t);                          \
     template void LaunchCompose<T>(const ClassDev&, int, int, hipStream_t);                       \
     template void LaunchTransposeScale<T>(const ClassDev&, hipStream_t);                          \
     template void LaunchFoldBack<T>(const ClassDev&, hipStream_t);                                \

@@ -111,7 +111,6 @@ struct ClassDev {
     int32_t *browBase = nullptr, *flist = nullptr, *fsrc = nullptr;
     FoldNode* foldNodes = nullptr;
     TransItem* packs = nullptr;
-    int npacks = 0;
     ComposeDesc* compose = nullptr;
     ComposeKey* fkeys = nullptr;
     GemmTile* composeTiles = nullptr;
@@ -216,10 +215,10 @@ template <typename T>
 void LaunchPanelSolveFused(const ClassDev& c, const ClassPlan& plan, int b, void* Xp, void* W,
                            void* P, void* G, int k, hipStream_t s, MvProfile* prof, int32_t* sync);
 bool FusedApplies(const ClassDev& c, const ClassPlan& plan, int k, int64_t eb);
-// Fold of the factored fronts into F: the copied pieces, then the composed
-// columns of one depth below the groups' tops.
+// Fold of the factored fronts of a depth group into F: the copied pieces, then
+// the composed columns of one depth below the group's tops.
 template <typename T>
-void LaunchPack(const ClassDev& c, hipStream_t s);
+void LaunchPack(const ClassDev& c, int start, int count, hipStream_t s);
 template <typename T>
 void LaunchCompose(const ClassDev& c, int tileStart, int tileCount, hipStream_t s);
 template <typename T>

@@ -55,7 +55,7 @@ struct psp_hip_ctx {
     int wsK = 0, wsM = 0;
     std::vector<void*> wsAllocs;
     int64_t wsSlots = 0;  // partial-sum slots the workspace holds
-    std::vector<void*> facAllocs;  // Schur-complement and inversion scratch, only while factoring
+    std::vector<void*> facAllocs;  // scratch of updates, inverses and E, only while factoring
     std::vector<void*> facStore;   // factors of every panel, from Initialize to Finalize
     bool facFused = false;         // the factors include those of the fused launches
     void* vec[3] = {nullptr, nullptr, nullptr};  // per class: the solve vector (VecRows)
@@ -348,10 +348,10 @@ int EnsureDevice(psp_hip_ctx* c)
         D.npanels = (int)c->classPanels[cl].size();
         D.fstore = P.fstore;
         // the update scratch also holds the fold's E (read one entry past it)
-        D.ustore = std::max(P.ustore, P.estore + 1);
+        // and, with its own stride, the inversion's T
+        D.ustore = std::max({P.ustore, P.estore + 1, P.tstore});
         D.xrows = P.xrows;
         D.fentries = (int64_t)(P.nblocks + 1) * kBlk * kBlk;  // and a block of zeros
-        D.npacks = (int)P.packs.size();
         D.tstore = P.tstore;
         D.wstore = P.wstore;
         D.ninv = (int)P.inv.size();
@@ -762,12 +762,15 @@ int FactorClasses(psp_hip_ctx* c, double* tFill, double* tLdl, double* tInv, dou
         HIPCHK(c, mark(2));
         LaunchInvDiag<T>(D, nb, s);
         for (const GemmLaunch& gl : P.invGemm) LaunchGemm<T>(D, gl.tileStart, gl.tileCount, s);
-        // merged fronts: E = -L_BL Linv per node, copied pieces, then the
-        // columns of the nodes below the groups' tops, depth by depth
-        LaunchGemm<T>(D, P.foldE.tileStart, P.foldE.tileCount, s);
-        LaunchPack<T>(D, s);
-        for (const GemmLaunch& gl : P.composeSteps)
-            LaunchCompose<T>(D, gl.tileStart, gl.tileCount, s);
+        // merged fronts, a depth group at a time: E = -L_BL Linv per node, copied
+        // pieces, then the columns of the nodes below the group's tops, depth by
+        // depth
+        for (const ClassPlan::FoldGroup& f : P.foldGroups) {
+            LaunchGemm<T>(D, f.e.tileStart, f.e.tileCount, s);
+            LaunchPack<T>(D, f.packStart, f.packCount, s);
+            for (int i = f.stepStart; i < f.stepStart + f.stepCount; ++i)
+                LaunchCompose<T>(D, P.composeSteps[i].tileStart, P.composeSteps[i].tileCount, s);
+        }
         if (c->plan.fused) {
             // layout of the fused launches: LT[:, :s] = Linv^T D^-1, LT[:, s:] =
             // (-L_BL Linv)^T, then L_BL = -L_BL Linv and a unit diagonal in L
@@ -809,13 +812,14 @@ int Factor(psp_hip_ctx* c, double t[4])
     const size_t storage = c->facStore.size();
     int st = EnsureFactorStorage(c);
     // The Schur-complement (U) and inversion (T) scratch lives only while
-    // factoring, so that many factored problems fit in HBM at once.
+    // factoring, so that many factored problems fit in HBM at once.  The inversion
+    // follows the last update and the fold's E the inversion: one array serves all.
     const size_t eb = FrontBytes(c);
     for (int cl = 0; cl < 3; ++cl) {
         if (st || !c->plan.present[cl]) continue;
         ClassDev& D = c->dev[cl];
         st = Alloc(c, &D.U, eb * (size_t)D.npanels * D.ustore, c->facAllocs);
-        if (!st) st = Alloc(c, &D.T, eb * (size_t)D.npanels * D.tstore, c->facAllocs);
+        D.T = D.U;
     }
     if (st) {  // the factors of an earlier call stay as they are
         FreeFactorScratch(c);

@@ -1093,48 +1093,57 @@ bool LayMerged(ClassPlan& C, int tile)
                                              : (int32_t)(V.g0 + p.u0 + r - kBlk * p.sb);
         }
     }
-    // fold: E = -L_BL Linv per node, top blocks and the tops' E copied,
-    // the other nodes' columns composed from their ancestors'
+    // fold, group by group: E = -L_BL Linv per node, top blocks and the tops' E
+    // copied, the other nodes' columns composed from their ancestors'
     C.foldNodes.assign(nn, FoldNode{});
     C.packs.clear();
     C.estore = 0;
-    C.foldE.tileStart = (int)C.tiles.size();
-    for (int t = 0; t < nn; ++t) {
-        const Node& n = C.nodes[t];
-        FoldNode& f = C.foldNodes[t];
-        f.l = n.loff;
-        f.e = C.estore;
-        f.s = n.size;
-        f.u = n.usize;
-        f.urow = -1;
-        if (n.size == 0) continue;
-        const BlockNode& b = C.bnodes[C.bnodeOf[t]];
-        f.mcol = mcol[t];
-        f.br0 = b.br0;
-        f.x0 = b.x0 + mcol[t];
-        if (b.top == t) f.urow = kBlk * b.sb;
-        C.estore += (int64_t)n.size * n.usize;
-        for (int j0 = 0; j0 < n.size; j0 += 32) {
-            for (int i0 = j0; i0 < n.size; i0 += 32) C.packs.push_back({t, i0, j0, 0});
-            if (b.top == t)
-                for (int i0 = 0; i0 < n.usize; i0 += 32) C.packs.push_back({t, n.size + i0, j0, 0});
+    C.foldGroups.assign(C.groups.size(), {});
+    for (size_t gr = 0; gr < C.groups.size(); ++gr) {
+        ClassPlan::FoldGroup& G = C.foldGroups[gr];
+        G.e.tileStart = (int)C.tiles.size();
+        G.packStart = (int)C.packs.size();
+        int64_t estore = 0;
+        for (int t = 0; t < nn; ++t) {
+            const Node& n = C.nodes[t];
+            if (groupOf[n.depth] != (int)gr) continue;
+            FoldNode& f = C.foldNodes[t];
+            f.l = n.loff;
+            f.e = estore;
+            f.s = n.size;
+            f.u = n.usize;
+            f.urow = -1;
+            if (n.size == 0) continue;
+            const BlockNode& b = C.bnodes[C.bnodeOf[t]];
+            f.mcol = mcol[t];
+            f.br0 = b.br0;
+            f.x0 = b.x0 + mcol[t];
+            if (b.top == t) f.urow = kBlk * b.sb;
+            estore += (int64_t)n.size * n.usize;
+            for (int j0 = 0; j0 < n.size; j0 += 32) {
+                for (int i0 = j0; i0 < n.size; i0 += 32) C.packs.push_back({t, i0, j0, 0});
+                if (b.top == t)
+                    for (int i0 = 0; i0 < n.usize; i0 += 32) C.packs.push_back({t, n.size + i0, j0, 0});
+            }
+            if (n.usize == 0) continue;
+            const int fs = n.size + n.usize;
+            GemmDesc g{};
+            g.a = n.loff + n.size;
+            g.b = n.loff;
+            g.c = f.e;
+            g.lda = g.ldb = fs;
+            g.ldc = n.usize;
+            g.M = n.usize;
+            g.N = g.K = n.size;
+            g.abuf = g.bbuf = g.dbuf = BUF_L;
+            g.cbuf = BUF_U;
+            g.flags = G_BUNIT | G_NEG | G_BETA0;
+            AddGemmTiles(C, g, tile);
         }
-        if (n.usize == 0) continue;
-        const int fs = n.size + n.usize;
-        GemmDesc g{};
-        g.a = n.loff + n.size;
-        g.b = n.loff;
-        g.c = f.e;
-        g.lda = g.ldb = fs;
-        g.ldc = n.usize;
-        g.M = n.usize;
-        g.N = g.K = n.size;
-        g.abuf = g.bbuf = g.dbuf = BUF_L;
-        g.cbuf = BUF_U;
-        g.flags = G_BUNIT | G_NEG | G_BETA0;
-        AddGemmTiles(C, g, tile);
+        G.e.tileCount = (int)C.tiles.size() - G.e.tileStart;
+        G.packCount = (int)C.packs.size() - G.packStart;
+        C.estore = std::max(C.estore, estore);
     }
-    C.foldE.tileCount = (int)C.tiles.size() - C.foldE.tileStart;
     C.flist.clear();
     C.fsrc.clear();
     C.compose.clear();
@@ -1142,57 +1151,63 @@ bool LayMerged(ClassPlan& C, int tile)
     C.composeTiles.clear();
     C.composeSteps.clear();
     std::vector<int> listOf(nn, -1), listLen(nn, 0), at;
-    for (int off = 1; off < kMaxGroup; ++off) {
-        GemmLaunch gl;
-        gl.tileStart = (int)C.composeTiles.size();
-        for (int c = 0; c < nn; ++c) {
-            const Node& n = C.nodes[c];
-            if (n.size == 0 || n.depth - C.nodes[top[c]].depth != off) continue;
-            const int m = C.bnodeOf[c], p = n.parent;
-            const BlockNode& b = C.bnodes[m];
-            if (listOf[p] < 0) {
-                listOf[p] = (int)C.flist.size();
-                for (int a = p;; a = C.nodes[a].parent) {
-                    for (int i = 0; i < C.nodes[a].size; ++i) C.flist.push_back(mcol[a] + i);
-                    if (a == b.top) break;
+    for (size_t gr = 0; gr < C.groups.size(); ++gr) {
+        ClassPlan::FoldGroup& G = C.foldGroups[gr];
+        G.stepStart = (int)C.composeSteps.size();
+        for (int off = 1; off < kMaxGroup; ++off) {
+            GemmLaunch gl;
+            gl.tileStart = (int)C.composeTiles.size();
+            for (int c = 0; c < nn; ++c) {
+                const Node& n = C.nodes[c];
+                if (n.size == 0 || n.depth != C.groups[gr][0] + off || n.depth > C.groups[gr][1])
+                    continue;
+                const int m = C.bnodeOf[c], p = n.parent;
+                const BlockNode& b = C.bnodes[m];
+                if (listOf[p] < 0) {
+                    listOf[p] = (int)C.flist.size();
+                    for (int a = p;; a = C.nodes[a].parent) {
+                        for (int i = 0; i < C.nodes[a].size; ++i) C.flist.push_back(mcol[a] + i);
+                        if (a == b.top) break;
+                    }
+                    for (int i = 0; i < b.u; ++i) C.flist.push_back(kBlk * b.sb + i);
+                    listLen[p] = (int)C.flist.size() - listOf[p];
                 }
-                for (int i = 0; i < b.u; ++i) C.flist.push_back(kBlk * b.sb + i);
-                listLen[p] = (int)C.flist.size() - listOf[p];
-            }
-            at.assign((size_t)kBlk * (b.sb + b.ub), -1);
-            for (int i = 0; i < listLen[p]; ++i) at[C.flist[listOf[p] + i]] = i;
-            ComposeDesc d{};
-            d.e = C.foldNodes[c].e;
-            d.lde = n.usize;
-            d.list = listOf[p];
-            d.rows = listLen[p];
-            d.br0 = b.br0;
-            d.piv = listLen[p] - b.u;
-            d.ccol = mcol[c];
-            d.n = n.size;
-            d.src = (int)C.fsrc.size();
-            C.fsrc.resize(C.fsrc.size() + listLen[p], -1);
-            for (int a = 0; a < n.usize; ++a) {
-                const int r = rowIn(m, C.structs[n.ustart + a]);
-                if (r < 0 || at[r] < 0) return false;
-                C.fsrc[d.src + at[r]] = a;
-            }
-            d.kl = (int)C.fkeys.size();
-            for (int i = 0; i < d.piv; ++i)
-                if (C.fsrc[d.src + i] >= 0)
-                    C.fkeys.push_back({C.flist[d.list + i], i, C.fsrc[d.src + i], 0});
-            d.k = (int)C.fkeys.size() - d.kl;
-            const int di = (int)C.compose.size();
-            C.compose.push_back(d);
-            for (int tn = 0; tn < d.n; tn += tile)
-                for (int tm = 0; tm < d.rows; tm += tile) {
-                    int32_t kend = 0;
-                    while (kend < d.k && C.fkeys[d.kl + kend].pos < tm + tile) ++kend;
-                    C.composeTiles.push_back({di, tm, tn, kend});
+                at.assign((size_t)kBlk * (b.sb + b.ub), -1);
+                for (int i = 0; i < listLen[p]; ++i) at[C.flist[listOf[p] + i]] = i;
+                ComposeDesc d{};
+                d.e = C.foldNodes[c].e;
+                d.lde = n.usize;
+                d.list = listOf[p];
+                d.rows = listLen[p];
+                d.br0 = b.br0;
+                d.piv = listLen[p] - b.u;
+                d.ccol = mcol[c];
+                d.n = n.size;
+                d.src = (int)C.fsrc.size();
+                C.fsrc.resize(C.fsrc.size() + listLen[p], -1);
+                for (int a = 0; a < n.usize; ++a) {
+                    const int r = rowIn(m, C.structs[n.ustart + a]);
+                    if (r < 0 || at[r] < 0) return false;
+                    C.fsrc[d.src + at[r]] = a;
                 }
+                d.kl = (int)C.fkeys.size();
+                for (int i = 0; i < d.piv; ++i)
+                    if (C.fsrc[d.src + i] >= 0)
+                        C.fkeys.push_back({C.flist[d.list + i], i, C.fsrc[d.src + i], 0});
+                d.k = (int)C.fkeys.size() - d.kl;
+                const int di = (int)C.compose.size();
+                C.compose.push_back(d);
+                for (int tn = 0; tn < d.n; tn += tile)
+                    for (int tm = 0; tm < d.rows; tm += tile) {
+                        int32_t kend = 0;
+                        while (kend < d.k && C.fkeys[d.kl + kend].pos < tm + tile) ++kend;
+                        C.composeTiles.push_back({di, tm, tn, kend});
+                    }
+            }
+            gl.tileCount = (int)C.composeTiles.size() - gl.tileStart;
+            if (gl.tileCount > 0) C.composeSteps.push_back(gl);
         }
-        gl.tileCount = (int)C.composeTiles.size() - gl.tileStart;
-        if (gl.tileCount > 0) C.composeSteps.push_back(gl);
+        G.stepCount = (int)C.composeSteps.size() - G.stepStart;
     }
     return true;
 }

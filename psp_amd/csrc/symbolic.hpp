@@ -213,7 +213,7 @@ static_assert(sizeof(BlockRed) == 64, "BlockRed is one 64-byte record");
 // Fold of one fine node into its merged front.
 struct FoldNode {
     int64_t l;           // factor offset (BUF_L), (s + u) x s
-    int64_t e;           // E = -L_BL Linv, u x s (in the update scratch)
+    int64_t e;           // E = -L_BL Linv, u x s (in the update scratch, of its depth group)
     int32_t s, u;
     int32_t mcol;        // first pivot within the merged front
     int32_t br0;         // the merged front's first block row
@@ -333,7 +333,7 @@ struct ClassPlan {
     int xrows = 0;                   // panel-vector rows in solve order, padding included
     int wrows = 0;                   // work rows
     int nblocks = 0;                 // 16 x 16 blocks of one panel's factor; block nblocks is zero
-    int64_t estore = 0;              // entries of all E of one panel
+    int64_t estore = 0;              // entries of all E of one panel, of the largest group
     std::vector<int32_t> sxy, sv;    // qxy, qv per panel-vector row (sv -1: padding)
     std::vector<int32_t> browBase, browLo;
     std::vector<int32_t> udst;       // vector row an update row is added into, see VecRows
@@ -343,9 +343,16 @@ struct ClassPlan {
     std::vector<ComposeDesc> compose;
     std::vector<ComposeKey> fkeys;
     std::vector<GemmTile> composeTiles;    // pad_: keys that meet the tile's rows
-    std::vector<GemmLaunch> composeSteps;  // by depth below the group's top, 1, 2, ...
+    std::vector<GemmLaunch> composeSteps;  // per group by depth below its top, 1, 2, ...
     std::vector<int32_t> flist, fsrc;
-    GemmLaunch foldE;                // E = -L_BL Linv
+    // The fold goes group by group, so that the update scratch holds the E of
+    // one group at a time: all of them at once were more than the updates of a
+    // level (7.8 against 7.3 GB at 100^3 in FP64, 39 against 33 at 200 x 200 x 100).
+    struct FoldGroup {
+        GemmLaunch e;                // E = -L_BL Linv
+        int packStart = 0, packCount = 0, stepStart = 0, stepCount = 0;
+    };
+    std::vector<FoldGroup> foldGroups;   // per depth group
     struct BlockLevel {              // one group: tiles and reduce items per direction
         int start[2] = {0, 0}, count[2] = {0, 0};
         int rstart[2] = {0, 0}, rcount[2] = {0, 0};

@@ -1,6 +1,6 @@
 // The host side of the C ABI (psp_amd/csrc/psp_hip.cpp) against a HIP runtime
 // made of host memory, without a GPU:
-//   host_driver_check fused|oom|retry nx ny nz [precision]
+//   host_driver_check fused|oom|retry|memory nx ny nz [precision]
 // The kernels' launch wrappers here compute nothing; they check that every
 // array they are given lies in live memory and is as large as the kernel needs,
 // and count.
@@ -8,9 +8,11 @@
 //         fused launches are switched on after Initialize;
 //  oom:   the same without the memory for their layout;
 //  retry: Initialize after a first one whose n-th allocation failed, for
-//         every n.
+//         every n;
+//  memory: the most memory that Initialize holds.
 #include <sys/mman.h>
 
+#include <algorithm>
 #include <complex>
 #include <cstdio>
 #include <cstdlib>
@@ -34,7 +36,7 @@ static void need(bool ok, const char* what, long a = 0, long b = 0)
 
 // ---- device memory -----------------------------------------------------------
 static std::map<char*, size_t> live;
-static size_t used = 0, smallest = 0;
+static size_t used = 0, most = 0, smallest = 0;
 static long allocs = 0, frees = 0, failAt = -1;  // failAt: allocations (of at least
                                                  // `smallest` bytes) until one fails
 static hipError_t lastError = hipSuccess;
@@ -63,6 +65,7 @@ hipError_t hipMalloc(void** p, size_t n)
     if (*p == MAP_FAILED) std::abort();
     live[(char*)*p] = n;
     used += n;
+    most = std::max(most, used);
     return hipSuccess;
 }
 hipError_t hipFree(void* p)
@@ -188,7 +191,7 @@ void LaunchGemm(const ClassDev& c, int, int n, hipStream_t)
 template <typename T>
 void LaunchInvDiag(const ClassDev& c, int, hipStream_t) { Factors<T>(c, false); }
 template <typename T>
-void LaunchPack(const ClassDev& c, hipStream_t)
+void LaunchPack(const ClassDev& c, int, int, hipStream_t)
 {
     Factors<T>(c, true);
     Live(c.F, Eb<T>(c) * c.fentries, "F");
@@ -280,7 +283,7 @@ BOTH(LaunchLdlDiag, const ClassDev&, int, int, int, hipStream_t)
 BOTH(LaunchLdlTrsm, const ClassDev&, int, int, int, hipStream_t)
 BOTH(LaunchGemm, const ClassDev&, int, int, hipStream_t)
 BOTH(LaunchInvDiag, const ClassDev&, int, hipStream_t)
-BOTH(LaunchPack, const ClassDev&, hipStream_t)
+BOTH(LaunchPack, const ClassDev&, int, int, hipStream_t)
 BOTH(LaunchCompose, const ClassDev&, int, int, hipStream_t)
 BOTH(LaunchTransposeScale, const ClassDev&, hipStream_t)
 BOTH(LaunchFoldBack, const ClassDev&, hipStream_t)
@@ -408,6 +411,51 @@ static void retry()
     }
 }
 
+// Bytes of the factors of all panels as two plain copies, and of the scratch of
+// their updates and inverses.
+static void plainSizes(double* factors, double* scratch)
+{
+    Plan plan;
+    std::string msg;
+    if (BuildPlan(desc, plan, msg) != PSP_HIP_OK) std::exit(2);
+    const double eb = desc.precision == PSP_HIP_FRONTS_FP32 ? 8 : 16;
+    *factors = *scratch = 0;
+    std::vector<int> panels(3, 0);
+    for (int p = 0; p < plan.geo.numPanels; ++p) ++panels[plan.geo.cls(p)];
+    for (int cl = 0; cl < 3; ++cl) {
+        if (!plan.present[cl]) continue;
+        const ClassPlan& C = plan.cls[cl];
+        *factors += 2 * eb * panels[cl] * C.fstore;
+        *scratch += eb * panels[cl] * (C.ustore + C.tstore);
+        // the pieces of a depth group's E do not overlap
+        for (const auto& g : C.groups) {
+            std::vector<std::pair<int64_t, int64_t>> e;
+            for (size_t t = 0; t < C.nodes.size(); ++t)
+                if (C.nodes[t].depth >= g[0] && C.nodes[t].depth <= g[1] && C.nodes[t].size > 0)
+                    e.push_back({C.foldNodes[t].e, (int64_t)C.nodes[t].size * C.nodes[t].usize});
+            std::sort(e.begin(), e.end());
+            for (size_t i = 0; i < e.size(); ++i)
+                need(e[i].first + e[i].second <= (i + 1 < e.size() ? e[i + 1].first : C.estore),
+                     "E", cl, (long)i);
+        }
+    }
+}
+
+static void memory()
+{
+    double factors, scratch;
+    plainSizes(&factors, &scratch);
+    psp_hip_ctx* c = Context();
+    need(Factor(c) == PSP_HIP_OK && Factor(c) == PSP_HIP_OK, "Initialize");
+    const double peak = (double)most;
+    psp_hip_finalize(c);
+    const double plan = (double)used;
+    std::printf("GB: at most %.2f, as plain copies %.2f\n", (peak - plan) / 1e9, (factors + scratch) / 1e9);
+    need(peak - plan <= factors + scratch, "memory of Initialize");
+    psp_hip_destroy(c);
+    need(used == 0, "given back", (long)used);
+}
+
 int main(int argc, char** argv)
 {
     if (argc < 5) return 2;
@@ -435,6 +483,8 @@ int main(int argc, char** argv)
         oom();
     else if (mode == "retry")
         retry();
+    else if (mode == "memory")
+        memory();
     else
         return 2;
     std::printf("%s: %ld allocations, %ld factorizations\n", mode.c_str(), allocs, factorizations);
