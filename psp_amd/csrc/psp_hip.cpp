@@ -58,6 +58,9 @@ struct psp_hip_ctx {
     std::vector<void*> facAllocs;  // scratch of updates, inverses and E, only while factoring
     std::vector<void*> facStore;   // factors of every panel, from Initialize to Finalize
     bool facFused = false;         // the factors include those of the fused launches
+    int device = -1;
+    bool sharedL = false, userL = false;     // SharedL: in use by this factorization, counted
+    bool tempL[3] = {false, false, false};   // per class: L is scratch
     void* vec[3] = {nullptr, nullptr, nullptr};  // per class: the solve vector (VecRows)
     void* P = nullptr;  // partial sums of split output blocks (64 rows x k per slot)
     // fused subtree launches only
@@ -115,13 +118,82 @@ int Upload(psp_hip_ctx* c, X** dst, const std::vector<X>& src)
     return PSP_HIP_OK;
 }
 
+constexpr int kMaxDevices = 64;
+
+// L, the plain factorization, is dead once F is folded from it, unless the fused
+// launches read it.  The factorizations of a device use one array for it, in turn,
+// which stays until no context of the device has factors any more or an allocation
+// needs its memory (allocating it for each would be 0.9 ms to 16 GB, but 28 ms a GB
+// in hipFree past that).  One that runs beside another, on another thread, takes
+// scratch of its own.
+struct SharedL {
+    void* p = nullptr;
+    size_t bytes = 0;
+    bool busy = false;
+    int users = 0;  // contexts with factors
+};
+std::mutex gLMutex;
+SharedL gL[kMaxDevices];
+
+bool DropIdle(SharedL& s)
+{
+    if (!s.p || s.busy) return false;
+    (void)hipFree(s.p);
+    s.p = nullptr;
+    s.bytes = 0;
+    return true;
+}
+
+hipError_t Malloc(psp_hip_ctx* c, void** p, size_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory || c->device < 0) return e;
+    {
+        std::lock_guard<std::mutex> lock(gLMutex);
+        if (!DropIdle(gL[c->device])) return e;
+    }
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
 int Alloc(psp_hip_ctx* c, void** p, size_t bytes, std::vector<void*>& list)
 {
     *p = nullptr;
     if (bytes == 0) bytes = 16;
-    HIPCHK(c, hipMalloc(p, bytes));
+    HIPCHK(c, Malloc(c, p, bytes));
     list.push_back(*p);
     return PSP_HIP_OK;
+}
+
+// Scratch for L until FreeFactorScratch.
+int TakeL(psp_hip_ctx* c, void** p, size_t bytes)
+{
+    {
+        std::lock_guard<std::mutex> lock(gLMutex);
+        SharedL& s = gL[c->device];
+        if (!s.busy) {
+            if (s.bytes < bytes) {
+                (void)DropIdle(s);
+                HIPCHK(c, hipMalloc(&s.p, bytes));
+                s.bytes = bytes;
+            }
+            s.busy = c->sharedL = true;
+            *p = s.p;
+            return PSP_HIP_OK;
+        }
+    }
+    return Alloc(c, p, bytes, c->facAllocs);
+}
+
+// Counts the context among SharedL's users while it has factors.
+void CountUser(psp_hip_ctx* c)
+{
+    if (c->userL == !c->facStore.empty()) return;
+    std::lock_guard<std::mutex> lock(gLMutex);
+    SharedL& s = gL[c->device];
+    c->userL = !c->userL;
+    s.users += c->userL ? 1 : -1;
+    if (s.users == 0) (void)DropIdle(s);
 }
 
 // PML profiles (initialize_finalize.hpp:415-525).
@@ -265,7 +337,6 @@ int UploadTiles(psp_hip_ctx* c, int cl);
 constexpr size_t kScratchBytes = size_t(64) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-constexpr int kMaxDevices = 64;
 std::mutex gScratchMutex;
 void* gScratchAddr[kMaxDevices] = {};
 
@@ -297,6 +368,10 @@ int EnsureDevice(psp_hip_ctx* c)
         HIPCHK(c, hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking));
         c->stream = c->own;
     }
+    int dev = 0, cus = 0;
+    HIPCHK(c, hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) return Fail(c, PSP_HIP_ERR_HIP, "device index out of range");
+    c->device = dev;
     c->xcdOk = XcdDealing(c);
     const Geometry& g = c->plan.geo;
     c->classPanels.assign(3, {});
@@ -332,8 +407,6 @@ int EnsureDevice(psp_hip_ctx* c)
     if ((st = Alloc(c, &vp, sizeof(double) * (size_t)d.nx * d.ny * d.nz, c->allocs))) return st;
     c->vel = (double*)vp;
 
-    int dev = 0, cus = 0;
-    HIPCHK(c, hipGetDevice(&dev));
     HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     if ((st = ScratchAddress(c, &c->scratch))) return st;
     PrimeSolveOccupancy();
@@ -426,11 +499,12 @@ void FreeFactorStorageFrom(psp_hip_ctx* c, size_t keep)
                 if (*q == p) *q = nullptr;
         (void)hipFree(p);
     }
+    CountUser(c);
 }
 
 // Factor storage, allocated by the first Initialize after construction or
-// Finalize and kept until Finalize: L (the factorization), F (the merged
-// solves) and, for the fused subtree launches, LT.
+// Finalize and kept until Finalize: F (the merged solves) and, for the fused
+// subtree launches, L and LT.
 int EnsureFactorStorage(psp_hip_ctx* c)
 {
     const size_t eb = FrontBytes(c);
@@ -451,14 +525,15 @@ int EnsureFactorStorage(psp_hip_ctx* c)
         const size_t body = eb * (size_t)D.npanels * D.fstore;
         const size_t fb = body + eb * (size_t)kSolvePad * maxFs;
         int st;
-        // only the padding needs zeroing here: every factorization zeroes L
-        // before assembly
-        if (!D.L && (st = add(&D.L, body, fb))) return st;
         // entries of F that no fold writes (padding of the blocks) stay zero
         if (!D.F && (st = add(&D.F, 0, eb * (size_t)D.npanels * D.fentries))) return st;
-        // the fold writes every entry of LT
-        if (c->plan.fused && !D.LT && (st = add(&D.LT, body, fb))) return st;
+        if (!c->plan.fused) continue;
+        // only the padding needs zeroing here: every factorization zeroes L
+        // before assembly, and the fold writes every entry of LT
+        if (!D.L && (st = add(&D.L, body, fb))) return st;
+        if (!D.LT && (st = add(&D.LT, body, fb))) return st;
     }
+    CountUser(c);
     return PSP_HIP_OK;
 }
 
@@ -485,6 +560,12 @@ void FreeFactorScratch(psp_hip_ctx* c)
     for (int cl = 0; cl < 3; ++cl) {
         c->dev[cl].U = nullptr;
         c->dev[cl].T = nullptr;
+        if (c->tempL[cl]) c->dev[cl].L = nullptr;
+        c->tempL[cl] = false;
+    }
+    if (c->sharedL) {
+        std::lock_guard<std::mutex> lock(gLMutex);
+        c->sharedL = gL[c->device].busy = false;
     }
 }
 
@@ -815,6 +896,20 @@ int Factor(psp_hip_ctx* c, double t[4])
     // factoring, so that many factored problems fit in HBM at once.  The inversion
     // follows the last update and the fold's E the inversion: one array serves all.
     const size_t eb = FrontBytes(c);
+    auto bytesL = [&](int cl) {
+        const ClassDev& D = c->dev[cl];
+        if (!c->plan.present[cl] || D.L) return (size_t)0;
+        return (eb * (size_t)D.npanels * D.fstore + 255) / 256 * 256;
+    };
+    const size_t l[3] = {bytesL(0), bytesL(1), bytesL(2)};
+    void* base = nullptr;
+    if (!st && l[0] + l[1] + l[2] > 0) st = TakeL(c, &base, l[0] + l[1] + l[2]);
+    for (int cl = 0; cl < 3 && !st; ++cl)
+        if (l[cl] > 0) {
+            c->dev[cl].L = base;
+            c->tempL[cl] = true;
+            base = (char*)base + l[cl];
+        }
     for (int cl = 0; cl < 3; ++cl) {
         if (st || !c->plan.present[cl]) continue;
         ClassDev& D = c->dev[cl];
@@ -832,15 +927,14 @@ int Factor(psp_hip_ctx* c, double t[4])
     st = c->desc.precision == PSP_HIP_FRONTS_FP32
              ? FactorClasses<float>(c, &t[0], &t[1], &t[2], &t[3])
              : FactorClasses<double>(c, &t[0], &t[1], &t[2], &t[3]);
-    if (st) {
-        (void)hipStreamSynchronize(c->stream);
+    // (the scratch is another context's next)
+    const hipError_t done = hipStreamSynchronize(c->stream);
+    if (st || done != hipSuccess)
         for (hipStream_t x : c->side)
             if (x) (void)hipStreamSynchronize(x);
-        FreeFactorScratch(c);
-        return st;
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     FreeFactorScratch(c);
+    if (st) return st;
+    HIPCHK(c, done);
     c->factored = true;
     c->facFused = c->plan.fused;
     return PSP_HIP_OK;

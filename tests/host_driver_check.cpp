@@ -1,6 +1,6 @@
 // The host side of the C ABI (psp_amd/csrc/psp_hip.cpp) against a HIP runtime
 // made of host memory, without a GPU:
-//   host_driver_check fused|oom|retry|memory nx ny nz [precision]
+//   host_driver_check fused|oom|retry|memory|several nx ny nz [precision]
 // The kernels' launch wrappers here compute nothing; they check that every
 // array they are given lies in live memory and is as large as the kernel needs,
 // and count.
@@ -9,16 +9,21 @@
 //  oom:   the same without the memory for their layout;
 //  retry: Initialize after a first one whose n-th allocation failed, for
 //         every n;
-//  memory: the most memory that Initialize holds.
+//  memory: the most memory that Initialize holds;
+//  several: what several factored contexts hold.
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <complex>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "kernels.hpp"
@@ -36,9 +41,11 @@ static void need(bool ok, const char* what, long a = 0, long b = 0)
 
 // ---- device memory -----------------------------------------------------------
 static std::map<char*, size_t> live;
-static size_t used = 0, most = 0, smallest = 0;
+static size_t used = 0, most = 0, smallest = 0, capacity = (size_t)-1;
 static long allocs = 0, frees = 0, failAt = -1;  // failAt: allocations (of at least
-                                                 // `smallest` bytes) until one fails
+                                                 // `smallest` bytes) until all fail
+static bool failed = false;
+static std::mutex mu;
 static hipError_t lastError = hipSuccess;
 
 static hipError_t Set(hipError_t e)
@@ -49,6 +56,7 @@ static hipError_t Set(hipError_t e)
 
 static void Live(const void* p, double bytes, const char* what)
 {
+    std::lock_guard<std::mutex> lock(mu);
     auto it = live.upper_bound((char*)p);
     if (p && it != live.begin()) {
         --it;
@@ -59,8 +67,13 @@ static void Live(const void* p, double bytes, const char* what)
 
 hipError_t hipMalloc(void** p, size_t n)
 {
+    std::lock_guard<std::mutex> lock(mu);
     ++allocs;
-    if (n >= smallest && failAt >= 0 && failAt-- == 0) return Set(hipErrorOutOfMemory);
+    if (used + n > capacity || (n >= smallest && failAt == 0)) {
+        failed = true;
+        return Set(hipErrorOutOfMemory);
+    }
+    if (n >= smallest && failAt > 0) --failAt;
     *p = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (*p == MAP_FAILED) std::abort();
     live[(char*)*p] = n;
@@ -70,6 +83,7 @@ hipError_t hipMalloc(void** p, size_t n)
 }
 hipError_t hipFree(void* p)
 {
+    std::lock_guard<std::mutex> lock(mu);
     ++frees;
     auto it = live.find((char*)p);
     need(p == nullptr || it != live.end(), "free of no allocation");
@@ -139,7 +153,8 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0, hipSuccess; }
 
 // ---- launches ------------------------------------------------------------------
-static long factorizations = 0, merged = 0, fusedSolves = 0, couplings = 0;
+static std::atomic<long> factorizations{0}, merged{0}, fusedSolves{0}, couplings{0};
+static std::atomic<bool> slow{false};
 
 namespace psp_amd {
 bool XcdRoundRobin(hipStream_t) { return true; }
@@ -173,6 +188,7 @@ template <typename T>
 void LaunchScatterOrig(const ClassDev& c, const StencilArgs&, const double*, double, hipStream_t)
 {
     ++factorizations;
+    if (slow) std::this_thread::sleep_for(std::chrono::milliseconds(50));
     Factors<T>(c, true);
     Live(c.T, Eb<T>(c) * c.tstore, "T");
     Live(c.F, Eb<T>(c) * c.fentries, "F");
@@ -375,22 +391,23 @@ static void oom()
         smallest = big;
         failAt = n;
         Counts t = Of("panel solve", c, [&] { return psp_hip_solve_panel(c, B, 9, 1); });
-        const bool failed = failAt < 0;
+        const bool short_ = failed;
+        failed = false;
         failAt = -1;
         smallest = 0;
-        if (failed) {
+        if (short_) {
             need(t.f == 0 && t.m == 1 && t.q == 0, "merged solves serve", n, t.f);
             t = Of("noalloc", c, [&] { return psp_hip_precondition_noalloc(c, B, 8); });
             need(t.f == 0 && t.m == solves, "noalloc", n);
             t = Of("Multiply", c, [&] { return psp_hip_multiply(c, B, B, 9); });
             psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 0);  // frees the workspace
-            need(used == resident, "memory given back", n, (long)(used - resident));
+            need(used <= resident, "memory given back", n, (long)(used - resident));
             psp_hip_set_option(c, PSP_HIP_OPT_SOLVE_FUSED, 1);
         }
         t = Of("sweep", c, [&] { return psp_hip_precondition(c, B, 9); });
-        need((t.f > 0) == failed && t.q > 0, "fused solves with the memory back", n, t.f);
+        need((t.f > 0) == short_ && t.q > 0, "fused solves with the memory back", n, t.f);
         psp_hip_destroy(c);
-        if (!failed) break;
+        if (!short_) break;
         need(n < 20, "big allocations");
     }
 }
@@ -401,25 +418,27 @@ static void retry()
         psp_hip_ctx* c = Context();
         failAt = n;
         const int st = Factor(c);
-        const bool failed = failAt < 0;
+        const bool short_ = failed;
+        failed = false;
         failAt = -1;
-        need(st == (failed ? PSP_HIP_ERR_MEMORY : PSP_HIP_OK), "Initialize", n, st);
-        if (failed) need(Factor(c) == PSP_HIP_OK, "Initialize again", n);
+        need(st == (short_ ? PSP_HIP_ERR_MEMORY : PSP_HIP_OK), "Initialize", n, st);
+        if (short_) need(Factor(c) == PSP_HIP_OK, "Initialize again", n);
         Of("sweep", c, [&] { return psp_hip_precondition(c, block.data(), 8); });
         psp_hip_destroy(c);
-        if (!failed) break;
+        need(used == 0, "given back", n, (long)used);
+        if (!short_) break;
     }
 }
 
 // Bytes of the factors of all panels as two plain copies, and of the scratch of
 // their updates and inverses.
-static void plainSizes(double* factors, double* scratch)
+static void plainSizes(double* factors, double* scratch, double* folded)
 {
     Plan plan;
     std::string msg;
     if (BuildPlan(desc, plan, msg) != PSP_HIP_OK) std::exit(2);
     const double eb = desc.precision == PSP_HIP_FRONTS_FP32 ? 8 : 16;
-    *factors = *scratch = 0;
+    *factors = *scratch = *folded = 0;
     std::vector<int> panels(3, 0);
     for (int p = 0; p < plan.geo.numPanels; ++p) ++panels[plan.geo.cls(p)];
     for (int cl = 0; cl < 3; ++cl) {
@@ -427,6 +446,7 @@ static void plainSizes(double* factors, double* scratch)
         const ClassPlan& C = plan.cls[cl];
         *factors += 2 * eb * panels[cl] * C.fstore;
         *scratch += eb * panels[cl] * (C.ustore + C.tstore);
+        *folded += eb * panels[cl] * 256.0 * (C.nblocks + 1);
         // the pieces of a depth group's E do not overlap
         for (const auto& g : C.groups) {
             std::vector<std::pair<int64_t, int64_t>> e;
@@ -443,8 +463,8 @@ static void plainSizes(double* factors, double* scratch)
 
 static void memory()
 {
-    double factors, scratch;
-    plainSizes(&factors, &scratch);
+    double factors, scratch, folded;
+    plainSizes(&factors, &scratch, &folded);
     psp_hip_ctx* c = Context();
     need(Factor(c) == PSP_HIP_OK && Factor(c) == PSP_HIP_OK, "Initialize");
     const double peak = (double)most;
@@ -453,6 +473,36 @@ static void memory()
     std::printf("GB: at most %.2f, as plain copies %.2f\n", (peak - plan) / 1e9, (factors + scratch) / 1e9);
     need(peak - plan <= factors + scratch, "memory of Initialize");
     psp_hip_destroy(c);
+    need(used == 0, "given back", (long)used);
+}
+
+// Contexts with factors at the same time, one after another and on threads.
+static void several()
+{
+    double factors, scratch, folded;
+    plainSizes(&factors, &scratch, &folded);
+    const double slack = 1 << 16;
+    psp_hip_ctx* c[3] = {Context(), Context(), Context()};
+    need(Factor(c[0]) == PSP_HIP_OK, "Initialize");
+    psp_hip_finalize(c[0]);
+    const double plan = (double)used;
+    for (psp_hip_ctx* x : c) need(Factor(x) == PSP_HIP_OK, "Initialize");
+    need(used <= 3 * (plan + folded) + factors / 2 + slack, "one L", (long)used);
+    // an allocation that needs L's memory gets it
+    capacity = used;
+    Of("sweep", c[1], [&] { return psp_hip_precondition(c[1], block.data(), 8); });
+    need(failed && used <= 3 * (plan + folded) + factors / 4, "memory of L", (long)used);
+    capacity = (size_t)-1;
+    failed = false;
+    need(Factor(c[2]) == PSP_HIP_OK, "Initialize again");
+    for (psp_hip_ctx* x : c) psp_hip_finalize(x);
+    need(used <= 3 * plan + slack, "given back", (long)used);
+    slow = true;
+    std::vector<std::thread> threads;
+    for (psp_hip_ctx* x : c) threads.emplace_back([x] { need(Factor(x) == PSP_HIP_OK, "Initialize"); });
+    for (std::thread& t : threads) t.join();
+    need(used <= 3 * (plan + folded) + factors / 2 + slack, "scratch of threads", (long)used);
+    for (psp_hip_ctx* x : c) psp_hip_destroy(x);
     need(used == 0, "given back", (long)used);
 }
 
@@ -485,8 +535,11 @@ int main(int argc, char** argv)
         retry();
     else if (mode == "memory")
         memory();
+    else if (mode == "several")
+        several();
     else
         return 2;
-    std::printf("%s: %ld allocations, %ld factorizations\n", mode.c_str(), allocs, factorizations);
+    std::printf("%s: %ld allocations, %ld factorizations\n", mode.c_str(), allocs,
+                factorizations.load());
     return fails ? 1 : 0;
 }

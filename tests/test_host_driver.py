@@ -4,8 +4,9 @@ against a HIP runtime of host memory, whose kernels compute nothing and check
 that their arrays are live and large enough.  Which calls factor and allocate
 when the fused launches are switched on after Initialize, with the memory for
 their layout and without it; Initialize after one that ran out of memory at any
-of its allocations; and the memory that Initialize takes at most, no more than
-the factors twice with the scratch of their updates and inverses."""
+of its allocations; the memory that Initialize takes at most, no more than the
+factors twice with the scratch of their updates and inverses; and several
+factored contexts, whose factorizations share an array."""
 import os
 import subprocess
 
@@ -33,6 +34,7 @@ def checker(tmp_path_factory):
 @pytest.mark.parametrize("args", [
     "fused 24 22 30", "fused 40 40 24 1", "oom 24 22 30", "oom 24 22 30 1", "retry 14 13 24",
     "retry 9 13 27 1", "memory 100 100 100", "memory 144 128 80", "memory 200 200 100 1",
+    "several 24 22 30", "several 61 47 83 1",
 ])
 def test_host_driver(checker, args):
     out = subprocess.run([checker] + args.split(), capture_output=True, text=True, timeout=300)
