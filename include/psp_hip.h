@@ -129,7 +129,8 @@ typedef struct {
     double seconds_inverse;  /* diagonal-block inversion (SELINV)         */
     double flops;            /* algorithmic real flops, 8 per complex MAC */
     double schur_flops;      /* subset spent in Schur-complement GEMMs    */
-    double bytes_factor;     /* bytes of stored factors                   */
+    double bytes_factor;     /* bytes of the fronts' factors, before they
+                                are merged                                */
     int num_panels;
     int num_fronts;          /* fronts over all panels                    */
     double seconds_schur;    /* GPU time of the Schur-complement GEMMs    */

@@ -1446,11 +1446,12 @@ __global__ __launch_bounds__(kThreads) void k_mv_reduce(const SolveTile* items, 
 // 4 (l / 16) .. + 4 of column l % 16 (the four steps then take the inner
 // index in the order t, 4 + t, 8 + t, 12 + t, which the staged vector
 // follows).  Either way a wave reads whole blocks, 2 or 4 KB, contiguous.
-// The inner vector is shared by the waves through LDS, CB blocks at a time in
-// two buffers: one barrier per chunk, the next chunk's vector and factor
-// loads in flight while a chunk is multiplied.  The first two chunks' factor
-// loads go out before anything is waited for; a tile is cut (DefaultSlices)
-// so that most waves have little more than that.
+// The inner vector is shared by the waves through LDS, CB blocks at a time.  Up
+// to 16 right-hand sides (BlockTileWork) a chunk has one buffer and two barriers:
+// its vector is loaded once the chunk before is multiplied, the first chunk's
+// before anything is waited for, and a ring of U factor blocks a wave is in flight
+// throughout, across chunks.  Passes of 32 (BlockTileWide) have two buffers and one
+// barrier a chunk, with two chunks of vector and factor blocks in flight.
 //
 // What bounds it: for k <= 16 the factor stream (HBM) and, on small launches,
 // the dependent round trips record -> (indices ->) operands -> stores; for
@@ -1950,9 +1951,11 @@ __device__ __forceinline__ void BlockTileWork(const BlockTile* tp, const BlockBu
 // its own registers, while one is multiplied from LDS (two buffers), and blocks
 // that a tile does not have are skipped.  The passes are workgroups of one
 // launch: a loop over them in one workgroup, on one staged chunk ahead, took
-// 41.7 ms a sweep at 100^3 k = 64 FP32 and 66.0 in FP64 (29.2 and 52.5 so);
-// 15.8 ms at 120 x 96 x 60 k = 32 FP32 (11.9).  CB = 4 and three workgroups a CU
-// spill registers and were slower.
+// 41.7 ms a sweep at 100^3 k = 64 FP32 and 66.0 in FP64 (28.5 and 50.4 now);
+// 15.8 ms at 120 x 96 x 60 k = 32 FP32 (11.3).  CB = 4 and three workgroups a CU
+// spill registers and were slower.  A block's sums for 8 right-hand sides run from
+// zero at a time (BlockSum): accumulators of all four, kept beside their sums,
+// took 29.0 and 52.0 ms.
 template <typename T, int KB>
 struct WideShape {
     static constexpr int NB = KB / 8;

@@ -236,8 +236,6 @@ template <typename T>
 void LaunchCopyOut(const PanelMap& m, c128* B, const void* Xp, int k, int nx, int ny, int nz,
                    int vOffset, int padding, int mode, hipStream_t s,
                    const StencilArgs* st = nullptr, const double* vel = nullptr, int v1 = -1);
-// Backward sweep, one pass: Xp = 0 except the superdiagonal coupling on the
-// panel's last local plane (MultiplySuperdiagonal, solve.hpp:725-733).
 // A panel's vector X in a pass from panel to panel: row[(v ny + y) nx + x] is
 // its row of (x, y, v), planes [padding, padding + depth) are the panel's own.
 struct PassPanel {
@@ -253,6 +251,8 @@ template <typename T>
 void LaunchPassOn(const StencilArgs& st, const double* vel, c128* B, int k, const PassPanel& o,
                   const PassPanel& i, int mode, int dir, hipStream_t s);
 
+// Backward sweep, one pass: Xp = 0 except the superdiagonal coupling on the
+// panel's last local plane (MultiplySuperdiagonal, solve.hpp:725-733).
 template <typename T>
 void LaunchZeroSetPlane(const PanelMap& m, const StencilArgs& st, const double* vel,
                         const c128* B, void* Xp, int k, int v2, int vlLast, hipStream_t s,

@@ -965,8 +965,6 @@ int EnsureFusedFactors(psp_hip_ctx* c, int k)
 // ---------------------------------------------------------------------------
 // Sweep: Precondition (solve.hpp:681-734) on a natural-order device block.
 // ---------------------------------------------------------------------------
-// couple >= 0: the copy-out also applies the subdiagonal coupling into the
-// next panel's first plane `couple` (SolvePanel + MultiplySubdiagonal).
 // The panel vector of a class's panel solves and its map to grid points, and
 // the solve between a copy in and a copy out.
 template <typename T>
@@ -995,6 +993,8 @@ struct PanelSolver {
     }
 };
 
+// couple >= 0: the copy-out also applies the subdiagonal coupling into the
+// next panel's first plane `couple` (SolvePanel + MultiplySubdiagonal).
 template <typename T>
 void PanelForward(psp_hip_ctx* c, c128* B, int k, int p, MvProfile* prof = nullptr,
                   int couple = -1)

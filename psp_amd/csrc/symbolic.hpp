@@ -273,7 +273,8 @@ struct ClassPlan {
     std::vector<InvItem> inv;
     std::vector<GemmLaunch> invGemm;      // alternating T = C*Ainv, X = -Binv*T
 
-    // Solve layout of the factors, made after the selective inversion:
+    // Layout of the fused launches, made after the selective inversion when they
+    // are on:
     //   L  ((s+u) x s, ld s+u): rows < s hold Linv (unit lower, ones stored
     //      on the diagonal), rows >= s hold -L_BL Linv;
     //   LT (s x (s+u), ld s):   columns < s hold Linv^T D^-1 (upper),
